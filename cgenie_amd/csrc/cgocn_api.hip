@@ -581,8 +581,14 @@ static int alloc_member(cgo_engine* e, MemberH* m) {
         HIPCHK(e, hipMemcpy(keep.data(), old, oldly.total, hipMemcpyDeviceToHost));
     }
     void* buf = nullptr;
-    if (hipMalloc(&buf, ly.total) != hipSuccess) return fail(e, CGO_E_NOMEM, "member: hipMalloc(%zu) failed", ly.total);
-    HIPCHK(e, hipMemset(buf, 0, ly.total));
+    // behind the member's state, what a step's flux hands its convection: the
+    // columns it sorted and their segments.  Formed anew in every step, so it
+    // is no part of the layout that checkpoints hold.
+    const size_t nwet = (size_t)g->dev.nwet, nseg = (size_t)std::max(g->dev.nfblk[0], g->dev.nfblk[1]);
+    const size_t scratch = (nwet + 1 + 2 * nseg) * 4;
+    if (hipMalloc(&buf, ly.total + scratch) != hipSuccess)
+        return fail(e, CGO_E_NOMEM, "member: hipMalloc(%zu) failed", ly.total + scratch);
+    HIPCHK(e, hipMemset(buf, 0, ly.total + scratch));
     if (old) {
         HIPCHK(e, hipMemcpy(buf, keep.data(), oldly.total, hipMemcpyHostToDevice));
         e->graveyard.push_back(old);  // the caller settled the member: nothing in flight reads it
@@ -614,6 +620,8 @@ static int alloc_member(cgo_engine* e, MemberH* m) {
     d.diag = reinterpret_cast<int32_t*>(b + ly.ctrl + 16);
     d.dmax = reinterpret_cast<double*>(b + ly.ctrl + 32);
     d.sfresh = reinterpret_cast<int32_t*>(b + ly.ctrl + 40);
+    d.ulist = reinterpret_cast<int32_t*>(b + ly.total);
+    d.useg = d.ulist + nwet;
     if (m->bgc) {
         d.ocn = reinterpret_cast<double*>(b + ly.ocn);
         d.part = reinterpret_cast<double*>(b + ly.part);

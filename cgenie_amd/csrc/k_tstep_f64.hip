@@ -12,20 +12,24 @@ void launch_flux64(const MemberDev* t, const int32_t* l, int n, const FluxShape&
 }
 
 void launch_co(const MemberDev* t, const int32_t* l, int n, int nwetmax, int maxkmax, int prec, hipStream_t s) {
-    // 64 wet columns per workgroup of 128 threads (32 convecting at a time,
-    // a group taking a second column when it has finished its first): small
-    // workgroups, many resident per CU whether few columns convect or most;
-    // fewer threads where the level arrays would not fit in 64 KiB of LDS
-    const int K = maxkmax + 2;
-    int nt = 128;
-    while (nt > 32 && co_lds_bytes(nt, nt / 2, K) > 65536) nt /= 2;
-    const int cb = nt / 2;
-    const dim3 grid((nwetmax + cb - 1) / cb, n);
-    const size_t lds = co_lds_bytes(nt, cb, K);
+    // A large batch (more chunks of CO_CB columns than the chip holds blocks:
+    // 4,096) runs one wave per block and up to four chunks per block, so that
+    // blocks that find no unstable column are few; a small one runs every
+    // chunk in a block of its own with more threads, so that a chunk's tracers
+    // are mixed in fewer rounds.  256 members of 36x36x16x24 FP32C per step:
+    // 1,175 us against 1,253 with 256 threads and one chunk per block (3.2
+    // against 14.7 us for the launch where every column is stable); eight
+    // members 201 against 206, one FP64 member 209 against 213.
+    const int KM = maxkmax, chunks = (nwetmax + CO_CB - 1) / CO_CB;
+    const bool large = (long long)chunks * n > 4096;
+    int nt = large ? 64 : CO_NT;
+    while (nt > 64 && co_lds_bytes(nt, KM) > 65536) nt /= 2;
+    const dim3 grid(large ? (chunks + 3) / 4 : chunks, n);
+    const size_t lds = co_lds_bytes(nt, KM);
     if (prec == 0)
-        hipLaunchKernelGGL(k_co<double>, grid, dim3(nt), lds, s, t, l, K, cb);
+        hipLaunchKernelGGL(k_co<double>, grid, dim3(nt), lds, s, t, l, KM);
     else
-        hipLaunchKernelGGL(k_co<float>, grid, dim3(nt), lds, s, t, l, K, cb);
+        hipLaunchKernelGGL(k_co<float>, grid, dim3(nt), lds, s, t, l, KM);
 }
 
 void launch_flip(const MemberDev* t, const int32_t* l, int n, hipStream_t s) {

@@ -275,6 +275,8 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
     };
 
     for (int q = 0; q < LB; q++) FB(q) = (R)0;
+    double rlow = 0.0;     // the new density of the level below, and whether
+    bool falls = true;     // it falls strictly from k1 up (co leaves such a column as it is)
     int32_t limps = 0;
     double dmaxv = 0.0;
     // The isoneutral slope terms are formed in FP64 in both forms.  The
@@ -633,11 +635,38 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
                 if (l0 + q == 1) newS = nv;
                 if (sums) add_sum(q, nv, s_os, s_mm, s_vv);
             }
-            if (l0 == 0) at(rhop, oc) = eos<double>(g.ec[0], g.ec[1], g.ec[2], g.ec[3], newT, newS);
+            if (l0 == 0) {
+                const double rn = eos<double>(g.ec[0], g.ec[1], g.ec[2], g.ec[3], newT, newS);
+                at(rhop, oc) = rn;
+                falls = falls & (k == k1c || rn < rlow);
+                rlow = rn;
+            }
         }
         if (FLUX_NBUF == 2) __syncthreads();  // plane k is read by every thread before it is replaced
         if (more) commit((k + 2) % FLUX_NBUF);
         __syncthreads();
+    }
+    if (IM != 1 && l0 == 0) {
+        // co's columns: this block's segment [w0, w1) of the member's list,
+        // its unstable columns first, in column order
+        constexpr int NW = FLUX_THREADS / 64;
+        __shared__ int s_uns[NW];
+        const int wv = tid >> 6;
+        const uint64_t mu = __ballot(active && !falls), before = ((uint64_t)1 << (tid & 63)) - 1;
+        if ((tid & 63) == 0) s_uns[wv] = __popcll(mu);
+        __syncthreads();
+        int pu = __popcll(mu & before), nu = 0;
+#pragma unroll
+        for (int q = 0; q < NW; q++) {
+            if (q < wv) pu += s_uns[q];
+            nu += s_uns[q];
+        }
+        if (active) gp(M.ulist)[w0 + (falls ? nu + tid - pu : pu)] = col;
+        if (tid == 0) {
+            gp(M.useg)[1 + 2 * B.x] = w0;
+            gp(M.useg)[2 + 2 * B.x] = nu;
+            if (B.x == 0) gp(M.useg)[0] = g.nfblk[V];
+        }
     }
     if (IM != 2 && l0 == 0 && M.diso && active) {
         if (limps) atomicAdd(&M.diag[0], limps);
@@ -716,240 +745,262 @@ void launch_flux_t(const MemberDev* t, const int32_t* l, int n, const FluxShape&
 }
 
 // co, goldstein.f90:2657-2777 (iconv = 0, ieos = 0): FP64 arithmetic on the
-// new state in place, in two passes over a workgroup of CB <= blockDim.x wet
-// columns.  Pass 1, a thread per column, all its density loads issued
-// together: a column whose density falls strictly from k1 up -- most
-// columns; the reference loop leaves them as they are -- only has its top T
-// and S noted; the others are listed in LDS.  Pass 2: each group of CO_LANES
-// lanes takes the next listed column whenever it has finished one.  The
-// column's level arrays (segment map, thicknesses, densities and its T and S
-// as the state stores them) sit in LDS, one copy per column: its lanes walk
-// the reference's mixing loop in lockstep and write the same values, so they
-// reach the same decisions; each lane mixes and copies its own share of the
-// tracers in memory (l = lane, lane + CO_LANES, ...), each tracer's
-// operations in the reference's order.  K = the level arrays' length (the
-// launch's deepest maxk + 2).  Fewer columns per workgroup (CB) make more
-// workgroups, which hold more convecting columns per CU at once where most
-// convect, and more that only run pass 1 where few do.
-constexpr int CO_LANES = 4;
-constexpr int CO_CH = 4;  // tracers whose loads one lane issues together
-__host__ __device__ constexpr size_t co_lds_bytes(int nt, int cb, int K) {
-    return (size_t)(nt / CO_LANES) * K * (4 * 8 + 4) + (size_t)cb * 4;
+// new state in place.  Which levels mix depends on T and S alone, so the
+// walk and the mixing of the other tracers are taken apart:
+//
+//   A  a thread per unstable column walks the reference's mixing loop on T, S
+//      and density in LDS and writes down what it mixed: the list of
+//      (level, thickness) terms of every mean, in the order they are added.
+//      The segments are a bit mask of their top levels (the reference's kk
+//      map holds the same tops, top to bottom), so a step of the walk reads
+//      one density.
+//   B  a thread per (unstable column, tracer) loads the tracer's column, all
+//      its levels at once, replays the list on its own LDS copy, writes the
+//      levels that changed and adds up the coupling's column sum.
+//
+// Every tracer's means are formed in the reference's order from the values
+// the state would hold in between, so FP64 members keep the reference's bits.
+// The columns come from the flux, which sees every column's new density and
+// leaves them sorted into unstable and stable: a launch finds its work packed,
+// and a stable ensemble's blocks read one count and end.
+//
+// Walking and mixing a column by four lanes together, each mean read from
+// and written back to memory, was bound by that chain of round trips.  In a
+// convecting state, per launch: 256 members of 36x36x16x24 FP32C 466 ->
+// 116 us, six of 72x72x32x40 1,078 -> 100 us, one FP64 member 124 -> 18 us;
+// every column stable (256 members): 11.9 -> 4.2 us.
+constexpr int CO_NT = 256;
+constexpr int CO_CB = 8;  // columns a block takes at a time: their walks share one wave
+// LDS of a block: nt private tracer columns of KM levels (before that A's T,
+// S, density and thickness of CO_CB <= nt / 4 columns), then the lists of up
+// to 2 (KM - 1) terms of the columns
+__host__ __device__ constexpr size_t co_lds_bytes(int nt, int KM) {
+    return (size_t)nt * KM * 8 + (size_t)CO_CB * 2 * KM * (8 + 1) + (size_t)CO_CB * (8 + 3 * 4);
 }
 template <typename R>
-__global__ __launch_bounds__(256) void k_co(const MemberDev* __restrict__ mems, const int32_t* __restrict__ list, int K, int CB) {
+__global__ __launch_bounds__(CO_NT) void k_co(const MemberDev* __restrict__ mems, const int32_t* __restrict__ list, int KM) {
+    constexpr int CB = CO_CB;
     extern __shared__ double co_lds[];
-    __shared__ int s_n, s_next;
     const BlockXYZ B = xcd_blk();
     const MemberDev& M = mems[list[B.y]];
     const GridDev& g = M.g;
-    const int nt = (int)blockDim.x, P = nt / CO_LANES;
+    const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
     const int maxi = g.maxi, maxk = g.maxk, L = M.L;
+    const AS_GLOBAL int32_t* useg = gp(M.useg);
+    const int nseg = useg[0];
+    int total = 0;  // unstable columns of the member
+    for (int q = 0; q < nseg; q++) total += useg[2 + 2 * q];
+    if (B.x * CB >= total && !M.sw) return;  // uniform for the block
     const int par = *gp(M.parity);
     void* st = M.st[par ^ 1];
     int16_t* lo = M.lo[par ^ 1];
     const bool carry = lo != nullptr;
-    const size_t plane = (size_t)g.ncol, tstride = (size_t)maxk * plane;
+    const uint32_t plane = (uint32_t)g.ncol, tstride = (uint32_t)g.ncell;
     AS_GLOBAL double* rho = gp(M.rho);
-    int* wl = reinterpret_cast<int*>(co_lds + (size_t)P * 4 * K) + (size_t)P * K;  // the list of pass 1
+    const int E = 2 * KM;                                   // terms a column's list holds
+    double* const r = co_lds;                               // A: [level - 1][CB]
+    double* const tp = r + (size_t)KM * CB;
+    double* const sp = tp + (size_t)KM * CB;
+    double* const dzm = sp + (size_t)KM * CB;
+    double* const lw = co_lds + (size_t)nt * KM;            // the lists: thickness [E][CB],
+    uint64_t* const ltops = reinterpret_cast<uint64_t*>(lw + (size_t)E * CB);  // the tops left
+    int* const lcol = reinterpret_cast<int*>(ltops + CB);   // column, bottom level, terms
+    int* const lk1 = lcol + CB;
+    int* const lne = lk1 + CB;
+    uint8_t* const llev = reinterpret_cast<uint8_t*>(lne + CB);  // level [E][CB], bit 7: last term of a mean
     // members with surface fluxes keep the top level's T and S as tstepo
     // leaves them (tsval_ocn, ssval_ocn of step_goldstein 427-430): the
     // next call of the fluxes reads them, whatever the coupling does after
-    auto snap = [&](int col, double t, double s) {
-        if (M.sw) {
-            gp(M.sw)[(size_t)SW_TSTAR * plane + col] = t;
-            gp(M.sw)[(size_t)SW_SSTAR * plane + col] = s;
-        }
+    auto snap = [&](int f, int col, double x) {
+        if (M.sw) gp(M.sw)[(size_t)f * plane + col] = x;
     };
-    if (threadIdx.x == 0) s_n = 0, s_next = 0;
-    __syncthreads();
-    // ---- pass 1: the loop below walks a stable column's m down to k1
-    // without mixing and the fill-in finds every level in place
-    {
-        const int w = B.x * CB + (int)threadIdx.x;
-        if ((int)threadIdx.x < CB && w < g.nwet) {
-            const int col = g.wetsorted[w];
-            const int k1 = k1at(g, col % maxi + 1, col / maxi + 1);
-            bool stable = true;
-            double rb = rho[(size_t)(maxk - 1) * plane + col];
-            for (int q = maxk - 1; q >= k1; q--) {
-                const double ra = rho[(size_t)(q - 1) * plane + col];
-                stable = stable & (rb < ra);
-                rb = ra;
-            }
-            if (stable) {
-                const size_t top = (size_t)(maxk - 1) * plane + col;
-                snap(col, StateIO<R>::ld(st, lo, top), StateIO<R>::ld(st, lo, tstride + top));
-            } else {
-                wl[atomicAdd(&s_n, 1)] = w;
+    // the column at place p of the segments' unstable or stable parts
+    auto place = [&](int p, bool stable) -> int {
+        for (int q = 0; q < nseg; q++) {
+            const int w0 = useg[1 + 2 * q], nu = useg[2 + 2 * q];
+            const int w1 = q + 1 < nseg ? useg[3 + 2 * q] : g.nwet;
+            const int m = stable ? w1 - w0 - nu : nu;
+            if (p < m) return gp(M.ulist)[w0 + (stable ? nu : 0) + p];
+            p -= m;
+        }
+        return 0;
+    };
+    if (M.sw)
+        for (int p = B.x * nt + tid; p < g.nwet - total; p += gridDim.x * nt) {
+            const int col = place(p, true);
+            const uint32_t top = (uint32_t)(maxk - 1) * plane + col;
+            snap(SW_TSTAR, col, StateIO<R>::ld(st, lo, top));
+            snap(SW_SSTAR, col, StateIO<R>::ld(st, lo, tstride + top));
+        }
+    for (int i0 = B.x * CB; i0 < total; i0 += gridDim.x * CB) {
+        const int n = min(CB, total - i0);
+        if (tid < n) {
+            const int col = place(i0 + tid, false);
+            lcol[tid] = col;
+            lk1[tid] = k1at(g, col % maxi + 1, col / maxi + 1);
+        }
+        __syncthreads();
+        for (int x = tid; x < n * maxk; x += nt) {
+            const int i = x % n, k = x / n;
+            if (k + 1 >= lk1[i]) {
+                const uint32_t o = (uint32_t)k * plane + lcol[i];
+                const auto a = StateIO<R>::ldr(st, lo, o), b = StateIO<R>::ldr(st, lo, tstride + o);
+                r[k * CB + i] = at(rho, o);
+                tp[k * CB + i] = StateIO<R>::val(a, carry);
+                sp[k * CB + i] = StateIO<R>::val(b, carry);
+                dzm[k * CB + i] = gp(g.mk)[MK_DZ * (maxk + 2) + k + 1];
             }
         }
-    }
-    __syncthreads();
-    const int n = s_n;
-    if (n == 0) return;  // uniform for the block
-    // ---- pass 2
-    const int sub = (int)threadIdx.x % CO_LANES, cl = (int)threadIdx.x / CO_LANES;
-    const AS_GLOBAL double* dz = gp(g.mk) + MK_DZ * (maxk + 2);
-    const double e0 = g.ec[0], e1 = g.ec[1], e2 = g.ec[2], e3 = g.ec[3];
-    double* r = co_lds + (size_t)cl * 4 * K;
-    double* dzm = r + K;
-    double* tp = dzm + K;
-    double* sp = tp + K;
-    int* kk = reinterpret_cast<int*>(co_lds + (size_t)P * 4 * K) + (size_t)cl * K;
-    // this lane's tracers: l = sub + CO_LANES * j, j < nmine
-    const int nmine = L > sub ? (L - sub + CO_LANES - 1) / CO_LANES : 0;
-    // the group's lanes sit side by side in one wave; its first lane takes
-    // the next list entry for the group
-    const int lead = ((int)threadIdx.x & 63) & ~(CO_LANES - 1);
-    for (;;) {
-        int idx = 0;
-        if (sub == 0) idx = atomicAdd(&s_next, 1);
-        idx = __shfl(idx, lead);
-        if (idx >= n) break;
-        {
-            const int w = wl[idx];
-            const int col = g.wetsorted[w];
-            const int k1 = k1at(g, col % maxi + 1, col / maxi + 1);
-            for (int m = 0; m <= maxk + 1; m++) kk[m] = 0;
-            for (int m = k1; m <= maxk; m++) {
-                r[m] = rho[(size_t)(m - 1) * plane + col];
-                tp[m] = StateIO<R>::ld(st, lo, (size_t)(m - 1) * plane + col);
-                sp[m] = StateIO<R>::ld(st, lo, tstride + (size_t)(m - 1) * plane + col);
-                kk[m] = m;
-                dzm[m] = dz[m];
-            }
-            int m = maxk, lastmix = 0;
-            bool mixed = false;
-            // every pass either moves m or merges two segments, so the
-            // reference loop ends within O(maxk^2) passes; the cap only
-            // guards non-finite densities
+        __syncthreads();
+        // ---- A
+        if (tid < n) {
+            const int i = tid, k1 = lk1[i], col = lcol[i];
+            const double e0 = g.ec[0], e1 = g.ec[1], e2 = g.ec[2], e3 = g.ec[3];
+            auto R_ = [&](int k) -> double& { return r[(k - 1) * CB + i]; };
+            auto T_ = [&](int k) -> double& { return tp[(k - 1) * CB + i]; };
+            auto S_ = [&](int k) -> double& { return sp[(k - 1) * CB + i]; };
+            auto W_ = [&](int k) -> double& { return dzm[(k - 1) * CB + i]; };
+            auto below = [](uint64_t m, int k) -> int {  // the highest top under level k, 0 if none
+                const uint64_t b = m & (((uint64_t)1 << k) - 1);
+                return b ? 63 - __clzll((long long)b) : 0;
+            };
+            const uint64_t all = (((uint64_t)2 << maxk) - 1) & ~(((uint64_t)1 << k1) - 1);  // bits k1..maxk
+            uint64_t tops = all;
+            int km = maxk, lastmix = 0, ne = 0;
+            double rk = R_(km);
+            // every pass either moves or merges two segments, and it moves up
+            // only once after a merge, so the loop ends within O(maxk^2) passes;
+            // the cap only guards non-finite densities
             int guard = 4 * maxk * maxk + 64;
-            while ((kk[m - 1] > 0 || (lastmix != 0 && kk[m] != maxk)) && --guard > 0) {
-                if (kk[m - 1] == 0 || r[kk[m]] < r[kk[m - 1]]) {
-                    if (lastmix == 0 || kk[m] == maxk)
-                        m = m - 1;
+            for (int low = below(tops, km); (low > 0 || (lastmix != 0 && km != maxk)) && --guard > 0; low = below(tops, km)) {
+                if (low == 0 || rk < R_(low)) {
+                    if (lastmix == 0 || km == maxk)
+                        km = low;
                     else
-                        m = m + 1;
+                        km = km + 1 + __builtin_ctzll(tops >> (km + 1));
                     lastmix = 0;
+                    rk = R_(km);
                 } else {
                     lastmix = 1;
-                    mixed = true;
-                    int nn = m - 1;
-                    while (kk[nn - 1] > 0 && r[kk[nn]] >= r[kk[nn - 1]]) nn = nn - 1;
-                    const int km = kk[m];
-                    double dsum = dzm[km];
-                    for (int ni = 1; ni <= m - nn; ni++) dsum = dsum + dzm[kk[m - ni]];
-                    // the thickness-weighted mean of levels kk[nn..m]: T and S
-                    // privately on every lane, this lane's tracers in memory,
-                    // CO_CH at a time (their loads issued together)
-                    {
-                        double at = tp[km] * dzm[km], as = sp[km] * dzm[km];
-                        for (int ni = 1; ni <= m - nn; ni++) {
-                            const int kq = kk[m - ni];
-                            at = at + tp[kq] * dzm[kq];
-                            as = as + sp[kq] * dzm[kq];
-                        }
-                        tp[km] = StateIO<R>::rt(at / dsum, carry);
-                        sp[km] = StateIO<R>::rt(as / dsum, carry);
+                    // the thickness-weighted mean of the segments from km down
+                    // through every one that is unstable against the next
+                    double dsum = W_(km), tm = T_(km) * dsum, sm = S_(km) * dsum;
+                    llev[ne * CB + i] = (uint8_t)km;
+                    lw[ne * CB + i] = dsum;
+                    ne++;
+                    for (int q = low, nx;; q = nx) {
+                        const double wq = W_(q);
+                        dsum = dsum + wq;
+                        tm = tm + T_(q) * wq;
+                        sm = sm + S_(q) * wq;
+                        tops &= ~((uint64_t)1 << q);
+                        nx = below(tops, q);
+                        const bool last = nx == 0 || !(R_(q) >= R_(nx));
+                        llev[ne * CB + i] = (uint8_t)(q | (last ? 128 : 0));
+                        lw[ne * CB + i] = wq;
+                        ne++;
+                        if (last) break;
                     }
-                    for (int j0 = 0; j0 < nmine; j0 += CO_CH) {
-                        double sm[CO_CH];
+                    tm = StateIO<R>::rt(tm / dsum, carry);
+                    sm = StateIO<R>::rt(sm / dsum, carry);
+                    T_(km) = tm;
+                    S_(km) = sm;
+                    W_(km) = dsum;
+                    rk = eos<double>(e0, e1, e2, e3, tm, sm);
+                    R_(km) = rk;
+                }
+            }
+            if (guard <= 0) atomicAdd(&M.diag[3], 1);
+            lne[i] = ne;
+            ltops[i] = tops;
+            // every level that is no segment's top takes its segment's density
+            // (and, in B, its tracers); each such level counts as one convection
+            const uint64_t fill = all & ~tops;
+            double v = 0.0;
+            for (int k = maxk; k >= k1; k--) {
+                if ((tops >> k) & 1) v = R_(k);
+                if (((fill | (fill << 1)) >> k) & 1) at(rho, (uint32_t)(k - 1) * plane + col) = v;
+            }
+            if (fill) gp(M.cost)[col] += (double)__popcll(fill);
+        }
+        __syncthreads();
+        // ---- B
+        double* const v = co_lds + tid;  // level k at v[(k - 1) * nt]
+        const double rSold = M.bgc ? 1.0 / gp(M.scal)[SC_SMEAN] : 0.0;
+        for (int x = tid; x < n * L; x += nt) {
+            const int i = x % n, l = x / n;
+            const int k1 = lk1[i], col = lcol[i], ne = lne[i];
+            const uint64_t tops = ltops[i];
+            const uint32_t base = (uint32_t)l * tstride + col;
+            for (int k0 = k1; k0 <= maxk; k0 += 8) {
+                typename StateIO<R>::Raw q[8];
 #pragma unroll
-                        for (int c = 0; c < CO_CH; c++)
-                            if (j0 + c < nmine)
-                                sm[c] = StateIO<R>::ld(st, lo, (size_t)(sub + CO_LANES * (j0 + c)) * tstride + col +
-                                                                   (size_t)(km - 1) * plane) * dzm[km];
-                        for (int ni = 1; ni <= m - nn; ni++) {
-                            const int kq = kk[m - ni];
-                            const double wq = dzm[kq];
+                for (int u = 0; u < 8; u++)
+                    if (k0 + u <= maxk) q[u] = StateIO<R>::ldr(st, lo, base + (uint32_t)(k0 + u - 1) * plane);
 #pragma unroll
-                            for (int c = 0; c < CO_CH; c++)
-                                if (j0 + c < nmine)
-                                    sm[c] = sm[c] + StateIO<R>::ld(st, lo, (size_t)(sub + CO_LANES * (j0 + c)) * tstride +
-                                                                               col + (size_t)(kq - 1) * plane) * wq;
+                for (int u = 0; u < 8; u++)
+                    if (k0 + u <= maxk) v[(k0 + u - 1) * nt] = StateIO<R>::val(q[u], carry);
+            }
+            {
+                double sum = 0.0, dsum = 0.0;
+                int km = 0;  // the level a mean is written to, 0 before its first term
+                for (int e = 0; e < ne; e++) {
+                    const int lev = llev[e * CB + i], k = lev & 127;
+                    const double wt = lw[e * CB + i], xv = v[(k - 1) * nt];
+                    if (km == 0) {
+                        km = k;
+                        dsum = wt;
+                        sum = xv * wt;
+                    } else {
+                        dsum = dsum + wt;
+                        sum = sum + xv * wt;
+                        if (lev & 128) {
+                            v[(km - 1) * nt] = StateIO<R>::rt(sum / dsum, carry);
+                            km = 0;
                         }
-#pragma unroll
-                        for (int c = 0; c < CO_CH; c++)
-                            if (j0 + c < nmine)
-                                StateIO<R>::st(st, lo, (size_t)(sub + CO_LANES * (j0 + c)) * tstride + col + (size_t)(km - 1) * plane,
-                                               sm[c] / dsum);
-                    }
-                    for (int ni = 1; ni <= m - nn; ni++) dzm[km] = dzm[km] + dzm[kk[m - ni]];
-                    r[km] = eos<double>(e0, e1, e2, e3, tp[km], sp[km]);
-                    int ni = m - 1;
-                    while (kk[ni + 1] > 0) {
-                        kk[ni] = kk[ni - m + nn];
-                        ni = ni - 1;
                     }
                 }
             }
-            if (guard <= 0 && sub == 0) atomicAdd(&M.diag[3], 1);
-            // fill-in: every level not left as a segment's own takes the
-            // values of the segment it lies in
-            m = maxk - 1;
-            double cost = 0.0;
-            for (int nn = maxk - 1; nn >= k1; nn--) {
-                if (nn > kk[m]) {
-                    const int kf = kk[m + 1];
-                    const size_t from = (size_t)(kf - 1) * plane + col, to = (size_t)(nn - 1) * plane + col;
-                    for (int j0 = 0; j0 < nmine; j0 += CO_CH) {
-                        double v[CO_CH];
-#pragma unroll
-                        for (int c = 0; c < CO_CH; c++)
-                            if (j0 + c < nmine) v[c] = StateIO<R>::ld(st, lo, (size_t)(sub + CO_LANES * (j0 + c)) * tstride + from);
-#pragma unroll
-                        for (int c = 0; c < CO_CH; c++)
-                            if (j0 + c < nmine) StateIO<R>::st(st, lo, (size_t)(sub + CO_LANES * (j0 + c)) * tstride + to, v[c]);
-                    }
-                    tp[nn] = tp[kf];
-                    sp[nn] = sp[kf];
-                    r[nn] = eos<double>(e0, e1, e2, e3, tp[nn], sp[nn]);
-                    cost += 1.0;
-                } else {
-                    m = m - 1;
-                }
+            const uint64_t all = (((uint64_t)2 << maxk) - 1) & ~(((uint64_t)1 << k1) - 1);
+            const uint64_t fill = all & ~tops, chg = fill | (fill << 1);
+            double sv = 0.0;
+            for (int k = maxk; k >= k1; k--) {
+                if ((tops >> k) & 1)
+                    sv = v[(k - 1) * nt];
+                else
+                    v[(k - 1) * nt] = sv;
+                if ((chg >> k) & 1) StateIO<R>::st(st, lo, base + (uint32_t)(k - 1) * plane, sv);
             }
-            if ((mixed || cost > 0.0) && M.bgc) {
+            if (l < 2) snap(l == 0 ? SW_TSTAR : SW_SSTAR, col, v[(maxk - 1) * nt]);
+            if (M.bgc && l >= 1) {
                 // the coupling's column sums of this column after mixing and fill-in
-                const double rSold = 1.0 / gp(M.scal)[SC_SMEAN];
-                const size_t ncl = (size_t)g.ncell, slot = (size_t)gp(g.vpos)[w];
-                AS_GLOBAL double* cs = gp(M.colsum);
-                if (sub == 0) {
-                    double aS = 0.0;
-                    for (int q = k1; q <= maxk; q++) aS += (sp[q] + SALN0 + 0.0) * gp(g.V)[(size_t)(q - 1) * plane + col];
-                    cs[slot] = aS;
-                }
-                // this lane's tracers from the third on
-                const int jfirst = sub >= 2 ? 0 : 1;
-                for (int j0 = jfirst; j0 < nmine; j0 += CO_CH) {
-                    double a[CO_CH];
+                const uint32_t ncl = (uint32_t)g.ncell;
+                double a = 0.0;
+                for (int k0 = k1; k0 <= maxk; k0 += 4) {
+                    double f0[4], f1[4];
 #pragma unroll
-                    for (int t = 0; t < CO_CH; t++) a[t] = 0.0;
-                    for (int q = k1; q <= maxk; q++) {
-                        const size_t c = (size_t)(q - 1) * plane + col;
-                        const double so = gp(M.ocn)[ncl + c], mm = gp(M.M)[c];
+                    for (int u = 0; u < 4; u++)
+                        if (k0 + u <= maxk) {
+                            const uint32_t c = (uint32_t)(k0 + u - 1) * plane + col;
+                            f0[u] = l == 1 ? at(gp(g.V), c) : at(gp(M.ocn), ncl + c);
+                            f1[u] = l == 1 ? 0.0 : at(gp(M.M), c);
+                        }
 #pragma unroll
-                        for (int t = 0; t < CO_CH; t++)
-                            if (j0 + t < nmine) {
-                                const double lv =
-                                    StateIO<R>::ld(st, lo, (size_t)(sub + CO_LANES * (j0 + t)) * tstride + c) * so * rSold;
-                                a[t] += lv * mm;
+                    for (int u = 0; u < 4; u++)
+                        if (k0 + u <= maxk) {
+                            const double xv = v[(k0 + u - 1) * nt];
+                            if (l == 1) {
+                                a += (xv + SALN0 + 0.0) * f0[u];
+                            } else {
+                                const double lv = xv * f0[u] * rSold;
+                                a += lv * f1[u];
                             }
-                    }
-#pragma unroll
-                    for (int t = 0; t < CO_CH; t++)
-                        if (j0 + t < nmine) cs[(size_t)(sub + CO_LANES * (j0 + t)) * g.nwet + slot] = a[t];
+                        }
                 }
-            }
-            if (sub == 0) {
-                if (mixed || cost > 0.0) {
-                    for (int q = k1; q <= maxk; q++) rho[(size_t)(q - 1) * plane + col] = r[q];
-                    if (cost > 0.0) gp(M.cost)[col] += cost;
-                }
-                snap(col, tp[maxk], sp[maxk]);
+                gp(M.colsum)[(size_t)(l == 1 ? 0 : l) * g.nwet + gp(g.cslot)[col]] = a;
             }
         }
+        __syncthreads();  // the next columns' T, S and density take B's place
     }
 }
 

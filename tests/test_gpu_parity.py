@@ -434,3 +434,47 @@ def test_split_calls_equal_step(eng):
     eng.tstepo([m2], 2)                   # transport alone is allowed again
     eng.remove_member(m1)
     eng.remove_member(m2)
+
+
+@pytest.mark.parametrize("dims,L,precision,n", [((5, 4, 2), 2, E.FP64, 1), ((12, 11, 2), 2, E.FP64, 1),
+                                                ((13, 9, 17), 5, E.FP64, 1), ((9, 7, 48), 3, E.FP64, 2),
+                                                ((18, 18, 8), 9, E.FP64, 170), ((18, 18, 8), 9, E.FP32C, 170),
+                                                ((13, 9, 33), 66, E.FP32C, 1)])
+def test_convection_at_its_edges(dims, L, precision, n):
+    """Convection with the fewest and most levels, one and many chunks of
+    columns per block, tracers over and under a block's threads, every column
+    unstable over its whole depth or in runs: FP64 members equal the oracle
+    bit for bit; FP32C members in a large batch equal the same member alone
+    (another launch shape) bit for bit."""
+    c = make_case(*dims, kind="ts", L=L, seed=47)
+    rng = np.random.default_rng(48)
+    w = wet(c)
+    c.ts[..., 0] = rng.uniform(0.0, 25.0, w.shape)                      # runs of unstable levels
+    c.ts[:, ::2, ::2, 0] = np.linspace(20.0, 1.0, dims[2])[:, None, None]  # cold over warm all the way
+    c.ts[:, 1::2, 1::2, 0] = np.linspace(1.0, 20.0, dims[2])[:, None, None]  # stable
+    c.ts[~w] = 0.0
+
+    def run(m):
+        eng = E.Engine(0)
+        ids = []
+        gid = eng.add_grid(c.g, c.k1)
+        for _ in range(m):
+            ids.append(eng.add_member(gid, L, precision, c.diff))
+            eng.set_velocity(ids[-1], c.u)
+            eng.upload(ids[-1], c.ts)
+        eng.tstepo(ids, 3)
+        out = [(eng.download(q, c.ts.shape), eng.rho(q, c.g), eng.diag(q).cost) for q in (ids[0], ids[-1])]
+        eng.close()
+        return out
+
+    got = run(n)
+    assert got[0][2] == got[1][2]
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1][w], got[1][1][w])
+    if precision == E.FP64:
+        o = O.GoldsteinOracle(c.og, c.k1, c.ts, c.u)
+        o.step(3)
+        say(dims, "levels filled by convection", o.cost.sum())
+        assert np.array_equal(got[0][0][w], o.ts[w]) and got[0][2] == o.cost.sum()
+    else:
+        alone = run(1)[0]
+        assert np.array_equal(got[0][0], alone[0]) and got[0][2] == alone[2]
