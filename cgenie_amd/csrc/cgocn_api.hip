@@ -19,10 +19,11 @@
 
 namespace cgo {
 void launch_flux64(const MemberDev*, const int32_t*, int nlist, const FluxShape&, int maxL, int lb, int nt, int nbuf,
-                   int iso_split, int part, size_t lds_cap, hipStream_t);
+                   int iso_split, const FluxSplit&, int part, size_t lds_cap, hipStream_t);
 void launch_flux32(const MemberDev*, const int32_t*, int nlist, const FluxShape&, int maxL, int lb, int nt, int nbuf,
-                   int iso_split, int part, size_t lds_cap, hipStream_t);
-void launch_co(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int prec, hipStream_t);
+                   int iso_split, const FluxSplit&, int part, size_t lds_cap, hipStream_t);
+void launch_co(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int prec, const FluxSplit&,
+               hipStream_t);
 void launch_flip(const MemberDev*, const int32_t*, int nlist, hipStream_t);
 void launch_bio(const MemberDev*, const int32_t*, int nlist, int nwetmax, int W, int prec, hipStream_t);
 void launch_coupling(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int maxL, int prec,
@@ -106,6 +107,7 @@ struct Graph {
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
     int32_t* d_lists = nullptr;
+    double* d_nv = nullptr;   // the split flux's new values (Lists::sp)
     // the captured members and the generation of their slots at capture:
     // launch extents, precision lists and stream windows are baked into the
     // graph, so a replay is refused once any of them was destroyed,
@@ -146,10 +148,15 @@ struct cgo_engine {
     int nt[2] = {256, 256};   // wet columns per block
     int nbuf[2] = {2, 2};     // level planes resident in LDS
     int isosplit[2] = {1, 1}; // isoneutral coefficients from a pre-pass
+    // no tile was set for the precision: a batch too small to fill the chip
+    // may take the flux split by levels (flux_split)
+    bool auto_tile[2] = {true, true};
     size_t lds_cap = 65536;   // LDS one workgroup may take
     std::vector<Graph> graphs;
     int32_t* d_list = nullptr;  // scratch lists for eager steps
     size_t d_list_cap = 0;
+    double* d_nv = nullptr;     // the split flux's new values of eager steps (Lists::sp)
+    size_t d_nv_cap = 0;        // doubles
     std::vector<int32_t> last_lists;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -266,6 +273,7 @@ int cgo_destroy(cgo_engine* e) {
         if (g.exec) hipGraphExecDestroy(g.exec);
         if (g.graph) hipGraphDestroy(g.graph);
         if (g.d_lists) hipFree(g.d_lists);
+        if (g.d_nv) hipFree(g.d_nv);
     }
     for (auto* m : e->members)
         if (m) {
@@ -281,6 +289,7 @@ int cgo_destroy(cgo_engine* e) {
             delete g;
         }
     if (e->d_list) hipFree(e->d_list);
+    if (e->d_nv) hipFree(e->d_nv);
     if (e->d_table) hipFree(e->d_table);
     if (e->ev0) hipEventDestroy(e->ev0);
     if (e->ev1) hipEventDestroy(e->ev1);
@@ -1992,10 +2001,46 @@ struct Lists {
     int maxk_bgc[2] = {0, 0}, wstream[2] = {0, 0}, maxk[2] = {0, 0};
     int ncol_atm = 0;  // widest grid of the members with air-sea exchange, 0 if none
     FluxShape fs[2] = {};
+    FluxSplit sp[2] = {};
+    size_t nv = 0;  // doubles of workspace the FP32 list's split flux needs
 };
+
+// The flux split by levels, for batches whose blocks of two tracers and whole
+// columns (nb) leave the chip short of work.  768 such blocks are resident at
+// once: up to there the levels are cut into as many chunks (of two levels at
+// least) as fill it.  Past it the two-tracer blocks still beat the wide
+// tracer blocks with their pre-pass for a while, for FP64 members up to half
+// as many again.  us per step, wide blocks against this: one FP64 member of
+// 36x36x16x24 206 / 141 (nb 48), 4 members 231 / 150, 16 members (768) 308 /
+// 265, 24 members 299 / 247, 32 members (1536) 363 / 360; FP32C 16 members
+// 204 / 193, 24 members 261 / 291; transport of 5 members of 25x21x11x7 78 /
+// 33, one of 72x72x32x40 255 / 133.
+static void flux_split(const cgo_engine* e, Lists& ls, size_t cells) {
+    constexpr int FULL = 768;
+    for (int p = 0; p < 2; p++) {
+        if (!e->auto_tile[p] || !ls.n[p] || ls.fs[p].nblk[1] == 0) continue;
+        const long long nb = (long long)ls.fs[p].nblk[1] * ((ls.maxL[p] + 1) / 2) * ls.n[p];
+        if (nb > (p == 0 ? FULL * 3 / 2 : FULL)) continue;
+        const int maxk = ls.fs[p].maxk;
+        const int chunks = (int)std::min<long long>(std::max<long long>(FULL / nb, 1), (maxk + 1) / 2);
+        ls.sp[p].kc = (maxk + chunks - 1) / chunks;
+        ls.sp[p].nbx = ls.fs[p].nblk[1];
+        if (p == 1 && ls.n[3]) {
+            ls.sp[p].stride = cells;
+            ls.nv = cells * ls.n[1];
+        }
+    }
+}
+// where its workspace cannot be had the flux marches whole columns
+static void no_flux_split(Lists& ls) {
+    hipGetLastError();
+    ls.sp[1] = FluxSplit{};
+    ls.nv = 0;
+}
 
 static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
     std::vector<int32_t> g[9];
+    size_t cells = 0;  // most tracer cells of an FP32 member with BIOGEM
     std::vector<int> dgrid;                 // grids of the dense solve, in order of first appearance
     std::vector<std::vector<int32_t>> dmem;
     for (int i = 0; i < n; i++) {
@@ -2039,6 +2084,8 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
             ls.fs[p].nblk[v] = std::max(ls.fs[p].nblk[v], m->dev.g.nfblk[v]);
             ls.fs[p].tw[v] = std::max(ls.fs[p].tw[v], e->grids[m->grid]->ftw[v]);
         }
+        ls.fs[p].maxk = std::max(ls.fs[p].maxk, m->dev.g.maxk);
+        if (m->bgc && p) cells = std::max(cells, (size_t)m->L * m->dev.g.ncell);
         if (m->bgc) {
             ls.maxwet_bgc[p] = std::max(ls.maxwet_bgc[p], m->dev.g.nwet);
             ls.maxk_bgc[p] = std::max(ls.maxk_bgc[p], m->dev.g.maxk);
@@ -2057,6 +2104,7 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
         ls.n[q] = (int)g[q].size();
         ls.v.insert(ls.v.end(), g[q].begin(), g[q].end());
     }
+    flux_split(e, ls, cells);
     return CGO_OK;
 }
 
@@ -2068,17 +2116,17 @@ static void enqueue_flux(cgo_engine* e, const Lists& ls, const int32_t* d_lists,
         const int32_t* l = d_lists + ls.off[p];
         if (p == 0)
             launch_flux64(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[0], e->nt[0], e->nbuf[0], e->isosplit[0],
-                          part, e->lds_cap, e->s);
+                          ls.sp[0], part, e->lds_cap, e->s);
         else
             launch_flux32(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[1], e->nt[1], e->nbuf[1], e->isosplit[1],
-                          part, e->lds_cap, e->s);
+                          ls.sp[1], part, e->lds_cap, e->s);
     }
 }
 
 // co and the parity flip that end tstepo
 static void enqueue_co_flip(cgo_engine* e, const Lists& ls, const int32_t* d_lists) {
     for (int p = 0; p < 2; p++)
-        if (ls.n[p]) launch_co(e->d_table, d_lists + ls.off[p], ls.n[p], ls.maxwet[p], ls.maxk[p], p, e->s);
+        if (ls.n[p]) launch_co(e->d_table, d_lists + ls.off[p], ls.n[p], ls.maxwet[p], ls.maxk[p], p, ls.sp[p], e->s);
     launch_flip(e->d_table, d_lists + ls.off[4], ls.n[4], e->s);
 }
 
@@ -2186,12 +2234,29 @@ static int upload_lists(cgo_engine* e, const Lists& ls) {
     return CGO_OK;
 }
 
+// the eager steps' workspace of the split flux
+static int flux_workspace(cgo_engine* e, Lists& ls) {
+    if (ls.nv > e->d_nv_cap) {
+        HIPCHK(e, hipStreamSynchronize(e->s));
+        if (e->d_nv) hipFree(e->d_nv);
+        e->d_nv = nullptr;
+        e->d_nv_cap = 0;
+        if (hipMalloc(&e->d_nv, ls.nv * 8) == hipSuccess)
+            e->d_nv_cap = ls.nv;
+        else
+            no_flux_split(ls);
+    }
+    ls.sp[1].nv = e->d_nv;
+    return CGO_OK;
+}
+
 static int prepare(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls, bool steps = true) {
     hipSetDevice(e->device);
     int rc = make_lists(e, ids, n, ls);
     if (rc) return rc;
     if ((rc = sync_table(e))) return rc;
     if ((rc = upload_lists(e, ls))) return rc;
+    if ((rc = flux_workspace(e, ls))) return rc;
     for (int i = 0; i < n; i++) {
         member(e, ids[i])->queued = true;
         if (steps) member(e, ids[i])->stepped = true;
@@ -2295,6 +2360,11 @@ int cgo_graph_capture(cgo_engine* e, const int32_t* ids, int32_t n, int32_t nste
     Graph gr;
     gr.ids.assign(ids, ids + n);
     for (int i = 0; i < n; i++) gr.gens.push_back(ids[i] < (int32_t)e->gen.size() ? e->gen[ids[i]] : 0);
+    if (ls.nv && hipMalloc(&gr.d_nv, ls.nv * 8) != hipSuccess) {
+        gr.d_nv = nullptr;
+        no_flux_split(ls);
+    }
+    ls.sp[1].nv = gr.d_nv;
     HIPCHK(e, hipMalloc(&gr.d_lists, ls.v.size() * 4));
     HIPCHK(e, hipMemcpy(gr.d_lists, ls.v.data(), ls.v.size() * 4, hipMemcpyHostToDevice));
     HIPCHK(e, hipStreamSynchronize(e->s));
@@ -2303,12 +2373,14 @@ int cgo_graph_capture(cgo_engine* e, const int32_t* ids, int32_t n, int32_t nste
     hipError_t r = hipStreamEndCapture(e->s, &gr.graph);
     if (r != hipSuccess) {
         hipFree(gr.d_lists);
+        hipFree(gr.d_nv);
         return fail(e, CGO_E_HIP, "hipStreamEndCapture: %s", hipGetErrorString(r));
     }
     r = hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0);
     if (r != hipSuccess) {
         hipGraphDestroy(gr.graph);
         hipFree(gr.d_lists);
+        hipFree(gr.d_nv);
         return fail(e, CGO_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(r));
     }
     int slot = -1;
@@ -2357,6 +2429,7 @@ int cgo_graph_destroy(cgo_engine* e, int32_t gid) {
     hipGraphExecDestroy(g.exec);
     hipGraphDestroy(g.graph);
     hipFree(g.d_lists);
+    hipFree(g.d_nv);
     g = Graph();
     return CGO_OK;
 }
@@ -2365,6 +2438,7 @@ int cgo_set_tile(cgo_engine* e, int32_t precision, int32_t tb) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (tb != 2 && tb != 4 && tb != 6 && tb != 8))
         return fail(e, CGO_E_ARG, "set_tile: precision %d tracer block %d", precision, tb);
     e->lb[precision == CGO_FP64 ? 0 : 1] = tb;
+    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
     return CGO_OK;
 }
 
@@ -2372,6 +2446,7 @@ int cgo_set_flux_cols(cgo_engine* e, int32_t precision, int32_t cols) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (cols != 128 && cols != 256))
         return fail(e, CGO_E_ARG, "set_flux_cols: precision %d columns %d", precision, cols);
     e->nt[precision == CGO_FP64 ? 0 : 1] = cols;
+    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
     return CGO_OK;
 }
 
@@ -2379,6 +2454,7 @@ int cgo_set_flux_ring(cgo_engine* e, int32_t precision, int32_t planes) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (planes != 2 && planes != 3))
         return fail(e, CGO_E_ARG, "set_flux_ring: precision %d planes %d", precision, planes);
     e->nbuf[precision == CGO_FP64 ? 0 : 1] = planes;
+    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
     return CGO_OK;
 }
 
@@ -2386,6 +2462,7 @@ int cgo_set_flux_iso(cgo_engine* e, int32_t precision, int32_t prepass) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (prepass != 0 && prepass != 1))
         return fail(e, CGO_E_ARG, "set_flux_iso: precision %d prepass %d", precision, prepass);
     e->isosplit[precision == CGO_FP64 ? 0 : 1] = prepass;
+    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
     return CGO_OK;
 }
 
@@ -2396,6 +2473,7 @@ int cgo_time_kernel(cgo_engine* e, int32_t which, const int32_t* ids, int32_t n,
     if (rc) return rc;
     if ((rc = sync_table(e))) return rc;
     if ((rc = upload_lists(e, ls))) return rc;
+    if ((rc = flux_workspace(e, ls))) return rc;
     HIPCHK(e, hipStreamSynchronize(e->s));
     HIPCHK(e, hipEventRecord(e->ev0, e->s));
     if (which == 3) {
@@ -2424,14 +2502,9 @@ int cgo_time_kernel(cgo_engine* e, int32_t which, const int32_t* ids, int32_t n,
             if (!ls.n[p]) continue;
             const int32_t* l = e->d_list + ls.off[p];
             if (which == 0) {
-                if (p == 0)
-                    launch_flux64(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[0], e->nt[0], e->nbuf[0], e->isosplit[0], 3, e->lds_cap,
-                          e->s);
-                else
-                    launch_flux32(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[1], e->nt[1], e->nbuf[1], e->isosplit[1], 3, e->lds_cap,
-                          e->s);
+                if (p == 0 || !ls.n[0]) enqueue_flux(e, ls, e->d_list, 3);  // both precisions
             } else if (which == 1) {
-                launch_co(e->d_table, l, ls.n[p], ls.maxwet[p], ls.maxk[p], p, e->s);
+                launch_co(e->d_table, l, ls.n[p], ls.maxwet[p], ls.maxk[p], p, ls.sp[p], e->s);
             } else if (which == 4) {
                 if (ls.n[2 + p])
                     launch_bio(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.wstream[p], p, e->s);

@@ -58,9 +58,18 @@ __host__ __device__ constexpr int flux_pf(int nt) { return nt == 128 ? 3 : 2; }
 // widest range of a 36x36 mask (266 and 439 positions) so the slots cost no
 // resident blocks; a single column spans 2 maxi + 1 positions.
 __host__ __device__ constexpr int flux_tw(int nt) { return nt == 128 ? 288 : 448; }
-// the flux grid of a batch: blocks and widest tile, per block width (128, 256)
+// the flux grid of a batch: blocks and widest tile, per block width (128,
+// 256), and the deepest grid's levels
 struct FluxShape {
-    int nblk[2], tw[2];
+    int nblk[2], tw[2], maxk;
+};
+// a flux split by levels (kc > 0): levels per block, the batch's column blocks
+// and, per member of the launch's list, `stride` doubles for the new values of
+// an FP32 member with BIOGEM, [L][ncell]
+struct FluxSplit {
+    double* nv;
+    size_t stride;
+    int kc, nbx;
 };
 
 struct GridDev {
@@ -308,6 +317,19 @@ __device__ __forceinline__ BlockXYZ xcd_blk() {
     const int v = xcd_block(dispatch_index(), dispatch_count());
     const int gx = (int)gridDim.x, gy = (int)gridDim.y;
     return BlockXYZ{v % gx, (v / gx) % gy, v / (gx * gy)};
+}
+
+// sum and maximum over a wave's 64 lanes: one atomic per wave instead of one
+// per lane, which a single address takes one after the other
+__device__ __forceinline__ int wave_sum(int v) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
+    return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v = fmax(v, __shfl_xor(v, d));
+    return v;
 }
 
 // unbiased binary exponent of a float, zero and subnormals taken as -126

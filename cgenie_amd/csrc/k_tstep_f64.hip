@@ -7,11 +7,12 @@
 namespace cgo {
 
 void launch_flux64(const MemberDev* t, const int32_t* l, int n, const FluxShape& fs, int maxL, int lb, int nt,
-                   int nbuf, int iso_split, int part, size_t lds_cap, hipStream_t s) {
-    launch_flux_t<double>(t, l, n, fs, maxL, lb, nt, nbuf, iso_split, part, lds_cap, s);
+                   int nbuf, int iso_split, const FluxSplit& sp, int part, size_t lds_cap, hipStream_t s) {
+    launch_flux_t<double>(t, l, n, fs, maxL, lb, nt, nbuf, iso_split, sp, part, lds_cap, s);
 }
 
-void launch_co(const MemberDev* t, const int32_t* l, int n, int nwetmax, int maxkmax, int prec, hipStream_t s) {
+void launch_co(const MemberDev* t, const int32_t* l, int n, int nwetmax, int maxkmax, int prec, const FluxSplit& sp,
+               hipStream_t s) {
     // A large batch (more chunks of CO_CB columns than the chip holds blocks:
     // 4,096) runs one wave per block and up to four chunks per block, so that
     // blocks that find no unstable column are few; a small one runs every
@@ -27,9 +28,9 @@ void launch_co(const MemberDev* t, const int32_t* l, int n, int nwetmax, int max
     const dim3 grid(large ? (chunks + 3) / 4 : chunks, n);
     const size_t lds = co_lds_bytes(nt, KM);
     if (prec == 0)
-        hipLaunchKernelGGL(k_co<double>, grid, dim3(nt), lds, s, t, l, KM);
+        hipLaunchKernelGGL(k_co<double>, grid, dim3(nt), lds, s, t, l, KM, sp);
     else
-        hipLaunchKernelGGL(k_co<float>, grid, dim3(nt), lds, s, t, l, KM);
+        hipLaunchKernelGGL(k_co<float>, grid, dim3(nt), lds, s, t, l, KM, sp);
 }
 
 void launch_flip(const MemberDev* t, const int32_t* l, int n, hipStream_t s) {

@@ -147,9 +147,18 @@ __device__ __forceinline__ float carry_residual(float h, int16_t c) {
 // block per column block, T and S only, LB = 2) that computes them once per
 // cell into the member's isoc planes; 2 the tracer blocks after that pre-pass,
 // which load them and stage only their own tracers.
-template <typename R, int LB, int FLUX_THREADS, int FLUX_NBUF, int IM>
+// MODE 3 is mode 0 for a batch too small to fill the chip with blocks that
+// march whole columns: blockIdx.x also runs over chunks of sp.kc levels.  A
+// block first forms the level under its chunk without storing it, for the
+// flux through its own bottom face.  What a march carries up a whole column,
+// the stability of the new density and the coupling's column sums, is left
+// to co, which then takes every column (FP32 members hand it their new values
+// unrounded, as the march sums them).
+template <typename R, int LB, int FLUX_THREADS, int FLUX_NBUF, int MODE>
 __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restrict__ mems,
-                                                       const int32_t* __restrict__ list) {
+                                                       const int32_t* __restrict__ list, FluxSplit sp_) {
+    constexpr bool SPLIT = MODE == 3;
+    constexpr int IM = SPLIT ? 0 : MODE;
     constexpr int NS = IM == 0 ? LB + 2 : LB;  // slots per staged level plane
     constexpr int TWS = flux_tw(FLUX_THREADS);  // positions per slot (>= every block's t1 - t0)
     extern __shared__ __align__(16) unsigned char smem[];
@@ -159,11 +168,12 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
     const int maxi = g.maxi, maxj = g.maxj, maxk = g.maxk, L = M.L;
     constexpr int V = FLUX_THREADS == 256 ? 1 : 0;
     const int l0 = B.y * LB;
-    if (B.x >= g.nfblk[V] || l0 >= L) return;  // uniform for the block
+    const int bx = SPLIT ? B.x % sp_.nbx : B.x;
+    if (bx >= g.nfblk[V] || l0 >= L) return;  // uniform for the block
     // every wet column's sums are formed below
-    if (IM != 1 && M.bgc && B.x == 0 && B.y == 0 && threadIdx.x == 0) *gp(M.sfresh) = 1;
+    if (!SPLIT && IM != 1 && M.bgc && B.x == 0 && B.y == 0 && threadIdx.x == 0) *gp(M.sfresh) = 1;
     const int nl = (L - l0) < LB ? (L - l0) : LB;
-    const AS_GLOBAL FluxBlk* blk = gp(g.fblk[V]) + B.x;
+    const AS_GLOBAL FluxBlk* blk = gp(g.fblk[V]) + bx;
     const int w0 = blk->w0, t0 = blk->t0, TW = blk->t1 - t0, nw = blk->w1 - w0;
     int* sk1 = reinterpret_cast<int*>(smem);
     R* sp = reinterpret_cast<R*>(smem + (size_t)TWS * 4);
@@ -190,8 +200,10 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
     const int k1n = k1at(g, I, J + 1), k1s = k1at(g, I, J - 1);
     if (k1c <= maxk) atomicMin(&s_kmin, k1c);
     __syncthreads();
-    const int kmin = s_kmin;
-    if (kmin > maxk) return;  // every column of the block is land
+    // the block's levels [klo, khi], entered at kmin: the level under klo where it has one
+    const int klo = SPLIT ? 1 + (B.x / sp_.nbx) * sp_.kc : 1, khi = SPLIT ? min(maxk, klo + sp_.kc - 1) : maxk;
+    const int kmin = SPLIT ? max(s_kmin, klo - 1) : s_kmin;
+    if (kmin > khi) return;  // no wet cell in the block's levels
 
     constexpr bool ANOM = sizeof(R) == 4;  // FP32 form: fluxes of q - q_cell plus q_cell * div(u)
     const int par = *gp(M.parity);
@@ -340,13 +352,13 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
             const double ssmax = mkD[MK_SSMAX * KS + k];
             if (tv1 > ssmax) {
                 slim = fdiv(ssmax * ssmax, tv1 * tv1);
-                limps++;
+                if (!SPLIT || k >= klo) limps++;
             } else {
                 slim = 1;
             }
             tv1 = tv1 * slim * diff1D * rdza;
             const double tvd = tv1 * dt * rdza;
-            if (tvd > dmaxv) dmaxv = tvd;
+            if (tvd > dmaxv && (!SPLIT || k >= klo)) dmaxv = tvd;
         }
     };
     // the FP32 form's isoneutral coefficients: corner differences times ax, ay
@@ -375,7 +387,9 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
     // Members with BIOGEM: the coupling's column sums of the new state
     // (biogem.f90:1984-1997, 2016-2025), accumulated up the column in the
     // order the coupling adds them; co redoes the columns it mixes.
-    const bool sums = IM != 1 && M.bgc != 0;
+    const bool sums = !SPLIT && IM != 1 && M.bgc != 0;
+    AS_GLOBAL double* const nvs =
+        SPLIT && ANOM && M.bgc ? gp(sp_.nv) + (size_t)B.z * sp_.stride : nullptr;  // [L][ncell]: co's sums
     const double rSold = sums ? 1.0 / gp(M.scal)[SC_SMEAN] : 0.0;
     double accs[LB], accS = 0.0;
 #pragma unroll
@@ -396,11 +410,12 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
         commit((kmin + 1) % FLUX_NBUF);
     }
     __syncthreads();
-    for (int k = kmin; k <= maxk; k++) {
+    for (int k = kmin; k <= khi; k++) {
         const int kz = k - 1;
         const int cb = k % FLUX_NBUF, ub = (k + 1) % FLUX_NBUF;
         const bool top = (k == maxk);
-        const bool more = k + 2 <= maxk;
+        const bool more = k + 2 <= (SPLIT ? min(khi + 1, maxk) : maxk);
+        const bool own = !SPLIT || k >= klo;
         if (more) fetch(kz + 2);
         if (IM == 1 && active && k >= k1c && !top && M.diso) {
             // the pre-pass: the cell's isoneutral coefficients, once
@@ -545,12 +560,13 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
                         // compensated accumulation: the rounding residual of every
                         // update is carried to the next step in the int16 plane
                         nv = ((double)Tc + (double)SR(cb, q, p)) + (double)inc + incs;
-                        StateIO<R>::st((R*)dst, lo_dst, idx, nv);
+                        if (own) StateIO<R>::st((R*)dst, lo_dst, idx, nv);
                     } else {
                         const R v = Tc + (inc + (R)incs);
-                        at(dst, (uint32_t)idx) = v;
+                        if (own) at(dst, (uint32_t)idx) = v;
                         nv = (double)v;
                     }
+                    if (SPLIT && own && nvs) at(nvs, (uint32_t)idx) = nv;
                     FB(q) = fbn;
                     if (l0 + q == 0) newT = nv;
                     if (l0 + q == 1) newS = nv;
@@ -627,7 +643,7 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
                     FB(q) = fbn;
                 } else {
                     const R v = Tc - dt * div;
-                    at(dst, (uint32_t)idx) = v;
+                    if (own) at(dst, (uint32_t)idx) = v;
                     nv = (double)v;
                     FB(q) = fa;
                 }
@@ -635,7 +651,7 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
                 if (l0 + q == 1) newS = nv;
                 if (sums) add_sum(q, nv, s_os, s_mm, s_vv);
             }
-            if (l0 == 0) {
+            if (l0 == 0 && own) {
                 const double rn = eos<double>(g.ec[0], g.ec[1], g.ec[2], g.ec[3], newT, newS);
                 at(rhop, oc) = rn;
                 falls = falls & (k == k1c || rn < rlow);
@@ -646,7 +662,7 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
         if (more) commit((k + 2) % FLUX_NBUF);
         __syncthreads();
     }
-    if (IM != 1 && l0 == 0) {
+    if (!SPLIT && IM != 1 && l0 == 0) {
         // co's columns: this block's segment [w0, w1) of the member's list,
         // its unstable columns first, in column order
         constexpr int NW = FLUX_THREADS / 64;
@@ -668,9 +684,13 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
             if (B.x == 0) gp(M.useg)[0] = g.nfblk[V];
         }
     }
-    if (IM != 2 && l0 == 0 && M.diso && active) {
-        if (limps) atomicAdd(&M.diag[0], limps);
-        if (dmaxv > 0.0) atomic_max_pos(M.dmax, dmaxv);
+    if (IM != 2 && l0 == 0 && M.diso) {
+        limps = wave_sum(limps);
+        dmaxv = wave_max(dmaxv);
+        if ((tid & 63) == 0) {
+            if (limps) atomicAdd(&M.diag[0], limps);
+            if (dmaxv > 0.0) atomic_max_pos(M.dmax, dmaxv);
+        }
     }
     if (sums && active && k1c <= maxk) {
         const int slot = gp(g.cslot)[col];
@@ -692,8 +712,14 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
 // ring shrink until the workgroup fits the LDS the device grants one block.
 template <typename R>
 void launch_flux_t(const MemberDev* t, const int32_t* l, int n, const FluxShape& fs, int maxL, int lb, int nt,
-                   int nbuf, int iso_split, int part, size_t lds_cap, hipStream_t s) {
+                   int nbuf, int iso_split, const FluxSplit& sp, int part, size_t lds_cap, hipStream_t s) {
     constexpr int es = sizeof(R);
+    if (sp.kc > 0) {
+        if (!(part & 2) || fs.nblk[1] == 0) return;
+        const dim3 grid(sp.nbx * ((fs.maxk + sp.kc - 1) / sp.kc), (maxL + 1) / 2, n);
+        hipLaunchKernelGGL((k_flux<R, 2, 256, 2, 3>), grid, dim3(256), flux_lds_bytes(4, 2, es, 256, 2), s, t, l, sp);
+        return;
+    }
     if (nt != 256) nt = 128;
     if (nbuf != 2) nbuf = 3;
     auto bytes = [&](int ns, int b) { return flux_lds_bytes(ns, b, es, nt, nbuf); };
@@ -706,7 +732,7 @@ void launch_flux_t(const MemberDev* t, const int32_t* l, int n, const FluxShape&
     const dim3 grid(fs.nblk[v], (maxL + lb - 1) / lb, n);
     const size_t lds = bytes(slots(), lb);
 #define CGO_FLUX(LB_, NT_, NB_, IM_) \
-    hipLaunchKernelGGL((k_flux<R, LB_, NT_, NB_, IM_>), grid, dim3(NT_), lds, s, t, l)
+    hipLaunchKernelGGL((k_flux<R, LB_, NT_, NB_, IM_>), grid, dim3(NT_), lds, s, t, l, sp)
 #define CGO_FLUX_LB(NT_, NB_, IM_)                    \
     do {                                              \
         if (lb == 2) CGO_FLUX(2, NT_, NB_, IM_);      \
@@ -720,11 +746,11 @@ void launch_flux_t(const MemberDev* t, const int32_t* l, int n, const FluxShape&
         if (part & 1) {
         const size_t lds1 = bytes(2, 2);
         if (nt == 256) {
-            if (nbuf == 2) hipLaunchKernelGGL((k_flux<R, 2, 256, 2, 1>), g1, dim3(256), lds1, s, t, l);
-            else hipLaunchKernelGGL((k_flux<R, 2, 256, 3, 1>), g1, dim3(256), lds1, s, t, l);
+            if (nbuf == 2) hipLaunchKernelGGL((k_flux<R, 2, 256, 2, 1>), g1, dim3(256), lds1, s, t, l, sp);
+            else hipLaunchKernelGGL((k_flux<R, 2, 256, 3, 1>), g1, dim3(256), lds1, s, t, l, sp);
         } else {
-            if (nbuf == 2) hipLaunchKernelGGL((k_flux<R, 2, 128, 2, 1>), g1, dim3(128), lds1, s, t, l);
-            else hipLaunchKernelGGL((k_flux<R, 2, 128, 3, 1>), g1, dim3(128), lds1, s, t, l);
+            if (nbuf == 2) hipLaunchKernelGGL((k_flux<R, 2, 128, 2, 1>), g1, dim3(128), lds1, s, t, l, sp);
+            else hipLaunchKernelGGL((k_flux<R, 2, 128, 3, 1>), g1, dim3(128), lds1, s, t, l, sp);
         }
         }
         if (!(part & 2)) {
@@ -778,7 +804,8 @@ __host__ __device__ constexpr size_t co_lds_bytes(int nt, int KM) {
     return (size_t)nt * KM * 8 + (size_t)CO_CB * 2 * KM * (8 + 1) + (size_t)CO_CB * (8 + 3 * 4);
 }
 template <typename R>
-__global__ __launch_bounds__(CO_NT) void k_co(const MemberDev* __restrict__ mems, const int32_t* __restrict__ list, int KM) {
+__global__ __launch_bounds__(CO_NT) void k_co(const MemberDev* __restrict__ mems, const int32_t* __restrict__ list, int KM,
+                                               FluxSplit sp_) {
     constexpr int CB = CO_CB;
     extern __shared__ double co_lds[];
     const BlockXYZ B = xcd_blk();
@@ -786,11 +813,13 @@ __global__ __launch_bounds__(CO_NT) void k_co(const MemberDev* __restrict__ mems
     const GridDev& g = M.g;
     const int nt = (int)blockDim.x, tid = (int)threadIdx.x;
     const int maxi = g.maxi, maxk = g.maxk, L = M.L;
+    const bool every = sp_.kc > 0;  // after a flux split by levels: every wet column
     const AS_GLOBAL int32_t* useg = gp(M.useg);
-    const int nseg = useg[0];
-    int total = 0;  // unstable columns of the member
+    const int nseg = every ? 0 : useg[0];
+    int total = every ? g.nwet : 0;  // the member's columns
     for (int q = 0; q < nseg; q++) total += useg[2 + 2 * q];
     if (B.x * CB >= total && !M.sw) return;  // uniform for the block
+    if (every && M.bgc && B.x == 0 && tid == 0) *gp(M.sfresh) = 1;
     const int par = *gp(M.parity);
     void* st = M.st[par ^ 1];
     int16_t* lo = M.lo[par ^ 1];
@@ -816,6 +845,7 @@ __global__ __launch_bounds__(CO_NT) void k_co(const MemberDev* __restrict__ mems
     };
     // the column at place p of the segments' unstable or stable parts
     auto place = [&](int p, bool stable) -> int {
+        if (every) return gp(g.wetsorted)[p];
         for (int q = 0; q < nseg; q++) {
             const int w0 = useg[1 + 2 * q], nu = useg[2 + 2 * q];
             const int w1 = q + 1 < nseg ? useg[3 + 2 * q] : g.nwet;
@@ -931,6 +961,7 @@ __global__ __launch_bounds__(CO_NT) void k_co(const MemberDev* __restrict__ mems
             const int i = x % n, l = x / n;
             const int k1 = lk1[i], col = lcol[i], ne = lne[i];
             const uint64_t tops = ltops[i];
+            if (ne == 0 && !(l >= 1 && M.bgc) && !(l < 2 && M.sw)) continue;
             const uint32_t base = (uint32_t)l * tstride + col;
             for (int k0 = k1; k0 <= maxk; k0 += 8) {
                 typename StateIO<R>::Raw q[8];
@@ -973,28 +1004,31 @@ __global__ __launch_bounds__(CO_NT) void k_co(const MemberDev* __restrict__ mems
             }
             if (l < 2) snap(l == 0 ? SW_TSTAR : SW_SSTAR, col, v[(maxk - 1) * nt]);
             if (M.bgc && l >= 1) {
-                // the coupling's column sums of this column after mixing and fill-in
+                // the coupling's column sums of this column after mixing and
+                // fill-in, or those the flux leaves to this kernel: the FP32
+                // form sums its new values before they are rounded, each
+                // product added in one rounding
+                const bool unr = sizeof(R) == 4 && ne == 0;
+                const AS_GLOBAL double* nvs =
+                    unr ? gp(sp_.nv) + (size_t)B.y * sp_.stride + base : nullptr;
                 const uint32_t ncl = (uint32_t)g.ncell;
                 double a = 0.0;
                 for (int k0 = k1; k0 <= maxk; k0 += 4) {
-                    double f0[4], f1[4];
+                    double f0[4], f1[4], xv[4];
 #pragma unroll
                     for (int u = 0; u < 4; u++)
                         if (k0 + u <= maxk) {
-                            const uint32_t c = (uint32_t)(k0 + u - 1) * plane + col;
+                            const uint32_t o = (uint32_t)(k0 + u - 1) * plane, c = o + col;
                             f0[u] = l == 1 ? at(gp(g.V), c) : at(gp(M.ocn), ncl + c);
                             f1[u] = l == 1 ? 0.0 : at(gp(M.M), c);
+                            xv[u] = unr ? at(nvs, o) : v[(k0 + u - 1) * nt];
                         }
 #pragma unroll
                     for (int u = 0; u < 4; u++)
                         if (k0 + u <= maxk) {
-                            const double xv = v[(k0 + u - 1) * nt];
-                            if (l == 1) {
-                                a += (xv + SALN0 + 0.0) * f0[u];
-                            } else {
-                                const double lv = xv * f0[u] * rSold;
-                                a += lv * f1[u];
-                            }
+                            const double x1 = l == 1 ? xv[u] + SALN0 + 0.0 : xv[u] * f0[u] * rSold;
+                            const double x2 = l == 1 ? f0[u] : f1[u];
+                            a = unr ? __builtin_fma(x1, x2, a) : a + x1 * x2;
                         }
                 }
                 gp(M.colsum)[(size_t)(l == 1 ? 0 : l) * g.nwet + gp(g.cslot)[col]] = a;

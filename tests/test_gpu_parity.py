@@ -478,3 +478,49 @@ def test_convection_at_its_edges(dims, L, precision, n):
     else:
         alone = run(1)[0]
         assert np.array_equal(got[0][0], alone[0]) and got[0][2] == alone[2]
+
+
+@pytest.mark.parametrize("dims,kind,L,prec,carry,n", [
+    ((36, 36, 16), "config2", 9, E.FP64, True, 1), ((36, 36, 16), "config2", 9, E.FP32C, True, 1),
+    ((13, 11, 7), "domc", 8, E.FP32C, True, 3), ((13, 11, 7), "domc", 8, E.FP32C, False, 2),
+    ((20, 9, 2), "ts", 2, E.FP64, True, 1), ((72, 40, 9), "config2", 11, E.FP32C, True, 5),
+    ((18, 18, 8), "config2", 7, E.FP32C, True, 40)])
+def test_split_flux_equals_whole_columns(dims, kind, L, prec, carry, n):
+    """Small batches take the flux split by levels, with every column's sums
+    and stability formed in the convection; setting a tile takes whole columns
+    with the pre-pass.  Both give the same bits: state, density, convection
+    counts, the slope limiter's count and the largest diffusion number, eager
+    and from a replayed graph, one and many levels per chunk, a remainder of
+    levels, FP32 members with and without the carry."""
+    c = make_case(*dims, kind=kind, L=L, seed=53, sflux=True)
+
+    def run(tile, graph):
+        eng = E.Engine(0)
+        if tile:
+            eng.set_tile(prec, *tile)
+        gid = eng.add_grid(c.g, c.k1)
+        ids = []
+        for q in range(n):
+            m = eng.add_member(gid, L, prec, c.diff, diso=True, carry=carry)
+            eng.set_velocity(m, c.u * (1.0 - 0.1 * (q % 4)))
+            eng.set_sflux(m, c.sflux)
+            eng.upload(m, c.ts)
+            if kind != "ts":
+                eng.bgc_init(m, E.default_bgc_params(1.0 / 96, c.tset), c.light, c.mld)
+            ids.append(m)
+        if graph:
+            gr = eng.capture(ids, 3)
+            eng.launch(gr, 2)
+        else:
+            eng.step(ids, 6)
+        out = []
+        for m in (ids[0], ids[-1]):
+            d = eng.diag(m)
+            out.append((eng.download(m, c.ts.shape), eng.rho(m, c.g), (d.limps, d.dmax, d.cost, d.smean)))
+        eng.close()
+        return out
+
+    want = run((4, 256, 2, 1), False)
+    for got in (run(None, False), run(None, True)):
+        for a, b in zip(got, want):
+            assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]) and a[2] == b[2]
