@@ -27,7 +27,7 @@ void launch_co(const MemberDev*, const int32_t*, int nlist, int nwetmax, int max
 void launch_flip(const MemberDev*, const int32_t*, int nlist, hipStream_t);
 void launch_bio(const MemberDev*, const int32_t*, int nlist, int nwetmax, int W, int prec, hipStream_t);
 void launch_coupling(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int maxL, int prec,
-                     size_t lds_cap, int phase, hipStream_t);
+                     int phase, hipStream_t);
 void launch_inventory(const MemberDev*, int32_t member, int L, double* out, const double* w, int prec, hipStream_t);
 void launch_carbconst_surface(const MemberDev*, int32_t member, int nwet, double* out, hipStream_t);
 void launch_atchem(const MemberDev*, const int32_t*, int nlist, int ncolmax, hipStream_t);
@@ -2169,7 +2169,7 @@ static void enqueue_coupling(cgo_engine* e, const Lists& ls, const int32_t* d_li
     for (int p = 0; p < 2; p++)
         if (ls.n[2 + p])
             launch_coupling(e->d_table, d_lists + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.maxk_bgc[p],
-                            ls.maxL[p], p, e->lds_cap, phase, e->s);
+                            ls.maxL[p], p, phase, e->s);
 }
 
 // Whole ocean steps in the genie.f90 order.  step_biogem reads only BIOGEM's
@@ -2511,7 +2511,7 @@ int cgo_time_kernel(cgo_engine* e, int32_t which, const int32_t* ids, int32_t n,
             } else if (ls.n[2 + p]) {
                 launch_bio(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.wstream[p], p, e->s);
                 launch_coupling(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.maxk_bgc[p],
-                                ls.maxL[p], p, e->lds_cap, 0, e->s);
+                                ls.maxL[p], p, 0, e->s);
             }
         }
     HIPCHK(e, hipEventRecord(e->ev1, e->s));

@@ -15,8 +15,8 @@
 // k_couple_sums    one block per (member, 64 wet columns): the column partial
 //             sums of the state after transport (biogem.f90:1984-1997,
 //             2016-2025).
-// k_couple_reduce  one block per member: the global sums, in the reference's
-//             column order (biogem.f90:1927-2031), staged through LDS.
+// k_couple_reduce  one block per (member, three tracers): the global sums, in the
+//             reference's column order (biogem.f90:1927-2031), staged through LDS.
 // k_couple_apply   one block per (member, 64 wet columns): the rescale and
 //             re-normalisation of every tracer, T, S, masses and
 //             particulates (2001-2061).
@@ -611,82 +611,91 @@ __global__ __launch_bounds__(CPL_THREADS) void k_couple_sums(const MemberDev* __
 }
 
 // global sums in the reference's column order (partialtot(n) summed over
-// n = 1..n_vocn, biogem.f90:1927-2031), then the coupling scalars.  The
-// block stages a chunk of columns of every partial-sum row in LDS, then each
-// sum is one thread's sequential pass over its row of the chunk; chunks go in
-// column order, so every sum is added in the reference's order.
-constexpr int RED_THREADS = 1024;  // one block per member: many loads in flight per chunk
-constexpr int RED_LDS_BYTES = 128 * 1024;
-constexpr int RED_MAXL = 256;
+// n = 1..n_vocn, biogem.f90:1927-2031), then the coupling scalars.  A block
+// per member and RED_T tracers: the NEW and OLD sum of each (the first block
+// also takes S), every sum one lane's sequential pass over its row, staged in
+// LDS a chunk of columns at a time, the next chunk's loads in flight while one
+// is added.  Bound by that chain of adds (8 cycles each) and the first
+// chunk's load.  One block per member for all sums staged its rows in large
+// rounds that nothing overlapped: one 36x36x16x24 member 23.5 -> 9.1 us, six of
+// 72x72x32x40 130 -> 32 us, 256 members 34 us as before.
+constexpr int RED_THREADS = 256;
+constexpr int RED_T = 3;                    // tracers per block
+constexpr int RED_ROWS = 2 * RED_T + 1;     // sums per block: S first, then NEW and OLD of each tracer
+constexpr int RED_CH = 512;                 // columns per chunk
+constexpr int RED_RS = RED_CH + 18;         // a row's stride in LDS: even (16-byte reads), past the last chunk's read-ahead
+constexpr int RED_PF = RED_ROWS * RED_CH / RED_THREADS;
 
 __global__ __launch_bounds__(RED_THREADS) void k_couple_reduce(const MemberDev* __restrict__ mems,
-                                                               const int32_t* __restrict__ list, int lds_bytes) {
-    extern __shared__ double rows[];
-    __shared__ double s_val[2 * RED_MAXL];
-    const MemberDev& M = mems[list[blockIdx.x]];
+                                                               const int32_t* __restrict__ list) {
+    __shared__ __align__(16) double rows[RED_ROWS * RED_RS];
+    __shared__ double s_val[RED_ROWS];
+    const MemberDev& M = mems[list[blockIdx.y]];
     const int nwet = M.g.nwet, L = M.L;
-    // sum q: 0 -> S (scaled by 1/Vtot), 1 + (l-2) -> NEW_l, L-1 + (l-2) -> OLD_l
-    const int nsum = 1 + 2 * (L - 2);
-    auto src = [&](int q) -> const AS_GLOBAL double* {
-        if (q == 0) return gp(M.colsum);
-        if (q < L - 1) return gp(M.colsum) + (size_t)(q + 1) * nwet;
-        return gp(M.colold) + (size_t)(q - L + 3) * nwet;
-    };
-    int ch = lds_bytes / (8 * nsum);   // columns per chunk, odd (LDS banks)
-    if (ch > nwet) ch = nwet;
-    if ((ch & 1) == 0) ch -= 1;
-    if (ch < 1) ch = 1;
+    const int l0 = 2 + (int)blockIdx.x * RED_T;   // the block's first tracer
+    if (l0 >= L && blockIdx.x > 0) return;        // uniform for the block
+    const int nl = L - l0 < RED_T ? L - l0 : RED_T;
     const int t = threadIdx.x;
+    // row q: 0 -> S (the first block), 1 + 2 i -> NEW of tracer l0 + i, 2 + 2 i -> its OLD
+    const AS_GLOBAL double* const sums = gp(M.colsum);
+    const AS_GLOBAL double* const olds = gp(M.colold);
     const double sc = M.g.rVtot;
-    double tot0 = 0.0, tot1 = 0.0;  // sums t and t + RED_THREADS
-    for (int c0 = 0; c0 < nwet; c0 += ch) {
-        const int n = nwet - c0 < ch ? nwet - c0 : ch;
-        // stage nsum x n values, eight loads in flight per thread
-        const int tot = nsum * n;
-        for (int b0 = t; b0 < tot; b0 += RED_THREADS * 8) {
-            double v[8];
-            int at[8];
+    double pf[RED_PF];
+    auto fetch = [&](int c0) {
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const int idx = b0 + u * RED_THREADS;
-                if (idx < tot) {
-                    const int q = idx / n, i = idx - q * n;
-                    v[u] = src(q)[c0 + i];
-                    at[u] = q * ch + i;
-                }
+        for (int u = 0; u < RED_PF; u++) {
+            const int x = t + u * RED_THREADS, q = x / RED_CH, c = c0 + x % RED_CH, i = (q - 1) >> 1;
+            if (c < nwet && (q == 0 ? blockIdx.x == 0 : i < nl)) {
+                const uint32_t row = q == 0 ? 0u : (uint32_t)(l0 + i) * (uint32_t)nwet;
+                pf[u] = at((q & 1) || q == 0 ? sums : olds, row + (uint32_t)c);
             }
+        }
+    };
+    auto commit = [&]() {
 #pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (b0 + u * RED_THREADS < tot) rows[at[u]] = v[u];
+        for (int u = 0; u < RED_PF; u++) {
+            const int x = t + u * RED_THREADS;
+            rows[(x / RED_CH) * RED_RS + x % RED_CH] = x / RED_CH == 0 ? pf[u] * sc : pf[u];
+        }
+    };
+    const bool mine = t < RED_ROWS && (t == 0 ? blockIdx.x == 0 : (t - 1) >> 1 < nl);
+    double tot = 0.0;
+    fetch(0);
+    for (int c0 = 0; c0 < nwet; c0 += RED_CH) {
+        commit();
+        __syncthreads();
+        if (c0 + RED_CH < nwet) fetch(c0 + RED_CH);
+        if (mine) {
+            const double* r = rows + t * RED_RS;
+            const int n = nwet - c0 < RED_CH ? nwet - c0 : RED_CH;
+            // eight columns are added while the next eight are read
+            double v[8], w[8];
+            auto read = [&](double* d, int i) {
+#pragma unroll
+                for (int u = 0; u < 8; u++) d[u] = r[i + u];
+            };
+            read(v, 0);
+            int i = 0;
+            for (; i + 16 <= n; i += 16) {
+                read(w, i + 8);
+#pragma unroll
+                for (int u = 0; u < 8; u++) tot += v[u];
+                read(v, i + 16);
+#pragma unroll
+                for (int u = 0; u < 8; u++) tot += w[u];
+            }
+            for (; i < n; i++) tot += r[i];
         }
         __syncthreads();
-        // each sum adds its columns in order; the LDS reads of eight columns
-        // are issued before the first of their adds
-        auto run = [&](const double* r, double tot, double f, bool scaled) {
-            int i = 0;
-            for (; i + 8 <= n; i += 8) {
-                double v[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = r[i + u];
-#pragma unroll
-                for (int u = 0; u < 8; u++) tot += scaled ? v[u] * f : v[u];
-            }
-            for (; i < n; i++) tot += scaled ? r[i] * f : r[i];
-            return tot;
-        };
-        if (t < nsum) tot0 = run(rows + t * ch, tot0, sc, t == 0);
-        if (t + RED_THREADS < nsum) tot1 = run(rows + (t + RED_THREADS) * ch, tot1, 1.0, false);
-        __syncthreads();
     }
-    if (t < nsum) s_val[t] = tot0;
-    if (t + RED_THREADS < nsum) s_val[t + RED_THREADS] = tot1;
+    if (mine) s_val[t] = tot;
     __syncthreads();
-    for (int l = 2 + t; l < L; l += RED_THREADS) {
-        const double nw = s_val[l - 1];
+    if (t < nl) {
+        const double nw = s_val[1 + 2 * t];
         const double rnew = fabs(nw) < NULLSMALL ? 0.0 : 1.0 / nw;
-        gp(M.scal)[SC_FACT0 + l] = s_val[L - 3 + l] * rnew;
+        gp(M.scal)[SC_FACT0 + l0 + t] = s_val[2 + 2 * t] * rnew;
     }
-    if (t == 0) {
+    if (t == 0 && blockIdx.x == 0) {
         const double Sold = gp(M.scal)[SC_SMEAN];
         const double Snew = s_val[0];
         const double Sratio = Snew / Sold;
@@ -703,10 +712,13 @@ __global__ __launch_bounds__(RED_THREADS) void k_couple_reduce(const MemberDev* 
 // (2001-2013), the new cell masses (2049-2052) and the particulates
 // (2042-2043).  The block owns its cells, so the old salinity and masses the
 // tracers need are read before the same threads rewrite them.
-template <typename R, int NJ, int TG>  // NJ cells per thread (NJ * CPL_LG >= maxk), TG >= tg
-__global__ __launch_bounds__(CPL_THREADS) void k_couple_apply(const MemberDev* __restrict__ mems,
-                                                              const int32_t* __restrict__ list) {
-    extern __shared__ double prod[];  // [tg][maxk][CPL_COLS]
+// A block holds TL groups of CPL_THREADS threads, each with its own tracers
+// (every TL-th): small batches take several, so that a block's chain of
+// rounds, two barriers and a column sum each, is TL times shorter.
+template <typename R, int NJ, int TG, int TL>  // NJ cells per thread (NJ * CPL_LG >= maxk), TG >= tg
+__global__ __launch_bounds__(CPL_THREADS * TL) void k_couple_apply(const MemberDev* __restrict__ mems,
+                                                                   const int32_t* __restrict__ list, int lds_stride) {
+    extern __shared__ double prod_all[];  // [TL][tg][maxk][CPL_COLS]
     __shared__ CplTile T;
     const BlockXYZ B = xcd_blk();
     const MemberDev& M = mems[list[B.y]];
@@ -715,7 +727,9 @@ __global__ __launch_bounds__(CPL_THREADS) void k_couple_apply(const MemberDev* _
     if (w0 >= g.nwet) return;  // uniform over the block
     cpl_tile(g, w0, T);
     const BgcParams& p = M.bp;
-    const int c = threadIdx.x % CPL_COLS, lg = threadIdx.x / CPL_COLS;
+    const int tl = (int)threadIdx.x / CPL_THREADS, tx = (int)threadIdx.x % CPL_THREADS;
+    const int c = tx % CPL_COLS, lg = tx / CPL_COLS;
+    double* const prod = prod_all + (size_t)tl * lds_stride;
     const int maxk = g.maxk, L = M.L, tg = cpl_tg(maxk) < TG ? cpl_tg(maxk) : TG;
     const int col = T.col[c], kb = T.kb[c];
     const size_t plane = (size_t)g.ncol, ncell = (size_t)g.ncell, tstride = (size_t)maxk * plane;
@@ -749,7 +763,8 @@ __global__ __launch_bounds__(CPL_THREADS) void k_couple_apply(const MemberDev* _
             }
         }
     }
-    for (int l0 = 2; l0 < L; l0 += tg) {
+    for (int lb = 2; lb < L; lb += tg * TL) {
+        const int l0 = lb + tl * tg;  // past L for the last round's idle groups
         // all loads of the group first, then the rescale
         typename StateIO<R>::Raw lv[TG][NJ];
         double vv[TG][NJ];
@@ -806,6 +821,10 @@ __global__ __launch_bounds__(CPL_THREADS) void k_couple_apply(const MemberDev* _
             }
         }
         __syncthreads();
+    }
+    if (TL > 1) {
+        __syncthreads();       // every group has read its cells' old salinity and masses
+        if (tl > 0) return;
     }
     // the state changes below: the next coupling's sums come from the next transport step
     if (B.x == 0 && threadIdx.x == 0) {
@@ -953,7 +972,7 @@ template <typename R>
 // phase 1: column sums (if stale) and the global sums; phase 2: the rescale;
 // phase 0: both; phase 3: the global sums alone (right after a transport step)
 static void launch_coupling_t(const MemberDev* mems, const int32_t* list, int nlist, int nwetmax, int maxkmax,
-                              size_t lds_cap, int phase, hipStream_t s) {
+                              int maxL, int phase, hipStream_t s) {
     const dim3 grid((nwetmax + CPL_COLS - 1) / CPL_COLS, nlist);
     // LDS for the largest grid of the batch; every member's tg fits in it
     const size_t lds = (size_t)cpl_tg(maxkmax) * maxkmax * CPL_COLS * 8;
@@ -970,27 +989,35 @@ static void launch_coupling_t(const MemberDev* mems, const int32_t* list, int nl
         } else {
             hipLaunchKernelGGL((k_couple_sums<R, 12, 1>), grid, dim3(CPL_THREADS), b, s, mems, list);
         }
-        // the staging chunk takes what LDS the device grants a block, up to RED_LDS_BYTES
-        const int red_lds = (int)std::min<size_t>(RED_LDS_BYTES, lds_cap - 2 * RED_MAXL * sizeof(double));
-        hipLaunchKernelGGL(k_couple_reduce, dim3(nlist), dim3(RED_THREADS), (size_t)red_lds, s, mems, list, red_lds);
+        hipLaunchKernelGGL(k_couple_reduce, dim3(std::max((maxL - 2 + RED_T - 1) / RED_T, 1), nlist),
+                           dim3(RED_THREADS), 0, s, mems, list);
     }
     if (phase == 1 || phase == 3) return;
+    const int st = (int)(b / 8);
+    // a batch of fewer than 512 blocks (two per CU) takes blocks of up to four
+    // groups, as many as the kernel's registers and LDS allow: one FP64 member of
+    // 36x36x16x24 33 -> 17 us, eight FP32C members 45 -> 24, six of 72x72x32x40
+    // (two groups) 157 -> 147.  Larger ones fill the chip either way, and their
+    // small blocks come and go without waiting for 16 waves' room.
+    const bool small = (long long)grid.x * nlist < 512;
+#define CGO_APPLY(NJ_, TL_)                                                                                         \
+    hipLaunchKernelGGL((k_couple_apply<R, NJ_, 1, TL_>), grid, dim3(CPL_THREADS * TL_), b * TL_, s, mems, list, st)
     if (maxkmax <= 4 * CPL_LG) {
-        hipLaunchKernelGGL((k_couple_apply<R, 4, 1>), grid, dim3(CPL_THREADS), b, s, mems, list);
+        if (small) CGO_APPLY(4, 4); else CGO_APPLY(4, 1);
     } else if (maxkmax <= 8 * CPL_LG) {
-        hipLaunchKernelGGL((k_couple_apply<R, 8, 1>), grid, dim3(CPL_THREADS), b, s, mems, list);
+        if (small) CGO_APPLY(8, 2); else CGO_APPLY(8, 1);
     } else {
-        hipLaunchKernelGGL((k_couple_apply<R, 12, 1>), grid, dim3(CPL_THREADS), b, s, mems, list);
+        if (small) CGO_APPLY(12, 2); else CGO_APPLY(12, 1);
     }
+#undef CGO_APPLY
 }
 
 void launch_coupling(const MemberDev* mems, const int32_t* list, int nlist, int nwetmax, int maxkmax, int maxL,
-                     int prec, size_t lds_cap, int phase, hipStream_t s) {
-    (void)maxL;
+                     int prec, int phase, hipStream_t s) {
     if (prec == 0)
-        launch_coupling_t<double>(mems, list, nlist, nwetmax, maxkmax, lds_cap, phase, s);
+        launch_coupling_t<double>(mems, list, nlist, nwetmax, maxkmax, maxL, phase, s);
     else
-        launch_coupling_t<float>(mems, list, nlist, nwetmax, maxkmax, lds_cap, phase, s);
+        launch_coupling_t<float>(mems, list, nlist, nwetmax, maxkmax, maxL, phase, s);
 }
 
 }  // namespace cgo

@@ -524,3 +524,38 @@ def test_split_flux_equals_whole_columns(dims, kind, L, prec, carry, n):
     for got in (run(None, False), run(None, True)):
         for a, b in zip(got, want):
             assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]) and a[2] == b[2]
+
+
+@pytest.mark.parametrize("dims,L,n", [((13, 11, 7), 7, 1), ((72, 40, 9), 9, 1), ((13, 11, 20), 8, 2), ((12, 10, 40), 10, 1),
+                                      ((18, 18, 8), 8, 140)])
+def test_coupling_at_its_edges(dims, L, n):
+    """The coupling's global sums over one chunk of columns, several and a
+    remainder, with tracer counts that leave a block of the sums one, two or
+    three tracers, and the rescale on shallow, middle and deep grids in small
+    batches and a large one: within 1e-12 of the oracle after three steps, and
+    a large batch's members equal to the member alone bit for bit."""
+    c = make_case(*dims, kind="config2", L=L, seed=61)
+
+    def run(m):
+        eng = E.Engine(0)
+        gid = eng.add_grid(c.g, c.k1)
+        ids = []
+        for _ in range(m):
+            ids.append(eng.add_member(gid, L, E.FP64, c.diff))
+            eng.set_velocity(ids[-1], c.u)
+            eng.upload(ids[-1], c.ts)
+            eng.bgc_init(ids[-1], E.default_bgc_params(1.0 / 96, c.tset, carb_tol=1e-12, carb_maxit=1000), c.light, c.mld)
+        eng.step(ids, 3)
+        out = [eng.download(q, c.ts.shape) for q in (ids[0], ids[-1])]
+        eng.close()
+        return out
+
+    got = run(n)
+    assert np.array_equal(got[0], got[1])
+    if n > 2:
+        assert np.array_equal(got[0], run(1)[0])
+    gold = O.GoldsteinOracle(c.og, c.k1, c.ts, c.u)
+    O.BiogemOracle(gold, O.bgc_params(1.0 / 96, c.tset), c.light, c.mld).step(3)
+    err = rel_err(got[0], gold.ts, wet(c))
+    say(dims, L, n, "max rel err", err.max())
+    assert np.all(err <= 1e-12)
