@@ -845,16 +845,11 @@ int cgo_grid_set_momentum(cgo_engine* e, int32_t grid_id, const cgo_momentum_des
             return fail(e, CGO_E_ARG, "grid_set_momentum: %zu island path points, at most %zu", np, mom_ring_terms(n) / 2);
         }
     }
-    // the elimination's multipliers by pivot row and the eliminated band by row
-    std::vector<double> fwd((size_t)std::max(N - 1, 1) * (n + 1), 0.0), bwd((size_t)N * (n + 2), 0.0);
+    // the elimination's multipliers by pivot row and the eliminated band's packed rows
+    std::vector<double> fwd((size_t)std::max(N - 1, 1) * (n + 1), 0.0), brec;
     for (int i = 1; i <= N - 1; i++)
         for (int q = 1; q <= n + 1 && i + q <= N; q++) fwd[(size_t)(i - 1) * (n + 1) + q - 1] = M->RATM(i + q, q);
-    std::vector<uint64_t> bmask(N, 0);
-    for (int i = 1; i <= N; i++)
-        for (int k = 0; k <= n + 1 && i + k <= N; k++) {
-            bwd[(size_t)(i - 1) * (n + 2) + k] = M->GAP(i, n + 2 + k);
-            if (k >= 1 && M->GAP(i, n + 2 + k) != 0.0) bmask[i - 1] |= (uint64_t)1 << (k - 1);
-        }
+    mom_back_rows(*M, mom_back_stride(n), brec);
     // one device buffer: the MomGridDev struct, then its arrays
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -877,8 +872,7 @@ int cgo_grid_set_momentum(cgo_engine* e, int32_t grid_id, const cgo_momentum_des
                  p_drag = add(M->drag.data(), M->drag.size() * 8), p_rtv = add(M->rtv.data(), M->rtv.size() * 8),
                  p_rtv3 = add(M->rtv3.data(), M->rtv3.size() * 8), p_ku = add(M->ku.data(), M->ku.size() * 4),
                  p_mk = add(M->mkv.data(), M->mkv.size() * 4), p_getj = add(M->getj.data(), M->getj.size()),
-                 p_fwd = add(fwd.data(), fwd.size() * 8), p_bwd = add(bwd.data(), bwd.size() * 8),
-                 p_bm = add(bmask.data(), bmask.size() * 8),
+                 p_fwd = add(fwd.data(), fwd.size() * 8), p_brec = add(brec.data(), brec.size() * 8),
                  p_ubisl = add(M->ubisl.data(), M->ubisl.size() * 8), p_psisl = add(M->psisl.data(), M->psisl.size() * 8),
                  p_erisl = add(M->erisl.data(), M->erisl.size() * 8), p_npi = add(M->npi.data(), (size_t)nis * 4),
                  p_lp = add(M->lpisl.data(), M->lpisl.size() * 4), p_ip = add(M->ipisl.data(), M->ipisl.size() * 4),
@@ -921,8 +915,8 @@ int cgo_grid_set_momentum(cgo_engine* e, int32_t grid_id, const cgo_momentum_des
     h.mk = (const int32_t*)at_(p_mk);
     h.getj = (const uint8_t*)at_(p_getj);
     h.fwd = (const double*)at_(p_fwd);
-    h.bwd = (const double*)at_(p_bwd);
-    h.bmask = (const uint64_t*)at_(p_bm);
+    h.brec = (const double*)at_(p_brec);
+    h.dN = M->GAP(N, n + 2);
     h.ubisl = (const double*)at_(p_ubisl);
     h.psisl = (const double*)at_(p_psisl);
     h.erisl = (const double*)at_(p_erisl);

@@ -113,8 +113,9 @@ struct BgcParams {
 //   mk    (0:maxi+1, 0:maxj+1)        getj (maxi, maxj) bytes
 //   fwd   [N-1][n+1]: row i, entry q-1 = ratm(i+q, q), the multiplier that
 //         elimination step i applies to row i+q (0 past row N)
-//   bwd   [N][n+2]:   row i, entry k = gap(i, n+2+k) of the eliminated band
-//   bmask [N]: row i, bit k-1 set where gap(i, n+2+k), k >= 1, is not zero
+//   brec  [N-1][mom_back_stride]: rows N-1 down to 1 of the eliminated band,
+//         packed for the back substitution (mom_back_rows); dN is row N's
+//         diagonal
 //   ubisl isles x (2, 0:maxi+1, 0:maxj), psisl isles x (0:maxi, 0:maxj)
 //   erisl (isles, isles+1) column-major, inverted in place (matinv_gold)
 //   paths (mpi, isles): lpisl, ipisl, jpisl; npi (isles)
@@ -135,8 +136,8 @@ struct MomGridDev {
     const int32_t* mk;
     const uint8_t* getj;
     const double* fwd;
-    const double* bwd;
-    const uint64_t* bmask;
+    const double* brec;
+    double dN;
     const double* ubisl;
     const double* psisl;
     const double* erisl;
@@ -146,6 +147,8 @@ struct MomGridDev {
     const int32_t* jpisl;
     const double* ainv;
 };
+// doubles of a packed row of the back substitution: 5, n - 1 coefficients, n - 1 bytes
+__host__ __device__ constexpr int mom_back_stride(int n) { return 5 + (n - 1) + (n + 6) / 8; }
 constexpr int MOM_MAXISL = 16;   // islands
 constexpr int MOM_DENSE_MAXN = 4096;  // psi points up to which a grid keeps the dense inverse
 constexpr int MOM_SPLITK = 8;         // slices of the dense solve's sums

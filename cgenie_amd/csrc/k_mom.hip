@@ -4,13 +4,14 @@
 // ubarsolv 3500-3565, the island correction with island() of
 // goldstein_lib.f90:186-241 and matmult 3470-3492, velc 3568-3679).
 //
-// Four launches per step over the members with a solve:
+// Five launches per step over the members with a solve:
 //   k_mom_cols_a  per column, many blocks per member: jbar's bottom pressure
 //                 and its integral, and velc's thermal-wind (and top-layer
 //                 Ekman) shear integrated up the column with its depth sum
-//   k_mom_solve   one block per member: the psi forcing (wind + JEBAR), the
-//                 banded substitutions, psi and the barotropic velocities,
-//                 the path integrals round the islands and psibc
+//   k_mom_force   a thread per psi point: the psi forcing (wind + JEBAR)
+//   k_mom_solve   one block per member: the banded substitutions, psi and the
+//                 barotropic velocities, the path integrals round the islands
+//                 and psibc
 //   k_mom_cols_b  velc's barotropic part and relaxation at every open face
 //   k_mom_cols_c  w from continuity and, for an FP32 member, the seven flux
 //                 coefficient planes formed from the FP64 velocities; the
@@ -196,6 +197,47 @@ __global__ __launch_bounds__(MOM_NT) void k_mom_cols_a(const MemberDev* __restri
     V.csum(2, i, j) = sum1;
 }
 
+// ------------------------------------------------------------ the psi forcing
+// The wind part (wind) plus the torque of the bottom pressure where the four
+// columns round a psi point differ in depth (jbar 3256-3313), a thread per
+// point.  It goes to the member's staging for the dense solve (dense) or to
+// its psi array, which k_mom_solve reads before it writes psi there.  Formed
+// inside the solve's one block per member it took 50 us for one member and 58-120
+// beside the BIOGEM kernel for 96; a launch of its own takes 11 and 21.
+__global__ __launch_bounds__(MOM_NT) void k_mom_force(const MemberDev* __restrict__ mems,
+                                                      const int32_t* __restrict__ list, int dense) {
+    const MomView V(mems[list[blockIdx.y]]);
+    const MomGridDev& G = V.G;
+    const int mi = V.mi, mj = V.mj, n = V.n, N = V.N, l = blockIdx.x * MOM_NT + threadIdx.x + 1;
+    if (l > N) return;
+    const double rdphi = G.rdphi;
+    const int i = (l - 1) % n + 1, j = (l - 1) / n;
+    double g = V.W[V.ML.gbw + l - 1];
+    if (j >= 1 && j <= mj - 1 && G.getj[V.col(i, j)]) {
+        const int ip1 = i % mi + 1;
+        auto span = [&](int k0, int k1_, int ii, int jj) {
+            double t = 0;
+            for (int k = k0; k <= k1_; k++) t = t + V.bp(ii, jj, k) * G.dz[k];
+            return t;
+        };
+        double tv1 = span(V.ku(2, ip1, j), V.mkk(ip1, j + 1), ip1, j + 1);
+        double tv2 = span(V.ku(2, ip1, j), V.mkk(ip1, j), ip1, j);
+        double tv3 = span(V.ku(2, i, j), V.mkk(i, j + 1), i, j + 1);
+        double tv4 = span(V.ku(2, i, j), V.mkk(i, j), i, j);
+        g = g + ((tv3 + V.sbp(i, j + 1) - tv4 - V.sbp(i, j)) * V.rh(2, i, j) -
+                 (tv1 + V.sbp(ip1, j + 1) - tv2 - V.sbp(ip1, j)) * V.rh(2, ip1, j)) *
+                    rdphi * V.jt(JT_RDSV, j);
+        tv1 = span(V.ku(1, i, j + 1), V.mkk(ip1, j + 1), ip1, j + 1);
+        tv2 = span(V.ku(1, i, j), V.mkk(ip1, j), ip1, j);
+        tv3 = span(V.ku(1, i, j + 1), V.mkk(i, j + 1), i, j + 1);
+        tv4 = span(V.ku(1, i, j), V.mkk(i, j), i, j);
+        g = g + ((tv1 + V.sbp(ip1, j + 1) - tv3 - V.sbp(i, j + 1)) * V.rh(1, i, j + 1) -
+                 (tv2 + V.sbp(ip1, j) - tv4 - V.sbp(i, j)) * V.rh(1, i, j)) *
+                    rdphi * V.jt(JT_RDSV, j);
+    }
+    V.W[(dense ? V.ML.gst : V.ML.psi) + l - 1] = g;
+}
+
 // ------------------------------------------------------------ the band solve
 // ubarsolv's substitutions (goldstein.f90:3508-3522) on the psi forcing g in
 // LDS (row i at g[i-1]), which ends as the solution.  Called by the whole
@@ -203,30 +245,55 @@ __global__ __launch_bounds__(MOM_NT) void k_mom_cols_a(const MemberDev* __restri
 // one chunk ahead, and the block synchronises once per chunk.
 //
 // Forward: elimination step i subtracts ratm(i+q, q) x_i from rows i+1..i+n+1.
-// Lane (j-1) mod 64 keeps row j in a register from the step it first changes
-// until it becomes the pivot (a row is live for at most n+2 < 64 steps, so
-// the 64 lanes hold every live row); step i reads the pivot from its lane and
-// every lane holding a row in the band updates it.  Ring row r of a chunk
-// holds the multipliers of one step.
+// Row j sits in lane (j-1) mod 64: the current 64 rows in one register, the
+// next 64 in another (a step reaches at most n+1 < 64 rows on), so a step is
+// one product and a masked difference on each, without a branch, and the rows
+// are written back 64 at a time.  The chain per step is the pivot's readlane,
+// the product, the difference and its select.
 //
 // Back substitution: row i subtracts gap(i, n+2+k) x_{i+k} for k = 1, 2, ..
 // in that order, then divides by the diagonal.  A term with a zero
-// coefficient subtracts a signed zero and leaves the value as it is, so only
-// the others are taken (bit k-1 of the row's mask): the k = 1 term from the
-// row just solved, and the products for k >= 2, which need only rows solved
-// earlier, formed one row ahead by the lanes and packed in order into a
-// zero-padded LDS buffer that the chain reads.  Dividing by a diagonal of
-// exactly 1 (land points) is the identity and is skipped.  Ring row r of a
-// chunk holds a row of the eliminated band (n+2 values) and its mask.
+// coefficient subtracts a signed zero and leaves the value as it is, so the
+// set-up packs each row's others (mom_back_rows).  The k = 1 and 2 terms use
+// the last two rows' values in registers; the products for k >= 3 need only
+// rows done a whole row earlier: while row i is summed, the lanes form row
+// i-1's products, one each, and hand them back through LDS as registers that
+// hold the same values in every lane, zero-padded to whole groups of eight.
+// A row's scalars sit in one lane each for a chunk of rows and are read with
+// readlane.  The chain was behind LDS round trips for those, and behind taken
+// branches, some 45 cycles each: ~1,200 cycles per row, half of them in rows
+// that have nothing to subtract.
+// The chain per row is its subtractions and the division, taken by the host's
+// reciprocal of the diagonal: with y = RN(1/d) and q1 within an ulp of t/d,
+// q1 + (t - d q1) y rounds to RN(t/d) (Markstein 1990); q1 itself comes from
+// one such step, far inside the range where nothing over- or underflows
+// (others divide).  36 x 36 worbe2, one member, the whole solve: 911 -> 516 us with the
+// forcing (11 us) launched apart.
+constexpr int MOM_CHB = 24;    // back-substitution rows per chunk of the ring
+
+// f(q) for every group of eight that holds some of cnt terms; nested, so that
+// the groups left out cost one taken branch together (each costs a refill of
+// the instruction buffer, as long as two or three terms)
+template <int NG, int Q = 0, typename F>
+__device__ __forceinline__ void groups(int cnt, F&& f) {
+    if constexpr (Q < NG) {
+        if (cnt > 8 * Q) {
+            f(Q);
+            groups<NG, Q + 1>(cnt, f);
+        }
+    }
+}
+
+template <int NG>  // groups of eight packed terms: n - 1 <= 8 NG
 __device__ __forceinline__ void band_solve(double* g, double* pbuf, double* ring, const MomGridDev& G, int tid) {
-    const int n = uni(G.n), N = uni(G.N), W1 = n + 1, W2 = n + 2, RS = n + 3;
+    const int n = uni(G.n), N = uni(G.N), W1 = n + 1, RS = n + 3, RB = mom_back_stride(n);
     const int lane = tid & 63;
     const double* __restrict__ fwd = G.fwd;
-    const double* __restrict__ bwd = G.bwd;
-    const uint64_t* __restrict__ bmask = G.bmask;
+    const double* __restrict__ brec = G.brec;
+    const int NA = N - 1;  // rows of the back substitution
     constexpr int PT = 12;  // ring values a producer thread moves per chunk (>= 32 x 64 / 192)
     auto slot = [&](int c) { return ring + (size_t)(c % MOM_RING) * MOM_CH * RS; };
-    // producers: the multipliers of steps [c CH + 1, c CH + CH]
+    // producers: the multipliers of steps [c CH + 1, c CH + CH], zero past the last step
     auto produce_f = [&](int c) {
         double* dst = slot(c);
         const int r0 = c * MOM_CH, nr = min(MOM_CH, N - 1 - r0), tot = nr * W1;
@@ -239,31 +306,23 @@ __device__ __forceinline__ void band_solve(double* g, double* pbuf, double* ring
 #pragma unroll
         for (int e = 0; e < PT; e++) {
             const int x = (tid - 64) + e * (MOM_NT - 64);
-            if (x < tot) dst[(x / W1) * RS + x % W1] = t[e];
+            if (x < MOM_CH * W1) dst[(x / W1) * RS + x % W1] = t[e];
         }
     };
-    // producers: rows i = N-1 - c CH - t of the eliminated band and their masks
+    // producers: the packed rows [c CHB, c CHB + CHB) of the back substitution
     auto produce_b = [&](int c) {
         double* dst = slot(c);
-        const int ihi = N - 1 - c * MOM_CH, nr = min(MOM_CH, ihi), tot = nr * (W2 + 1);
-        double t[PT + 1];
+        const int r0 = c * MOM_CHB, tot = min(MOM_CHB, NA - r0) * RB;
+        double t[PT];
 #pragma unroll
-        for (int e = 0; e < PT + 1; e++) {
+        for (int e = 0; e < PT; e++) {
             const int x = (tid - 64) + e * (MOM_NT - 64);
-            const int r = x / (W2 + 1), k = x % (W2 + 1), i = ihi - r;
-            double val = 0.0;
-            if (x < tot) {
-                if (k < W2)
-                    val = bwd[(size_t)(i - 1) * W2 + k];
-                else
-                    val = __longlong_as_double((long long)bmask[i - 1]);
-            }
-            t[e] = val;
+            t[e] = x < tot ? brec[(size_t)r0 * RB + x] : 0.0;
         }
 #pragma unroll
-        for (int e = 0; e < PT + 1; e++) {
+        for (int e = 0; e < PT; e++) {
             const int x = (tid - 64) + e * (MOM_NT - 64);
-            if (x < tot) dst[(x / (W2 + 1)) * RS + x % (W2 + 1)] = t[e];
+            if (x < tot) dst[x] = t[e];
         }
     };
 
@@ -273,8 +332,8 @@ __device__ __forceinline__ void band_solve(double* g, double* pbuf, double* ring
         produce_f(0);
         if (nchf > 1) produce_f(1);
     }
-    double v = 0.0, vn = 0.0;
-    if (tid < 64) v = lane < N ? g[lane] : 0.0;
+    double va = 0.0, vb = 0.0;
+    if (tid < 64) vb = lane < N ? g[lane] : 0.0;
     __syncthreads();
     for (int c = 0; c < nchf; c++) {
         c = uni(c);
@@ -282,30 +341,31 @@ __device__ __forceinline__ void band_solve(double* g, double* pbuf, double* ring
             const double* rr = slot(c);
             const int sb = (c & ~1) * MOM_CH;             // the 64-step block's first step, minus one
             const int pb = (c & 1) * MOM_CH;              // the pivot lane of the chunk's first step
-            if ((c & 1) == 0) vn = g[min(sb + lane + 64, N - 1)];   // row sb+L+65's forcing, untouched so far
+            if (pb == 0) {
+                va = vb;
+                vb = sb + 64 + lane < N ? g[sb + 64 + lane] : 0.0;
+            }
+            // pivot lane p = pb + d: the row e + 1 past it is lane's, and its
+            // multiplier (n the most, read where the lane has none)
+            const int L1 = lane - pb - 1;
+            auto past = [&](int d) { return (unsigned)((L1 - d) & 63); };
+            auto mult = [&](int d) { return rr[d * RS + (int)min(past(d), (unsigned)n)]; };
             double r[MOM_PRE];
 #pragma unroll
-            for (int d = 0; d < MOM_PRE; d++) {
-                const int q = (lane - (pb + d)) & 63;
-                r[d] = rr[d * RS + (q >= 1 && q <= n + 1 ? q - 1 : 0)];
-            }
+            for (int d = 0; d < MOM_PRE; d++) r[d] = mult(d);
 #pragma unroll
             for (int d = 0; d < MOM_CH; d++) {
-                const int p = pb + d, s = c * MOM_CH + d + 1;
-                const double rd = r[d % MOM_PRE];
-                if (d + MOM_PRE < MOM_CH) {
-                    const int q2 = (lane - (p + MOM_PRE)) & 63;
-                    r[d % MOM_PRE] = rr[(d + MOM_PRE) * RS + (q2 >= 1 && q2 <= n + 1 ? q2 - 1 : 0)];
-                }
-                if (s <= N - 1) {
-                    const double x = readlane_d(v, p);
-                    const int q = (lane - p) & 63;
-                    const bool act = q >= 1 && q <= n + 1 && s + q <= N;
-                    const double upd = v - rd * x;
-                    v = act ? upd : v;
-                    if (lane == 0) g[s - 1] = x;
-                    if (lane == p) v = sb + lane + 65 <= N ? vn : 0.0;
-                }
+                const double x = readlane_d(va, pb + d);
+                const double pr = r[d % MOM_PRE] * x;
+                if (d + MOM_PRE < MOM_CH) r[d % MOM_PRE] = mult(d + MOM_PRE);
+                const bool in = past(d) <= (unsigned)n;
+                const double ua = va - pr, ub = vb - pr;
+                va = in && L1 >= d ? ua : va;   // rows of this block
+                vb = in && L1 < d ? ub : vb;    // and of the next
+            }
+            if (pb != 0 || c == nchf - 1) {
+                if (sb + lane < N) g[sb + lane] = va;
+                if (c == nchf - 1 && sb + 64 + lane < N) g[sb + 64 + lane] = vb;  // row N, where it starts a block
             }
         } else if (c + 2 < nchf) {
             produce_f(c + 2);
@@ -313,101 +373,84 @@ __device__ __forceinline__ void band_solve(double* g, double* pbuf, double* ring
         __syncthreads();
     }
     // ---- back substitution
-    const int nchb = uni((N - 1 + MOM_CH - 1) / MOM_CH);   // rows N-1 .. 1
+    const int nchb = uni((NA + MOM_CHB - 1) / MOM_CHB);
     if (tid >= 64) {
         produce_b(0);
         if (nchb > 1) produce_b(1);
     }
-    double xp = 0.0;
+    double x1 = 0.0, x2 = 0.0;  // the values of the last row taken and of the one before it
     if (tid < 64) {
-        // row N is final after the last step: it sits in lane (N-1) mod 64
-        xp = readlane_d(v, uni((N - 1) & 63));
-        const double dN = bwd[(size_t)(N - 1) * W2];
-        if (dN != 1.0) xp = xp / dN;
-        if (lane == 0) g[N - 1] = xp;
-        pbuf[lane] = 0.0;
-        pbuf[64 + lane] = 0.0;
+        x1 = g[N - 1];
+        if (G.dN != 1.0) x1 = x1 / G.dN;
+        if (lane == 0) g[N - 1] = x1;
     }
     __syncthreads();
-    const int ql = min(lane + 1, n + 1);
-    // ring row of band row i
-    auto brow = [&](int i) { return slot((N - 1 - i) / MOM_CH) + (size_t)((N - 1 - i) % MOM_CH) * RS; };
-    auto maskof = [&](const double* r) { return (uint64_t)__double_as_longlong(r[W2]); };
-    // carried from one row to the next: row i's mask, k = 1 coefficient,
-    // diagonal and forward value; row i-1's mask and this lane's coefficient
-    uint64_t m_i = 0, m_p = 0;
-    double a1_i = 0.0, d_i = 1.0, g_i = 0.0, c_p = 0.0;
-    if (tid < 64) {
-        const double* r0 = brow(N - 1);
-        m_i = maskof(r0);
-        a1_i = r0[1];
-        d_i = r0[0];
-        g_i = g[N - 2];
-        if (N - 2 >= 1) {
-            const double* r1 = brow(N - 2);
-            m_p = maskof(r1);
-            c_p = r1[ql];
-        }
-    }
+    // this lane's packed term (coefficient, k) of row t of chunk c, t < 2 CHB
+    const int le = min(lane, n - 2);
+    auto term = [&](int c, int t, double& cf, int& k) {
+        const double* r = t < MOM_CHB ? slot(c) + t * RB : slot(c + 1) + (t - MOM_CHB) * RB;
+        cf = r[5 + le];
+        k = reinterpret_cast<const uint8_t*>(r + 5 + (n - 1))[le];
+    };
+    double P0[8 * NG], P1[8 * NG];
+    double cf = 0.0;           // the next row's term
+    int kf = 0;
+#pragma unroll
+    for (int e = 0; e < 8 * NG; e++) P0[e] = P1[e] = 0.0;
+    if (tid < 64) term(0, 1, cf, kf);  // the first row has no packed terms
     for (int c = 0; c < nchb; c++) {
         c = uni(c);
         if (tid < 64) {
-            const int ihi = N - 1 - c * MOM_CH, ilo = max(1, ihi - MOM_CH + 1);
-            for (int i = ihi; i >= ilo; i--) {
-                i = uni(i);
-                const double* pc = pbuf + (i & 1) * 64;
-                const int pad = uni((__popcll(m_i & ~(uint64_t)1) + 7) & ~7);
-                double pa[8], pn[8];
+            // lane t holds the scalars of the chunk's row t
+            const int nr = min(MOM_CHB, NA - c * MOM_CHB);
+            const double* rec = slot(c) + min(lane, nr - 1) * RB;
+            const double sd = rec[0], sr = rec[1], sa1 = rec[2], sa2 = rec[3];
+            const int sha = reinterpret_cast<const int*>(rec + 4)[0], shb = reinterpret_cast<const int*>(rec + 4)[1];
+            const double sg = g[(shb & 0xffff) - 1];
+            // row t from its products P; the next row's products into Pn
+            auto row = [&](int t, const double* P, double* Pn) {
+                const int ha = __builtin_amdgcn_readlane(sha, t), hb = __builtin_amdgcn_readlane(shb, t);
+                const int cnt = (ha >> 8) & 255, cntn = (ha >> 16) & 255;
+                double cf2;
+                int kf2;
+                term(c, t + 2, cf2, kf2);
+                const double xk = g[min(max((hb >> 16) + kf - 1, 0), N - 1)];
+                double v = readlane_d(sg, t);
+                if (!(ha & 16)) {
+                    if (ha & 1) v = v - readlane_d(sa1, t) * x1;
+                    if (ha & 2) v = v - readlane_d(sa2, t) * x2;
+                    groups<NG>(cnt, [&](int q) {
 #pragma unroll
-                for (int e = 0; e < 8; e++) pa[e] = pc[e];
-                // the next rows' data, read now and used in the next iteration
-                uint64_t m_n = 0, m_pn = 0;
-                double a1_n = 0.0, d_n = 1.0, g_n = 0.0, c_pn = 0.0;
-                if (i >= 2) {
-                    const double* rn = brow(i - 1);
-                    m_n = maskof(rn);
-                    a1_n = rn[1];
-                    d_n = rn[0];
-                    g_n = g[i - 2];
+                        for (int e = 0; e < 8; e++) v = v - P[8 * q + e];
+                    });
                 }
-                if (i >= 3) {
-                    const double* rnn = brow(i - 2);
-                    m_pn = maskof(rnn);
-                    c_pn = rnn[ql];
-                }
-                const double xk = g[min(i + lane - 1, N - 1)];   // x_{i-1+q}, q = lane + 1 (rows i+1.. for q >= 2)
-                // the chain of row i
-                double t = g_i;
-                if (m_i & 1) t = t - a1_i * xp;
-                for (int q = 0; q < pad; q += 8) {
-                    if (q + 8 < pad) {
+                if (cntn > 0) {
+                    double* pb = pbuf + (t & 1) * 64;
+                    pb[lane] = lane < cntn ? cf * xk : 0.0;
+                    groups<NG>(cntn, [&](int q) {
 #pragma unroll
-                        for (int e = 0; e < 8; e++) pn[e] = pc[q + 8 + e];
+                        for (int e = 0; e < 8; e++) Pn[8 * q + e] = pb[8 * q + e];
+                    });
+                }
+                if (!(ha & 4)) {
+                    const double d = readlane_d(sd, t), rd = readlane_d(sr, t), av = fabs(v);
+                    if (uni(!(ha & 8) && av >= 0x1p-600 && av <= 0x1p600)) {
+                        const double q0 = v * rd;
+                        const double q1 = __builtin_fma(__builtin_fma(-d, q0, v), rd, q0);
+                        v = __builtin_fma(__builtin_fma(-d, q1, v), rd, q1);
+                    } else {
+                        v = v / d;
                     }
-#pragma unroll
-                    for (int e = 0; e < 8; e++) t = t - pa[e];
-#pragma unroll
-                    for (int e = 0; e < 8; e++) pa[e] = pn[e];
                 }
-                if (d_i != 1.0) t = t / d_i;
-                if (lane == 0) g[i - 1] = t;
-                xp = t;
-                // products of row i-1 for k >= 2 into its buffer
-                if (i >= 2) {
-                    const uint64_t m = m_p & ~(uint64_t)1;
-                    const bool set = (m >> lane) & 1;
-                    const int rank = __popcll(m & (((uint64_t)1 << lane) - 1));
-                    const int cnt = __popcll(m), ppad = (cnt + 7) & ~7;
-                    double* pb = pbuf + ((i - 1) & 1) * 64;
-                    if (lane >= cnt && lane < ppad) pb[lane] = 0.0;   // the padding (rank < cnt: no overlap)
-                    if (set) pb[rank] = c_p * xk;
-                }
-                m_i = m_n;
-                a1_i = a1_n;
-                d_i = d_n;
-                g_i = g_n;
-                m_p = m_pn;
-                c_p = c_pn;
+                if (lane == 0) g[(hb & 0xffff) - 1] = v;
+                x2 = x1;
+                x1 = v;
+                cf = cf2;
+                kf = kf2;
+            };
+            for (int t = 0; t < nr; t += 2) {
+                row(t, P0, P1);
+                if (t + 1 < nr) row(t + 1, P1, P0);
             }
         } else if (c + 2 < nchb) {
             produce_b(c + 2);
@@ -417,57 +460,26 @@ __device__ __forceinline__ void band_solve(double* g, double* pbuf, double* ring
 }
 
 // ------------------------------------------------------------ one block per member
-// mode 0: the whole solve; the FP32 form's dense solve splits it round
-// k_mom_gemm: mode 1 forms the psi forcing and stages it, mode 2 takes psi
-// from the staging and goes on from there
+// The psi forcing's solution through the band (NG > 0, the groups of its back
+// substitution) or, for the FP32 form's dense solve (NG = 0), from the slice
+// sums of k_mom_gemm; then psi and what follows from it.
+template <int NG>
 __global__ __launch_bounds__(MOM_NT) void k_mom_solve(const MemberDev* __restrict__ mems,
-                                                      const int32_t* __restrict__ list, int mode) {
-    extern __shared__ double lds[];
+                                                      const int32_t* __restrict__ list) {
+    extern __shared__ __align__(16) double lds[];
     const MomView V(mems[list[blockIdx.x]]);
     const MomGridDev& G = V.G;
     const int mi = V.mi, mj = V.mj, n = V.n, N = V.N, isles = G.isles, tid = threadIdx.x;
-    double* gbs = lds;                          // the psi forcing, then psi (N)
-    double* erhs = lds + N;                     // island integrals, then psibc (isles)
-    double* pbuf = erhs + MOM_MAXISL;           // back substitution's staged products (2 x 64)
-    double* ring = pbuf + 128;                  // factor rows (MOM_RING x MOM_CH x (n+3)), then island terms
+    double* pbuf = lds;                         // back substitution's staged products (2 x 64)
+    double* gbs = lds + 128;                    // the psi forcing, then psi (N)
+    double* erhs = gbs + N;                     // island integrals, then psibc (isles)
+    double* ring = erhs + MOM_MAXISL;           // factor rows (MOM_RING x MOM_CH x (n+3)), then island terms
     const double rdphi = G.rdphi, dphi = G.dphi;
 
-    // ---- the psi forcing: the wind part (wind) plus the torque of the bottom
-    // pressure where the four columns round a psi point differ in depth
-    // (jbar 3256-3313)
-    for (int l = tid + 1; l <= N && mode != 2; l += MOM_NT) {
-        const int i = (l - 1) % n + 1, j = (l - 1) / n;
-        double g = V.W[V.ML.gbw + l - 1];
-        if (j >= 1 && j <= mj - 1 && G.getj[V.col(i, j)]) {
-            const int ip1 = i % mi + 1;
-            auto span = [&](int k0, int k1_, int ii, int jj) {
-                double t = 0;
-                for (int k = k0; k <= k1_; k++) t = t + V.bp(ii, jj, k) * G.dz[k];
-                return t;
-            };
-            double tv1 = span(V.ku(2, ip1, j), V.mkk(ip1, j + 1), ip1, j + 1);
-            double tv2 = span(V.ku(2, ip1, j), V.mkk(ip1, j), ip1, j);
-            double tv3 = span(V.ku(2, i, j), V.mkk(i, j + 1), i, j + 1);
-            double tv4 = span(V.ku(2, i, j), V.mkk(i, j), i, j);
-            g = g + ((tv3 + V.sbp(i, j + 1) - tv4 - V.sbp(i, j)) * V.rh(2, i, j) -
-                     (tv1 + V.sbp(ip1, j + 1) - tv2 - V.sbp(ip1, j)) * V.rh(2, ip1, j)) *
-                        rdphi * V.jt(JT_RDSV, j);
-            tv1 = span(V.ku(1, i, j + 1), V.mkk(ip1, j + 1), ip1, j + 1);
-            tv2 = span(V.ku(1, i, j), V.mkk(ip1, j), ip1, j);
-            tv3 = span(V.ku(1, i, j + 1), V.mkk(i, j + 1), i, j + 1);
-            tv4 = span(V.ku(1, i, j), V.mkk(i, j), i, j);
-            g = g + ((tv1 + V.sbp(ip1, j + 1) - tv3 - V.sbp(i, j + 1)) * V.rh(1, i, j + 1) -
-                     (tv2 + V.sbp(ip1, j) - tv4 - V.sbp(i, j)) * V.rh(1, i, j)) *
-                        rdphi * V.jt(JT_RDSV, j);
-        }
-        gbs[l - 1] = g;
-        if (mode == 1) V.W[V.ML.gst + l - 1] = g;
-    }
-    if (mode == 1) return;
-    __syncthreads();
-
-    if (mode == 0) {
-        band_solve(gbs, pbuf, ring, G, tid);
+    if constexpr (NG > 0) {
+        for (int l = tid; l < N; l += MOM_NT) gbs[l] = V.W[V.ML.psi + l];
+        __syncthreads();
+        band_solve<NG>(gbs, pbuf, ring, G, tid);
     } else {
         for (int l = tid; l < N; l += MOM_NT) {
             double p = V.W[V.ML.gst + N + l];
@@ -782,17 +794,24 @@ void launch_mom(const MemberDev* mems, const int32_t* list, int nlist, const int
     const size_t lds = mom_solve_lds(maxN, maxn);
     if (part & 1) hipLaunchKernelGGL(k_mom_cols_a, dim3(cb, nlist), dim3(MOM_NT), 0, s, mems, list);
     if (!(part & 2)) return;
-    if (nband > 0) hipLaunchKernelGGL(k_mom_solve, dim3(nband), dim3(MOM_NT), lds, s, mems, band, 0);
+    const int fb = (maxN + MOM_NT - 1) / MOM_NT;
+    if (nband > 0) {
+        hipLaunchKernelGGL(k_mom_force, dim3(fb, nband), dim3(MOM_NT), 0, s, mems, band, 0);
+        if (maxn <= 41)
+            hipLaunchKernelGGL(k_mom_solve<5>, dim3(nband), dim3(MOM_NT), lds, s, mems, band);
+        else
+            hipLaunchKernelGGL(k_mom_solve<8>, dim3(nband), dim3(MOM_NT), lds, s, mems, band);
+    }
     int ndense = 0;
     for (int q = 0; q < ngroups; q++) ndense += groups[3 * q + 1];
     if (ndense > 0) {
-        hipLaunchKernelGGL(k_mom_solve, dim3(ndense), dim3(MOM_NT), lds, s, mems, dense, 1);
+        hipLaunchKernelGGL(k_mom_force, dim3(fb, ndense), dim3(MOM_NT), 0, s, mems, dense, 1);
         for (int q = 0; q < ngroups; q++) {
             const int off = groups[3 * q], nm = groups[3 * q + 1], N = groups[3 * q + 2];
             hipLaunchKernelGGL(k_mom_gemm, dim3((N + GT - 1) / GT, (nm + GT - 1) / GT, MOM_SPLITK), dim3(256), 0, s,
                                mems, dense + off, nm);
         }
-        hipLaunchKernelGGL(k_mom_solve, dim3(ndense), dim3(MOM_NT), lds, s, mems, dense, 2);
+        hipLaunchKernelGGL(k_mom_solve<0>, dim3(ndense), dim3(MOM_NT), lds, s, mems, dense);
     }
     hipLaunchKernelGGL(k_mom_cols_b, dim3(cb, nlist), dim3(MOM_NT), 0, s, mems, list);
     hipLaunchKernelGGL(k_mom_cols_c, dim3(cb2, nlist), dim3(MOM_NT), 0, s, mems, list);

@@ -12,8 +12,10 @@
 // flat with the layouts listed in MomGridDev (cgocn_dev.h).
 #pragma once
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdlib>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -48,6 +50,44 @@ struct MomSetup {
     static double& UB(double* u, int mi, int l, int i, int j) { return u[(l - 1) + 2 * ((size_t)i + (size_t)(mi + 2) * j)]; }
     static double& PS(double* p, int mi, int i, int j) { return p[(size_t)i + (size_t)(mi + 1) * j]; }
 };
+
+// The eliminated band's rows N-1 down to 1 as the back substitution reads
+// them, `stride` doubles each: the diagonal d = gap(i, n+2), RN(1/d), the
+// k = 1 and k = 2 coefficients, a header (bits 0 and 1: those two are not
+// zero; bit 2: d = 1; bit 3: divide by d, whose exponent or reciprocal leaves
+// too little room; bit 4: no terms; bits 8-15: packed terms, 16-23: the next
+// record's), the row and, in the upper half, the next record's, then the
+// non-zero coefficients for k = 3 .. n+1 in that order and, a byte each, k.
+inline void mom_back_rows(MomSetup& M, int stride, std::vector<double>& rec) {
+    const int n = M.n, N = M.N;
+    rec.assign((size_t)std::max(N - 1, 1) * stride, 0.0);
+    int32_t next[2] = {0, 0};  // header and row of the record after this one
+    for (int i = 1; i <= N - 1; i++) {
+        double* r = &rec[(size_t)(N - 1 - i) * stride];
+        uint8_t* kb = reinterpret_cast<uint8_t*>(r + 5 + (n - 1));
+        const double d = M.GAP(i, n + 2), ad = std::fabs(d);
+        int32_t hdr = 0, cnt = 0;
+        r[0] = d;
+        r[1] = 1.0 / d;
+        if (d == 1.0) hdr |= 4;
+        if (!(ad >= 0x1p-300 && ad <= 0x1p300)) hdr |= 8;
+        for (int k = 1; k <= n + 1 && i + k <= N; k++) {
+            const double c = M.GAP(i, n + 2 + k);
+            if (k <= 2) {
+                r[1 + k] = c;
+                if (c != 0.0) hdr |= k;
+            } else if (c != 0.0) {
+                r[5 + cnt] = c;
+                kb[cnt++] = (uint8_t)k;
+            }
+        }
+        if (cnt == 0 && !(hdr & 3)) hdr |= 16;
+        const int32_t w[2] = {hdr | cnt << 8 | (next[0] & 0xff00) << 8, i | next[1] << 16};
+        std::memcpy(r + 4, w, sizeof w);
+        next[0] = w[0];
+        next[1] = i;
+    }
+}
 
 inline int isign1(int x) { return x >= 0 ? 1 : -1; }
 

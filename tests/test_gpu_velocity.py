@@ -259,3 +259,54 @@ def test_set_velocity_switches_the_solve_off(eng, world):
     with pytest.raises(E.CgoError):
         eng.psi(m, g)
     assert np.abs(eng.velocity(m, g)).max() == 0.0
+
+
+@pytest.mark.parametrize("mi,mj,mk", [(3, 5, 2), (9, 13, 4), (41, 10, 3), (42, 7, 3), (50, 12, 5)])
+def test_band_solve_of_other_bands(eng, mi, mj, mk):
+    """Channels of other widths, walls north and south and a ridge of land
+    across part of each: the narrowest band, row counts that leave part of a
+    chunk, and the widest band of the smaller and the narrowest of the larger
+    set of packed terms.  Velocities and psi after three steps against the
+    oracle's from the same densities."""
+    rng = np.random.default_rng(mi)
+    k1 = np.ones((mj + 2, mi + 2), dtype=np.int32)
+    k1[1:-1, 1:-1] = rng.integers(1, mk, (mj, mi)) if mk > 2 else 1
+    k1[0, :] = k1[mj + 1, :] = 94
+    k1[mj - 1:mj + 1, 1:2 + mi // 4] = 94          # land, part of the northern wall
+    k1[:, 0], k1[:, mi + 1] = k1[:, mi], k1[:, 1]
+    labels = np.zeros((mj + 1, mi), dtype=np.int32)
+    labels[0, :] = 2
+    labels[mj, :] = 1
+    wet = k1 <= mk
+    for j in range(1, mj):                          # psi points with no wet corner belong to the northern landmass
+        for i in range(1, mi + 1):
+            if not (wet[j, i] or wet[j, i + 1] or wet[j + 1, i] or wet[j + 1, i + 1]):
+                labels[j, i - 1] = 1
+    npi = np.array([mi], dtype=np.int32)
+    paths = np.array([[1, i, 2] for i in range(1, mi + 1)], dtype=np.int32).ravel()
+    g, og = G.make_grid(mi, mj, mk), O.grid(mi, mj, mk)
+    st = rng.normal(0.0, 0.05, (mj, mi, 4))
+    ts = np.zeros((mk, mj, mi, 2))
+    ts[..., 0] = 2 + 3 * np.arange(mk)[:, None, None] + rng.normal(0.0, 0.3, (mk, mj, mi))
+    ts[..., 1] = rng.normal(0.0, 0.1, (mk, mj, mi))
+    w = np.arange(1, mk + 1)[:, None, None] >= k1[None, 1:-1, 1:-1]
+    ts[~w] = 0.0
+    mo = O.MomOracle(og, k1, labels, 1, npi, paths)
+    mo.set_wind(st)
+    u = np.zeros((mk, mj + 1, mi + 1, 3))
+    gold = O.GoldsteinOracle(og, k1, ts, u, diso=True)
+    gold.rho[...] = O.rho_from_ts(og, k1, ts)
+    for _ in range(3):
+        mo.step(gold.rho, u)
+        gold.step(1)
+    gid = eng.add_grid(g, k1)
+    eng.set_momentum(gid, g, G.World(k1, labels, 1, npi, paths))
+    m = eng.add_member(gid, 2, E.FP64, DIFF, diso=True)
+    eng.upload(m, ts)
+    eng.set_wind(m, st)
+    eng.step([m], 3)
+    eu, ep = rel(eng.velocity(m, g), u[:, 1:, 1:, :]), rel(eng.psi(m, g), mo.psi())
+    es = rel(eng.download(m, ts.shape), gold.ts, w)
+    say((mi, mj, mk), "velocity, psi, state rel err", eu, ep, es)
+    assert np.abs(u).max() > 0 and np.isfinite(u).all()
+    assert eu <= 1e-12 and ep <= 1e-12 and es <= 1e-12
