@@ -15,6 +15,8 @@
 #pragma once
 #include "cgocn_dev.h"
 
+#include <type_traits>
+
 namespace cgo {
 
 
@@ -28,8 +30,22 @@ template <> struct Met<float> {
     static __device__ __forceinline__ const float* k(const GridDev& g) { return g.mkf; }
 };
 
+// 2^e for e within a double's normal exponents
+__device__ __forceinline__ double pow2(int e) { return __hiloint2double((1023 + e) << 20, 0); }
+
 // weight of one unit of the int16 carry of a float value x: 2^-16 ulp(x)
-__device__ __forceinline__ double carry_unit(float x) { return ldexp(1.0, carry_exp(x) - 23 - 16); }
+__device__ __forceinline__ double carry_unit(float x) { return pow2(carry_exp(x) - 23 - 16); }
+
+// the carry of a value x stored as the float h: x - h in those units, rounded
+// to nearest (x - h is exact, scaling it by a power of two too, and adding
+// 1.5 2^52 leaves the rounded integer in the low word: one instruction in
+// place of ldexp, rint and a conversion, each of a quarter of the rate).  It
+// lies within +-2^15; the clamp is taken on the integer.
+__device__ __forceinline__ int carry_of(double x, float h) {
+    const double r = __builtin_fma(x - (double)h, pow2(23 + 16 - carry_exp(h)), 0x1.8p52);
+    const int ri = __double2loint(r);
+    return ri < -32767 ? -32767 : (ri > 32767 ? 32767 : ri);
+}
 
 // state access as double (FP32 form: hi + carry)
 // a / b: the IEEE quotient in FP64; in the FP32 form the hardware reciprocal
@@ -84,27 +100,14 @@ template <> struct StateIO<float> {
     static __device__ __forceinline__ void st(void* s, int16_t* lo, uint32_t i, double x) {
         float h = (float)x;
         at((AS_GLOBAL float*)s, i) = h;
-        if (lo) {
-            // x - h in units of carry_unit(h): scaling by the exact power of two
-            // 2^(39 - e) rounds exactly as dividing by 2^(e - 39) would; the
-            // rounded value is within +-2^15, so the clamp is taken on the integer
-            const double r = rint(ldexp(x - (double)h, 23 + 16 - carry_exp(h)));
-            int ri = (int)r;
-            ri = ri < -32767 ? -32767 : (ri > 32767 ? 32767 : ri);
-            at((AS_GLOBAL int16_t*)lo, i) = (int16_t)ri;
-        }
+        if (lo) at((AS_GLOBAL int16_t*)lo, i) = (int16_t)carry_of(x, h);
     }
     // the value a later ld returns after st(x): the float, plus the carry
     // split and clamped as st stores it
     static __device__ __forceinline__ double rt(double x, bool carry) {
         const float h = (float)x;
         double v = (double)h;
-        if (carry) {
-            const double r = rint(ldexp(x - (double)h, 23 + 16 - carry_exp(h)));
-            int ri = (int)r;
-            ri = ri < -32767 ? -32767 : (ri > 32767 ? 32767 : ri);
-            v += (double)(int16_t)ri * carry_unit(h);
-        }
+        if (carry) v += (double)carry_of(x, h) * carry_unit(h);
         return v;
     }
 };
@@ -155,7 +158,7 @@ __device__ __forceinline__ float carry_residual(float h, int16_t c) {
 // to co, which then takes every column (FP32 members hand it their new values
 // unrounded, as the march sums them).
 template <typename R, int LB, int FLUX_THREADS, int FLUX_NBUF, int MODE>
-__global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restrict__ mems,
+__global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __restrict__ mems,
                                                        const int32_t* __restrict__ list, FluxSplit sp_) {
     constexpr bool SPLIT = MODE == 3;
     constexpr int IM = SPLIT ? 0 : MODE;
@@ -226,11 +229,14 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
     const AS_GLOBAL R* mk = gp(Met<R>::k(g));
     const int JS = maxj + 2, KS = maxk + 2;
     const R rc = mj[MJ_RC * JS + J], rc2 = mj[MJ_RC2 * JS + J];
-    const R cvn = mj[MJ_CV * JS + J], cv2n = mj[MJ_CV2 * JS + J];
-    const R cvs = mj[MJ_CV * JS + J - 1], cv2s = mj[MJ_CV2 * JS + J - 1];
-    const R dsvn = mj[MJ_DSVM * JS + J], dsvs = mj[MJ_DSVM * JS + J - 1];
+    // (the walls' northward metrics are the caller's to leave undefined; their
+    // faces are closed, and zero keeps a product with a closed face's zero)
+    const bool wallN = J == maxj, wallS = J == 1;
+    const R cvn = mj[MJ_CV * JS + J], cv2n = wallN ? (R)0 : mj[MJ_CV2 * JS + J];
+    const R cvs = mj[MJ_CV * JS + J - 1], cv2s = wallS ? (R)0 : mj[MJ_CV2 * JS + J - 1];
+    const R dsvn = mj[MJ_DSVM * JS + J], dsvs = wallS ? (R)0 : mj[MJ_DSVM * JS + J - 1];
     const R rds = mj[MJ_RDS * JS + J];
-    const R rdsvn = mj[MJ_RDSV * JS + J], rdsvs = mj[MJ_RDSV * JS + J - 1];
+    const R rdsvn = wallN ? (R)0 : mj[MJ_RDSV * JS + J], rdsvs = wallS ? (R)0 : mj[MJ_RDSV * JS + J - 1];
     const R dphi = (R)g.dphi, rdphi = (R)g.rdphi;
     const R diff1 = sizeof(R) == 8 ? (R)M.diff1 : (R)M.diff1f;
     const R diffv = sizeof(R) == 8 ? (R)M.diff2 : (R)M.diff2f;
@@ -300,7 +306,7 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
     // expressions on the same values, bit for bit.
     const double rcD = gp(g.mj)[MJ_RC * JS + J], cvnD = gp(g.mj)[MJ_CV * JS + J];
     const double cvsD = gp(g.mj)[MJ_CV * JS + J - 1];
-    const double rdsvnD = gp(g.mj)[MJ_RDSV * JS + J], rdsvsD = gp(g.mj)[MJ_RDSV * JS + J - 1];
+    const double rdsvnD = wallN ? 0.0 : gp(g.mj)[MJ_RDSV * JS + J], rdsvsD = wallS ? 0.0 : gp(g.mj)[MJ_RDSV * JS + J - 1];
     const double rdphiD = g.rdphi, diff1D = M.diff1;
     const double e0D = g.ec[0], e1D = g.ec[1], e2D = g.ec[2], e3D = g.ec[3];
     const double sccD = M.diso ? e1D : 0.0;
@@ -318,6 +324,21 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
             return ((double)SP(bu, q, pp) - (double)SP(bc, q, pp)) + ((double)SR(bu, q, pp) - (double)SR(bc, q, pp));
         return (double)(SP(bu, q, pp) - SP(bc, q, pp));
     };
+    // The tile positions of a cell's neighbours at a level: its own where the
+    // face between them is closed, so that every difference across a closed
+    // face is zero without a test.  A test per face and tracer was a branch
+    // each, with an LDS read waited for behind it: twenty a tracer, the largest
+    // part of the 20,000 cycles a level of eight FP64 tracers took.  Without
+    // them the flux alone takes, 64 FP64 members of 36x36x16x24, 250 -> 201 us
+    // a launch, 256 FP32C members 512 -> 461 us, six of 72x72x32x40 209 -> 154.
+    // (Loading a level's coefficients while the one below it is formed hid no
+    // more and cost a wave per SIMD: 483 us for the 256.)
+    struct Nbr {
+        int e, w, n, s;
+    };
+    auto nbrs = [&](int k) {
+        return Nbr{k >= k1e ? pe : p, k >= k1w ? pw : p, k >= k1n ? pn : p, k >= k1s ? ps : p};
+    };
     // the isoneutral slope terms of a cell at level k < maxk from the staged
     // T and S (2489-2501, 2561-2605): dzrho, the four corner gradients, the
     // slope limiter; counts limps and the diffusive stability number
@@ -330,6 +351,7 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
         const double tec = -e0D - e2D * tatw * 2 - e3D * tatw * tatw * 3;
         dzrho = (e1D * DKD(ub, cb, qS, p) - tec * DKD(ub, cb, qT, p)) * rdza;
         if (M.diso && dzrho < -1.0E-12) {
+            const Nbr nc = nbrs(k), nu = nbrs(k + 1);
             iso = true;
             rdzrho = fdiv(1.0, dzrho);
             double tv1 = 0;
@@ -337,13 +359,12 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
 #pragma unroll
             for (int n = 0; n < 4; n++) {
                 const int b = n < 2 ? cb : ub;
-                const int kn = n < 2 ? k : k + 1;
                 const bool east = n & 1;
-                const bool mx = kn >= (east ? k1e : k1w), my = kn >= (east ? k1n : k1s);
-                const double dxT = mx ? (east ? DD(b, qT, pe, p) : DD(b, qT, p, pw)) * rcD * rdphiD : 0.0;
-                const double dxS = mx ? (east ? DD(b, qS, pe, p) : DD(b, qS, p, pw)) * rcD * rdphiD : 0.0;
-                const double dyT = my ? (east ? DD(b, qT, pn, p) * cvnD * rdsvnD : DD(b, qT, p, ps) * cvsD * rdsvsD) : 0.0;
-                const double dyS = my ? (east ? DD(b, qS, pn, p) * cvnD * rdsvnD : DD(b, qS, p, ps) * cvsD * rdsvsD) : 0.0;
+                const Nbr& m = n < 2 ? nc : nu;
+                const double dxT = (east ? DD(b, qT, m.e, p) : DD(b, qT, p, m.w)) * rcD * rdphiD;
+                const double dxS = (east ? DD(b, qS, m.e, p) : DD(b, qS, p, m.w)) * rcD * rdphiD;
+                const double dyT = east ? DD(b, qT, m.n, p) * cvnD * rdsvnD : DD(b, qT, p, m.s) * cvsD * rdsvsD;
+                const double dyS = east ? DD(b, qS, m.n, p) * cvnD * rdsvnD : DD(b, qS, p, m.s) * cvsD * rdsvsD;
                 dxr[n] = sccD * dxS - tec * dxT;
                 dyr[n] = sccD * dyS - tec * dyT;
                 tv1 = tv1 + dxr[n] * dxr[n] + dyr[n] * dyr[n];
@@ -394,15 +415,6 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
     double accs[LB], accS = 0.0;
 #pragma unroll
     for (int q = 0; q < LB; q++) accs[q] = 0.0;
-    auto add_sum = [&](int q, double nv, double os, double mm, double vv) {
-        const int l = l0 + q;
-        if (l == 1) {
-            accS += (nv + SALN0 + 0.0) * vv;
-        } else if (l >= 2) {
-            const double lv = nv * os * rSold;
-            accs[q] += lv * mm;
-        }
-    };
     fetch(kmin - 1);
     commit(kmin % FLUX_NBUF);
     if (kmin < maxk) {
@@ -454,10 +466,11 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
             R ue_ = 0, uw_ = 0, un_ = 0, us_ = 0, ua_ = 0;
             R upe = 0, upw = 0, upn = 0, ups = 0, upa = 0;
             if constexpr (!ANOM) {
-                ue_ = at(u, oc);
-                uw_ = at(u, (uint32_t)(o + cw));
-                un_ = at(u, ncell + oc);
-                us_ = at(u, (uint32_t)(ncell + o + cs));
+                // (closed faces carry nothing)
+                ue_ = k >= k1e ? at(u, oc) : (R)0;
+                uw_ = k >= k1w ? at(u, (uint32_t)(o + cw)) : (R)0;
+                un_ = k >= k1n ? at(u, ncell + oc) : (R)0;
+                us_ = k >= k1s ? at(u, (uint32_t)(ncell + o + cs)) : (R)0;
                 ua_ = at(u, 2 * ncell + oc);
                 R pec;
                 pec = ue_ * dphi / diff1; upe = pec / ((R)2.0 + fabs(pec));
@@ -466,8 +479,7 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
                 pec = us_ * dsvs / diff1; ups = pec / ((R)2.0 + fabs(pec));
                 pec = ua_ * dza / diffv; upa = pec / ((R)2.0 + fabs(pec));
             }
-            const bool oe = k >= max(k1c, k1e), ow = k >= max(k1w, k1c);
-            const bool on = k >= max(k1c, k1n), os = k >= max(k1s, k1c);
+            const Nbr nc = nbrs(k), nu = nbrs(k + 1);
             // isoneutral coefficients from T and S (2489-2501, 2561-2605)
             bool iso = false;
             double dzrho = 0, rdzrho = 0, slim = 1, dxr[4] = {0, 0, 0, 0}, dyr[4] = {0, 0, 0, 0};
@@ -484,7 +496,6 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
                                 ay[n] = at(ic, (uint32_t)((4 + n) * ncell) + oc);
                             }
                             qq = at(ic, (uint32_t)(8 * ncell) + oc);
-                            iso = true;
                         } else {
                             const AS_GLOBAL double* ic = gp(M.isoc);
                             dzrho = at(ic, oc);
@@ -515,142 +526,133 @@ __global__ __launch_bounds__(FLUX_THREADS) void k_flux(const MemberDev* __restri
                 s_mm = at(gp(M.M), oc);
                 if (l0 == 0) s_vv = at(gp(g.V), oc);
             }
-            if constexpr (ANOM) {
-                // FP32 form in coefficient form: each face flux is the
-                // neighbour difference times a coefficient of the cell, and the
-                // isoneutral flux a sum of corner differences times
-                // coefficients.  The face coefficients depend on the velocity,
-                // the diffusivities and the mask only: cgo_set_velocity forms
-                // them in FP64 and rounds each once (closed faces are zero)
-                const R ce = at(u, oc), cw = at(u, ncell + oc);
-                const R cn = at(u, 2 * ncell + oc), cs = at(u, 3 * ncell + oc);
-                const R ca = at(u, 4 * ncell + oc), cbn = at(u, 5 * ncell + oc);
+            if (!sums || l0 != 0) s_vv = 0.0;
+            // a tracer's new value joins the sums of its column (S in slot 1 of
+            // the first block; without BIOGEM the factors are zero)
+            auto add_sum = [&](int q, double nv) {
+                if (q == 0) newT = nv;
+                if (q == 1) {
+                    newS = nv;
+                    accS = ANOM ? __builtin_fma(nv + SALN0 + 0.0, s_vv, accS) : accS + (nv + SALN0 + 0.0) * s_vv;
+                }
+                const double lv = nv * s_os * rSold;
+                accs[q] = ANOM ? __builtin_fma(lv, s_mm, accs[q]) : accs[q] + lv * s_mm;
+            };
+            // the level's tracers: every value of the cell above is in, so a
+            // tracer is one run of instructions with no test but the store's
+            auto tracers = [&](auto top_) {
+                constexpr bool TOP = decltype(top_)::value;
+                if constexpr (ANOM) {
+#pragma clang fp contract(off)
+                    // (the contractions are written out, so that every tile and
+                    // mode rounds alike whatever else its blocks hold)
+                    // FP32 form in coefficient form: each face flux is the
+                    // neighbour difference times a coefficient of the cell, and the
+                    // isoneutral flux a sum of corner differences times
+                    // coefficients.  The face coefficients depend on the velocity,
+                    // the diffusivities and the mask only: cgo_set_velocity forms
+                    // them in FP64 and rounds each once (closed faces are zero)
+                    auto fma_ = [](R a, R b, R c) -> R { return __builtin_fmaf(a, b, c); };
+                    const R ce = at(u, oc), cw = at(u, ncell + oc);
+                    const R cn = at(u, 2 * ncell + oc), cs = at(u, 3 * ncell + oc);
+                    const R ca = at(u, 4 * ncell + oc), cbn = at(u, 5 * ncell + oc);
 #pragma unroll
-                for (int q = 0; q < LB; q++) {
-                    if (q >= nl) break;
-                    const R Tc = SP(cb, q, p);
-                    const R dE = D(cb, q, pe, p), dW = D(cb, q, pw, p), dN = D(cb, q, pn, p), dS = D(cb, q, ps, p);
-                    R fa, fbn = 0;
-                    // the top cell's surface flux enters in FP64: rounded to
-                    // float it would bias every step's forcing alike
-                    double fsurf = 0.0;
-                    if (top) {
-                        fa = (R)0;
-                        if (M.sflux) fsurf = at(gp(M.sflux), (uint32_t)((l0 + q) * plane + col));
-                    } else {
-                        const R dU = DK(ub, cb, q, p);
-                        R tv = 0;
-                        if (iso) {
+                    for (int q = 0; q < LB; q++) {
+                        const R Tc = SP(cb, q, p);
+                        const R dE = D(cb, q, pe, p), dW = D(cb, q, pw, p), dN = D(cb, q, pn, p), dS = D(cb, q, ps, p);
+                        R fa = 0, fbn = 0;
+                        // the top cell's surface flux enters in FP64: rounded to
+                        // float it would bias every step's forcing alike
+                        double incs = 0.0;
+                        if constexpr (TOP) {
+                            if (M.sflux && q < nl) {
+                                const double fsurf = at(gp(M.sflux), (uint32_t)((l0 + q) * plane + col));
+                                if (fsurf != 0.0) incs = -(gp(g.mk)[MK_DT * KS + k] * (fsurf * gp(g.mk)[MK_RDZ * KS + k]));
+                            }
+                        } else {
+                            const R dU = DK(ub, cb, q, p);
                             // corner differences with the sign of the west/south
                             // corners folded into ax[0], ax[2], ay[0], ay[2]
-                            tv = ax[0] * dW + ax[1] * dE + ay[0] * dS + ay[1] * dN;
-                            tv = tv + ax[2] * D(ub, q, pw, p) + ax[3] * D(ub, q, pe, p) + ay[2] * D(ub, q, ps, p) +
-                                 ay[3] * D(ub, q, pn, p);
-                            tv = tv - qq * dU;
+                            R tv = fma_(ax[1], dE, ax[0] * dW);
+                            tv = fma_(ay[0], dS, tv);
+                            tv = fma_(ay[1], dN, tv);
+                            tv = fma_(ax[2], D(ub, q, pw, p), tv);
+                            tv = fma_(ax[3], D(ub, q, pe, p), tv);
+                            tv = fma_(ay[2], D(ub, q, ps, p), tv);
+                            tv = fma_(ay[3], D(ub, q, pn, p), tv);
+                            tv = fma_(-qq, dU, tv);
+                            fa = fma_(dU, ca, tv);
+                            fbn = fma_(dU, cbn, tv);
                         }
-                        fa = dU * ca + tv;
-                        fbn = dU * cbn + tv;
-                    }
-                    const R div = ((dE * ce - dW * cw) + (dN * cn - dS * cs)) + (fa - FB(q)) * rdz;
-                    const int idx = (l0 + q) * tstride + o + col;
-                    const R inc = -(dt * (div + Tc * divu));
-                    const double incs = fsurf != 0.0 ? -(gp(g.mk)[MK_DT * KS + k] * (fsurf * gp(g.mk)[MK_RDZ * KS + k])) : 0.0;
-                    double nv;
-                    if (lo_src) {
-                        // compensated accumulation: the rounding residual of every
-                        // update is carried to the next step in the int16 plane
-                        nv = ((double)Tc + (double)SR(cb, q, p)) + (double)inc + incs;
-                        if (own) StateIO<R>::st((R*)dst, lo_dst, idx, nv);
-                    } else {
-                        const R v = Tc + (inc + (R)incs);
-                        if (own) at(dst, (uint32_t)idx) = v;
-                        nv = (double)v;
-                    }
-                    if (SPLIT && own && nvs) at(nvs, (uint32_t)idx) = nv;
-                    FB(q) = fbn;
-                    if (l0 + q == 0) newT = nv;
-                    if (l0 + q == 1) newS = nv;
-                    if (sums) add_sum(q, nv, s_os, s_mm, s_vv);
-                }
-            } else
-#pragma unroll
-            for (int q = 0; q < LB; q++) {
-                if (q >= nl) break;
-                const R Tc = SP(cb, q, p), Te = SP(cb, q, pe), Tw = SP(cb, q, pw), Tn = SP(cb, q, pn), Ts = SP(cb, q, ps);
-                R fe, fw, fn, fs, fa, fbn = 0;
-                if (!ANOM) {
-                    fe = oe ? ue_ * rc * (((R)1.0 - upe) * Te + ((R)1.0 + upe) * Tc) * (R)0.5 - (Te - Tc) * rc2 * diff1 : (R)0;
-                    fw = ow ? uw_ * rc * (((R)1.0 - upw) * Tc + ((R)1.0 + upw) * Tw) * (R)0.5 - (Tc - Tw) * rc2 * diff1 : (R)0;
-                    fn = on ? cvn * un_ * (((R)1.0 - upn) * Tn + ((R)1.0 + upn) * Tc) * (R)0.5 - cv2n * (Tn - Tc) * diff1 : (R)0;
-                    fs = os ? cvs * us_ * (((R)1.0 - ups) * Tc + ((R)1.0 + ups) * Ts) * (R)0.5 - cv2s * (Tc - Ts) * diff1 : (R)0;
-                } else {
-                    const R dE = D(cb, q, pe, p), dW = D(cb, q, pw, p), dN = D(cb, q, pn, p), dS = D(cb, q, ps, p);
-                    fe = oe ? ue_ * rc * ((R)1.0 - upe) * dE * (R)0.5 - dE * rc2 * diff1 : (R)0;
-                    fw = ow ? uw_ * rc * ((R)1.0 + upw) * dW * (R)0.5 + dW * rc2 * diff1 : (R)0;
-                    fn = on ? cvn * un_ * ((R)1.0 - upn) * dN * (R)0.5 - cv2n * dN * diff1 : (R)0;
-                    fs = os ? cvs * us_ * ((R)1.0 + ups) * dS * (R)0.5 + cv2s * dS * diff1 : (R)0;
-                }
-                if (top) {
-                    fa = M.sflux ? (R)at(gp(M.sflux), (uint32_t)((l0 + q) * plane + col)) : (R)0;
-                } else {
-                    const R Tu = SP(ub, q, p);
-                    const R dUc = DK(ub, cb, q, p);
-                    R nadv = -dUc * rdza * diffv;
-                    if (!ANOM) {
-                        fa = ua_ * (((R)1.0 - upa) * Tu + ((R)1.0 + upa) * Tc) * (R)0.5;
-                        fa = fa - (Tu - Tc) * rdza * diffv;
-                    }
-                    if (iso) {
-                        const R dzts = dUc * rdza;
-                        R tv = 0;
-#pragma unroll
-                        for (int n = 0; n < 4; n++) {
-                            const int b = n < 2 ? cb : ub;
-                            const bool east = n & 1;
-                            const int kn = n < 2 ? k : k + 1;
-                            const R dx = kn >= (east ? k1e : k1w)
-                                             ? (east ? D(b, q, pe, p) : D(b, q, p, pw)) * rc * rdphi
-                                             : (R)0;
-                            const R dy = kn >= (east ? k1n : k1s)
-                                             ? (east ? D(b, q, pn, p) * cvn * rdsvn : D(b, q, p, ps) * cvs * rdsvs)
-                                             : (R)0;
-                            tv = tv + ((R)2 * dzrho * dx - dxr[n] * dzts) * dxr[n] + ((R)2 * dzrho * dy - dyr[n] * dzts) * dyr[n];
+                        const R lat = fma_(ce, dE, -(cw * dW)) + fma_(cn, dN, -(cs * dS));
+                        const R div = fma_(Tc, divu, fma_(fa - FB(q), rdz, lat));
+                        const int idx = (l0 + q) * tstride + o + col;
+                        const R inc = -(dt * div);
+                        double nv;
+                        if (lo_src) {
+                            // compensated accumulation: the rounding residual of every
+                            // update is carried to the next step in the int16 plane
+                            nv = ((double)Tc + (double)SR(cb, q, p)) + (double)inc + incs;
+                            if (own && q < nl) StateIO<R>::st((R*)dst, lo_dst, idx, nv);
+                        } else {
+                            const R v = Tc + (inc + (R)incs);
+                            if (own && q < nl) at(dst, (uint32_t)idx) = v;
+                            nv = (double)v;
                         }
-                        tv = isoc * tv / (dzrho * dzrho);
-                        if (!ANOM) fa = fa + tv;
-                        nadv = nadv + tv;
+                        if (SPLIT && own && nvs && q < nl) at(nvs, (uint32_t)idx) = nv;
+                        FB(q) = fbn;
+                        add_sum(q, nv);
                     }
-                    if (ANOM) {
-                        fa = ua_ * ((R)1.0 - upa) * dUc * (R)0.5 + nadv;       // relative to this cell
-                        fbn = -(ua_ * ((R)1.0 + upa) * dUc * (R)0.5) + nadv;   // relative to the cell above
-                    }
-                }
-                const R div = ((fe - fw) * rdphi + (fn - fs) * rds) + (fa - FB(q)) * rdz;
-                const int idx = (l0 + q) * tstride + o + col;
-                double nv;
-                if (ANOM) {
-                    const R inc = -(dt * (div + Tc * divu));
-                    if (lo_src) {
-                        // compensated accumulation: the rounding residual of every
-                        // update is carried to the next step in the int16 plane
-                        nv = ((double)Tc + (double)SR(cb, q, p)) + (double)inc;
-                        StateIO<R>::st((R*)dst, lo_dst, idx, nv);
-                    } else {
-                        const R v = Tc + inc;
-                        at(dst, (uint32_t)idx) = v;
-                        nv = (double)v;
-                    }
-                    FB(q) = fbn;
                 } else {
-                    const R v = Tc - dt * div;
-                    if (own) at(dst, (uint32_t)idx) = v;
-                    nv = (double)v;
-                    FB(q) = fa;
+                    // a cell without the isoneutral flux has zero gradients here
+                    const R dzr = iso ? (R)dzrho : (R)1, dz2 = dzr * dzr, rdz2 = (R)1 / dz2;
+#pragma unroll
+                    for (int q = 0; q < LB; q++) {
+                        const R Tc = SP(cb, q, p), Te = SP(cb, q, nc.e), Tw = SP(cb, q, nc.w);
+                        const R Tn = SP(cb, q, nc.n), Ts = SP(cb, q, nc.s);
+                        const R fe = ue_ * rc * (((R)1.0 - upe) * Te + ((R)1.0 + upe) * Tc) * (R)0.5 - (Te - Tc) * rc2 * diff1;
+                        const R fw = uw_ * rc * (((R)1.0 - upw) * Tc + ((R)1.0 + upw) * Tw) * (R)0.5 - (Tc - Tw) * rc2 * diff1;
+                        const R fn = cvn * un_ * (((R)1.0 - upn) * Tn + ((R)1.0 + upn) * Tc) * (R)0.5 - cv2n * (Tn - Tc) * diff1;
+                        const R fs = cvs * us_ * (((R)1.0 - ups) * Tc + ((R)1.0 + ups) * Ts) * (R)0.5 - cv2s * (Tc - Ts) * diff1;
+                        R fa = 0;
+                        if constexpr (TOP) {
+                            if (M.sflux && q < nl) fa = (R)at(gp(M.sflux), (uint32_t)((l0 + q) * plane + col));
+                        } else {
+                            const R Tu = SP(ub, q, p);
+                            fa = ua_ * (((R)1.0 - upa) * Tu + ((R)1.0 + upa) * Tc) * (R)0.5;
+                            fa = fa - (Tu - Tc) * rdza * diffv;
+                            const R dzts = (Tu - Tc) * rdza;
+                            R tv = 0;
+#pragma unroll
+                            for (int n = 0; n < 4; n++) {
+                                const int b = n < 2 ? cb : ub;
+                                const bool east = n & 1;
+                                const Nbr& m = n < 2 ? nc : nu;
+                                const R dx = (east ? D(b, q, m.e, p) : D(b, q, p, m.w)) * rc * rdphi;
+                                const R dy = east ? D(b, q, m.n, p) * cvn * rdsvn : D(b, q, p, m.s) * cvs * rdsvs;
+                                tv = tv + ((R)2 * dzr * dx - dxr[n] * dzts) * dxr[n] + ((R)2 * dzr * dy - dyr[n] * dzts) * dyr[n];
+                            }
+                            // (isoc tv) / dz2, rounded as the division rounds
+                            // (Markstein 1990): with y = RN(1 / dz2) and q1 within an
+                            // ulp of the quotient, q1 + (a - dz2 q1) y rounds to it
+                            const R a = isoc * tv;
+                            const R q0 = a * rdz2;
+                            const R q1 = __builtin_fma(__builtin_fma(-dz2, q0, a), rdz2, q0);
+                            fa = fa + __builtin_fma(__builtin_fma(-dz2, q1, a), rdz2, q1);
+                        }
+                        const R div = ((fe - fw) * rdphi + (fn - fs) * rds) + (fa - FB(q)) * rdz;
+                        const int idx = (l0 + q) * tstride + o + col;
+                        const R v = Tc - dt * div;
+                        if (own && q < nl) at(dst, (uint32_t)idx) = v;
+                        FB(q) = fa;
+                        add_sum(q, (double)v);
+                    }
                 }
-                if (l0 + q == 0) newT = nv;
-                if (l0 + q == 1) newS = nv;
-                if (sums) add_sum(q, nv, s_os, s_mm, s_vv);
-            }
+            };
+            if (top)
+                tracers(std::true_type{});
+            else
+                tracers(std::false_type{});
             if (l0 == 0 && own) {
                 const double rn = eos<double>(g.ec[0], g.ec[1], g.ec[2], g.ec[3], newT, newS);
                 at(rhop, oc) = rn;
