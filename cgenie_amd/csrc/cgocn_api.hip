@@ -9,7 +9,6 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -125,6 +124,8 @@ double carry_unit_h(float x) {
 
 }  // namespace
 
+constexpr int INV_MAXL = 256;  // most tracers of a member
+
 struct cgo_engine {
     int device = 0;
     hipStream_t s = nullptr;
@@ -159,20 +160,10 @@ struct cgo_engine {
     size_t d_nv_cap = 0;        // doubles
     std::vector<int32_t> last_lists;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    double* h_inv = nullptr;    // [INV_MAXL] pinned: the inventory kernel stores its sums here
 };
 
-// Device memory of cgo_inventory_noalloc: the per-tracer sums of one call,
-// in place of the buffer cgo_inventory allocates.  Every GPU the library
-// runs on holds its own copy until the process ends.  Host code never uses
-// the array's name as an address: the device address of each GPU's copy is
-// taken once per device, with that device current, by
-// hipGetSymbolAddress (noalloc_setup, called from cgo_create), and only
-// that address reaches kernels and copies.
-constexpr int NOALLOC_MAXL = 64;  // tracers one allocation-free inventory takes
-static __device__ __align__(256) double scratch[NOALLOC_MAXL];
-constexpr int NOALLOC_MAXDEV = 64;
-static double* noalloc_ptr[NOALLOC_MAXDEV] = {};
-static std::mutex noalloc_mu;
+constexpr int NOALLOC_MAXL = 64;  // tracers one cgo_inventory_noalloc takes
 
 static int fail(cgo_engine* e, int code, const char* fmt, ...) {
     char buf[512];
@@ -229,18 +220,6 @@ int cgo_abi_info(int64_t* sizes, char* stamp, size_t n) {
     return CGO_OK;
 }
 
-// the device address of this device's scratch array, once per device
-// (the device is current); false if the runtime cannot give it
-static bool noalloc_setup(int device) {
-    if (device >= NOALLOC_MAXDEV) return true;  // such devices just have no allocation-free path
-    std::lock_guard<std::mutex> lk(noalloc_mu);
-    if (noalloc_ptr[device]) return true;
-    double* ptr = nullptr;
-    if (hipGetSymbolAddress((void**)&ptr, HIP_SYMBOL(scratch)) != hipSuccess || !ptr) return false;
-    noalloc_ptr[device] = ptr;
-    return true;
-}
-
 int cgo_create(int32_t device, cgo_engine** out) {
     if (!out) return CGO_E_ARG;
     *out = nullptr;
@@ -253,7 +232,8 @@ int cgo_create(int32_t device, cgo_engine** out) {
         hipMalloc(&e->d_table, TABLE_CAP * sizeof(MemberDev)) != hipSuccess ||
         hipEventCreate(&e->ev0) != hipSuccess || hipEventCreate(&e->ev1) != hipSuccess ||
         hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming) != hipSuccess || !noalloc_setup(device)) {
+        hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming) != hipSuccess ||
+        hipHostMalloc((void**)&e->h_inv, INV_MAXL * 8, hipHostMallocDefault) != hipSuccess) {
         delete e;
         return CGO_E_HIP;
     }
@@ -291,6 +271,7 @@ int cgo_destroy(cgo_engine* e) {
     if (e->d_list) hipFree(e->d_list);
     if (e->d_nv) hipFree(e->d_nv);
     if (e->d_table) hipFree(e->d_table);
+    if (e->h_inv) hipHostFree(e->h_inv);
     if (e->ev0) hipEventDestroy(e->ev0);
     if (e->ev1) hipEventDestroy(e->ev1);
     if (e->ev_fork) hipEventDestroy(e->ev_fork);
@@ -661,7 +642,7 @@ int cgo_member_create(cgo_engine* e, int32_t grid_id, int32_t maxl, int32_t prec
                       int32_t* member_id) {
     if (!e || !p || !member_id) return fail(e, CGO_E_ARG, "member_create: null argument");
     if (grid_id < 0 || grid_id >= (int)e->grids.size()) return fail(e, CGO_E_ARG, "member_create: bad grid %d", grid_id);
-    if (maxl < 2 || maxl > 256) return fail(e, CGO_E_ARG, "member_create: maxl %d outside 2..256", maxl);
+    if (maxl < 2 || maxl > INV_MAXL) return fail(e, CGO_E_ARG, "member_create: maxl %d outside 2..256", maxl);
     if (precision != CGO_FP64 && precision != CGO_FP32C) return fail(e, CGO_E_ARG, "member_create: bad precision");
     // kernels address per-member arrays with 32-bit byte offsets
     if ((size_t)maxl * e->grids[grid_id]->dev.ncell * sizeof(double) >= ((size_t)1 << 31))
@@ -1442,19 +1423,22 @@ int cgo_download_rho(cgo_engine* e, int32_t id, double* rho) {
     return CGO_OK;
 }
 
+// the launch stores every one of the member's L sums in pinned host memory,
+// where a device buffer's copy took as long as the kernel
+static int inventory(cgo_engine* e, const MemberH* m, int32_t id, double* inv) {
+    launch_inventory(e->d_table, id, m->L, e->h_inv, e->grids[m->grid]->d_invw, m->prec, e->s);
+    HIPCHK(e, hipGetLastError());
+    HIPCHK(e, hipStreamSynchronize(e->s));
+    std::copy(e->h_inv, e->h_inv + m->L, inv);
+    return CGO_OK;
+}
+
 int cgo_inventory(cgo_engine* e, int32_t id, double* inv) {
     MemberH* m = member(e, id);
     if (!m || !inv) return fail(e, CGO_E_ARG, "inventory: bad argument");
     int rc = sync_table(e);
     if (rc) return rc;
-    double* d_out = nullptr;
-    HIPCHK(e, hipMalloc(&d_out, (size_t)m->L * 8));
-    launch_inventory(e->d_table, id, m->L, d_out, e->grids[m->grid]->d_invw, m->prec, e->s);
-    HIPCHK(e, hipGetLastError());
-    HIPCHK(e, hipStreamSynchronize(e->s));
-    HIPCHK(e, hipMemcpy(inv, d_out, (size_t)m->L * 8, hipMemcpyDeviceToHost));
-    hipFree(d_out);
-    return CGO_OK;
+    return inventory(e, m, id, inv);
 }
 
 int cgo_inventory_noalloc(cgo_engine* e, int32_t id, double* inv) {
@@ -1463,8 +1447,6 @@ int cgo_inventory_noalloc(cgo_engine* e, int32_t id, double* inv) {
     if (m->L > NOALLOC_MAXL)
         return fail(e, CGO_E_ARG, "inventory_noalloc: member %d has %d tracers, at most %d without allocation", id, m->L,
                     NOALLOC_MAXL);
-    double* ptr = e->device < NOALLOC_MAXDEV ? noalloc_ptr[e->device] : nullptr;
-    if (!ptr) return fail(e, CGO_E_STATE, "inventory_noalloc: no scratch address for device %d", e->device);
     HIPCHK(e, hipSetDevice(e->device));
     if (e->table_dirty) {
         // bring this member's table entry up to date from the host copy (the
@@ -1473,12 +1455,7 @@ int cgo_inventory_noalloc(cgo_engine* e, int32_t id, double* inv) {
         HIPCHK(e, hipStreamSynchronize(e->s));
         HIPCHK(e, hipMemcpy(e->d_table + id, &m->dev, sizeof(MemberDev), hipMemcpyHostToDevice));
     }
-    // every one of the member's L sums is written by the launch: nothing to clear
-    launch_inventory(e->d_table, id, m->L, ptr, e->grids[m->grid]->d_invw, m->prec, e->s);
-    HIPCHK(e, hipGetLastError());
-    HIPCHK(e, hipStreamSynchronize(e->s));
-    HIPCHK(e, hipMemcpy(inv, ptr, (size_t)m->L * 8, hipMemcpyDeviceToHost));
-    return CGO_OK;
+    return inventory(e, m, id, inv);
 }
 
 // the device copy of the BIOGEM parameters, with each carried species' slot

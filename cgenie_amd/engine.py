@@ -366,7 +366,7 @@ class Engine:
         return out
 
     def inventory_noalloc(self, m: int) -> np.ndarray:
-        """cgo_inventory through the library's static scratch (no device allocation)."""
+        """cgo_inventory without any allocation by the library (at most 64 tracers)."""
         out = np.zeros(self.members[m])
         self._chk(self.L.cgo_inventory_noalloc(self.h, m, _ptr(out)), "inventory_noalloc")
         return out
