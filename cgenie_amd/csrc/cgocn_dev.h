@@ -274,6 +274,16 @@ enum { RT_LAYER = 0, RT_POC1, RT_POC2, RT_CAL1, RT_CAL2, RT_N };
 // following coupling), 1 after initialisation.
 enum { SC_SMEAN = 0, SC_SNEW, SC_SRATIO, SC_RSRATIO, SC_SOLD, SC_PSCALE, SC_FACT0 };  // SC_FACT0 + l : OLD_l * rNEW_l
 
+// planes [L][ncell] on their way to the host (launch_pack): doubles, or the
+// FP32 form with its carry planes (lo may be null); parity picks the buffer,
+// null: the first
+struct PackSrc {
+    const void* st[2];
+    const int16_t* lo[2];
+    const int32_t* parity;
+    uint32_t L, ncell;
+};
+
 // ---------------------------------------------------------------- helpers
 // Pointers read from the member table are generic (flat) to the compiler;
 // casting them to the global address space turns flat loads/stores into

@@ -95,4 +95,51 @@ void launch_inventory(const MemberDev* t, int32_t m, int L, double* out, const d
         hipLaunchKernelGGL(k_inventory<float>, dim3(L), dim3(256), 0, s, t, m, out, w);
 }
 
+// Cells [c0, c0 + nc) of planes [L][ncell] as rows of L doubles, the order the
+// host takes them in (go_ts(maxl, ...)), into pinned host memory: a block
+// turns CT cells around in LDS (an odd stride, so that neither side
+// meets a bank twice), reads whole lines of every plane and writes one
+// contiguous range.  Bound by PCIe (~56 GB/s).  FP32 states are decoded as the
+// host did it: float plus carry times 2^-16 ulp, the ulp of an infinity
+// infinite (an infinite value comes out NaN where its carry is zero).
+template <typename R, uint32_t CT>
+__global__ __launch_bounds__(256) void k_pack(PackSrc p, uint32_t c0, uint32_t nc, double* __restrict__ out) {
+    extern __shared__ __align__(16) double tile[];  // [L][CT + 1]
+    const int q = p.parity ? *gp(p.parity) : 0;
+    const AS_GLOBAL R* st = gp((const R*)p.st[q]);
+    const AS_GLOBAL int16_t* lo = p.lo[q] ? gp(p.lo[q]) : nullptr;
+    const uint32_t b0 = blockIdx.x * CT, n = min(CT, nc - b0), L = p.L;
+    for (uint32_t i = threadIdx.x; i < L * CT; i += 256) {
+        const uint32_t l = i / CT, c = i % CT;
+        if (c >= n) continue;
+        const uint32_t s = l * p.ncell + c0 + b0 + c;
+        double v;
+        if constexpr (sizeof(R) == 8) {
+            v = at(st, s);
+        } else {
+            const float h = at(st, s);
+            const double unit = (__float_as_uint(h) << 1) == 0xff000000u ? (double)INFINITY : carry_unit(h);
+            v = (double)h + (lo ? (double)at(lo, s) : 0.0) * unit;
+        }
+        tile[l * (CT + 1) + c] = v;
+    }
+    __syncthreads();
+    AS_GLOBAL double* o = gp(out) + (size_t)b0 * L;
+    for (uint32_t i = threadIdx.x; i < n * L; i += 256) o[i] = tile[(i % L) * (CT + 1) + i / L];
+}
+
+template <typename R, uint32_t CT>
+static void launch_pack_ct(const PackSrc& p, uint32_t c0, uint32_t nc, double* out, hipStream_t s) {
+    hipLaunchKernelGGL((k_pack<R, CT>), dim3((nc + CT - 1) / CT), dim3(256), (size_t)p.L * (CT + 1) * 8, s, p, c0, nc, out);
+}
+
+void launch_pack(const PackSrc& p, int prec, uint32_t c0, uint32_t nc, double* out, hipStream_t s) {
+    // 64 cells a block while their rows fit 64 KiB of LDS, else 16 (35 KB for 256 tracers)
+    const bool wide = p.L <= 126;
+    if (prec == 0)
+        (wide ? launch_pack_ct<double, 64> : launch_pack_ct<double, 16>)(p, c0, nc, out, s);
+    else
+        (wide ? launch_pack_ct<float, 64> : launch_pack_ct<float, 16>)(p, c0, nc, out, s);
+}
+
 }  // namespace cgo

@@ -559,3 +559,40 @@ def test_coupling_at_its_edges(dims, L, n):
     err = rel_err(got[0], gold.ts, wet(c))
     say(dims, L, n, "max rel err", err.max())
     assert np.all(err <= 1e-12)
+
+
+@pytest.mark.parametrize("dims,L,prec,carry", [
+    ((18, 18, 8), 2, E.FP64, True),        # one piece of the staging, the fewest tracers
+    ((19, 13, 7), 3, E.FP32C, True),       # odd sizes, a ragged last block
+    ((19, 13, 7), 126, E.FP32C, False),    # the most tracers of the wide blocks, no carry planes
+    ((19, 13, 7), 127, E.FP64, True),      # the first of the narrow blocks
+    ((18, 18, 8), 256, E.FP32C, True),     # the most tracers
+    ((36, 36, 16), 41, E.FP64, True),      # more pieces than the staging holds at once
+    ((36, 36, 16), 41, E.FP32C, True),
+])
+def test_download_rows(eng, dims, L, prec, carry):
+    """A downloaded state is the uploaded one, land and special values
+    included: FP64 as it was; FP32 forms as the float plus the carry times
+    2^-16 ulp, an infinity (its ulp infinite, its carry 0) as NaN."""
+    say("case", dims, L, prec, carry)
+    c = make_case(*dims, kind="ts", L=L)
+    rng = np.random.default_rng(17)
+    x = rng.normal(size=c.ts.shape) * 10.0 ** rng.integers(-12, 4, c.ts.shape)
+    flat = x.reshape(-1)
+    for i, v in enumerate((0.0, -0.0, np.inf, -np.inf, np.nan, 1e-41, -3e-40, 1e-310)):
+        flat[i::997] = v
+    m = eng.add_member(eng.add_grid(c.g, c.k1), L, prec, c.diff, carry=carry)
+    eng.upload(m, x)
+    got = eng.download(m, x.shape)
+    eng.remove_member(m)
+    if prec == E.FP64:
+        want = x
+    else:
+        with np.errstate(over="ignore", invalid="ignore"):
+            f = x.astype(np.float32).astype(np.float64)
+            ex = np.maximum(np.where((f == 0) | ~np.isfinite(f), -126, np.frexp(f)[1] - 1), -126)
+            lo = np.clip(np.rint(np.ldexp(x - f, 39 - ex)), -32767, 32767) if carry else 0.0
+            want = f + lo * np.ldexp(1.0, ex - 39)
+        want = np.where(np.isinf(x), np.nan, want)
+    assert np.array_equal(np.signbit(got) & ~np.isnan(want), np.signbit(want) & ~np.isnan(want))
+    assert np.array_equal(got, want, equal_nan=True)
