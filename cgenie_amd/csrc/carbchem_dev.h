@@ -98,20 +98,19 @@ __device__ inline void calc_carbconst(double D, double T, double S, double* cc) 
 struct Spec { double CO2, CO3, HCO3, H1, H2; };
 
 // one speciation sweep at [H] (gem_carbchem.f90:355-427); SiO2, H2S and NH4
-// are zero for the species the engine carries
+// are zero for the species the engine carries, and so are their terms
 __device__ __forceinline__ void carb_sweep(double H, double DIC, double ALK, double PO4t, double Bt, double SO4t,
                                            double Ft, const double* cc, Spec& o) {
     const double H2 = H * H, H3 = H * H2;
     const double OH = cc[CC_KW] / H;
     const double H4BO4 = Bt / (1.0 + H / cc[CC_KB]);
-    const double H3SiO4 = 0.0 / (1.0 + H / cc[CC_KSI]);
     const double HSO4 = SO4t / (1.0 + cc[CC_KHSO4] / H);
     const double HF = Ft / (1.0 + cc[CC_KHF] / H);
     const double P1 = cc[CC_KP1], P2 = cc[CC_KP2], P3 = cc[CC_KP3];
     const double H3PO4 = PO4t / (1.0 + P1 / H + (P1 * P2) / H2 + (P1 * P2 * P3) / H3);
     const double HPO4 = PO4t / (1.0 + H / P2 + H2 / (P1 * P2) + P3 / H);
     const double PO4 = PO4t / (1.0 + H / P3 + H2 / (P2 * P3) + H3 / (P1 * P2 * P3));
-    const double A = ALK - H4BO4 - OH - HPO4 - 2.0 * PO4 - H3SiO4 - 0.0 - 0.0 + H + HSO4 + HF + H3PO4;
+    const double A = ALK - H4BO4 - OH - HPO4 - 2.0 * PO4 + H + HSO4 + HF + H3PO4;
     const double K = cc[CC_K];
     const double t = 4.0 * A + DIC * K - A * K;
     const double zed = sqrt(t * t + 4.0 * (K - 4.0) * (A * A));
@@ -174,19 +173,98 @@ __device__ __forceinline__ void carb_sweep_fast(double H, double DIC, double ALK
     o.H2 = cc[CC_K2] * o.HCO3 * rcp_nr(o.CO3);
 }
 
+// Lane K of the quad's value, in all four lanes
+template <int K>
+__device__ __forceinline__ double quad_bcast(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), K * 0x55, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), K * 0x55, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// One solve's sweeps by Q lanes a column (1 or 4).  A sweep is one long chain
+// of ~25 IEEE divisions whose order is fixed, but many of them do not depend
+// on each other: with four lanes each takes one of the three-term
+// denominators (H3PO4, HPO4, PO4; HSO4 with two terms zero) and one of OH,
+// H4BO4 and HF, and even and odd lanes the two halves of what follows, the
+// same operations on the same operands.  For batches that leave most lanes of
+// the chip idle (launch_bio): one 36x36x16 FP64 member's whole step 105 -> 90 us.
+template <int Q>
+struct CarbSolve {
+    double DIC, ALK, PO4t, Bt, SO4t, Ft;
+    const double* cc;
+    int j;                  // this lane of the quad
+    double c1, c2, c3, T1, cb, T2;
+    __device__ __forceinline__ CarbSolve(double DIC_, double ALK_, double PO4_, double B_, double SO4_, double F_,
+                                         const double* cc_)
+        : DIC(DIC_), ALK(ALK_), PO4t(PO4_), Bt(B_), SO4t(SO4_), Ft(F_), cc(cc_), j(threadIdx.x & 3) {
+        if constexpr (Q == 4) {
+            const double P1 = cc[CC_KP1], P2 = cc[CC_KP2], P3 = cc[CC_KP3];
+            c1 = j == 0 ? P1 : j == 1 ? P2 : j == 2 ? P3 : cc[CC_KHSO4];
+            c2 = j <= 1 ? P1 * P2 : j == 2 ? P2 * P3 : 1.0;
+            c3 = j == 1 ? P3 : j == 3 ? 1.0 : P1 * P2 * P3;
+            T1 = j == 3 ? SO4t : PO4t;
+            cb = j == 0 ? cc[CC_KW] : j == 1 ? cc[CC_KB] : j == 2 ? cc[CC_KHF] : 1.0;
+            T2 = j == 1 ? Bt : Ft;
+        }
+    }
+    // x / y of the even lanes, u / v of the odd ones
+    __device__ __forceinline__ void div2(double x, double y, double u, double v, double& xy, double& uv) const {
+        if constexpr (Q == 4) {
+            const double q = (j & 1 ? u : x) / (j & 1 ? v : y);
+            xy = quad_bcast<0>(q);
+            uv = quad_bcast<1>(q);
+        } else {
+            xy = x / y;
+            uv = u / v;
+        }
+    }
+    __device__ __forceinline__ void sweep(double H, Spec& o) const {
+        if constexpr (Q == 1) {
+            carb_sweep(H, DIC, ALK, PO4t, Bt, SO4t, Ft, cc, o);
+        } else {
+            const double H2 = H * H, H3 = H * H2;
+            const bool inv = j == 0 || j == 3;
+            const double a1 = (inv ? c1 : H) / (inv ? H : c1);
+            const double a2 = (j == 0 ? c2 : j == 3 ? 0.0 : H2) / (j == 0 ? H2 : c2);
+            const double a3 = (j <= 1 ? c3 : j == 3 ? 0.0 : H3) / (j == 0 ? H3 : j == 1 ? H : c3);
+            const double s1 = T1 / (1.0 + a1 + a2 + a3);
+            const double b = (j == 1 ? H : cb) / (j == 1 ? cb : H);
+            const double s2 = j == 0 ? b : T2 / (1.0 + b);
+            const double H3PO4 = quad_bcast<0>(s1), HPO4 = quad_bcast<1>(s1), PO4 = quad_bcast<2>(s1);
+            const double HSO4 = quad_bcast<3>(s1);
+            const double OH = quad_bcast<0>(s2), H4BO4 = quad_bcast<1>(s2), HF = quad_bcast<2>(s2);
+            const double A = ALK - H4BO4 - OH - HPO4 - 2.0 * PO4 + H + HSO4 + HF + H3PO4;
+            const double K = cc[CC_K];
+            const double t = 4.0 * A + DIC * K - A * K;
+            const double zed = sqrt(t * t + 4.0 * (K - 4.0) * (A * A));
+            div2(DIC * K - zed, K - 4.0, A * K - DIC * K - 4.0 * A + zed, 2.0 * (K - 4.0), o.HCO3, o.CO3);
+            o.CO2 = DIC - A + o.CO3;
+            div2(cc[CC_K1] * o.CO2, o.HCO3, cc[CC_K2] * o.HCO3, o.CO3, o.H1, o.H2);
+        }
+    }
+};
+
 // sub_calc_carb: >0 iterations, -1 negative [H] estimate, -2 iteration limit
 // (ctrl_carbchem_fail: carb is left unchanged, no random re-seed)
+template <int Q>
 __device__ inline int calc_carb(double DIC, double ALK, double Ca, double PO4, double Bt, double SO4t, double Ft,
-                                const double* cc, AS_GLOBAL double* carb, size_t cs, double tol, int maxit) {
+                                const double* cc, AS_GLOBAL double* carb, size_t cs, double tol, int maxit, double& Hout,
+                                double& CO2out) {
+    const CarbSolve<Q> S(DIC, ALK, PO4, Bt, SO4t, Ft, cc);
     int n = 1;
-    double H = carb[IC_H * cs];
+    double H = Hout;
     Spec o;
     for (;;) {
         const double Hold = H;
-        carb_sweep(H, DIC, ALK, PO4, Bt, SO4t, Ft, cc, o);
+        S.sweep(H, o);
         if ((o.H1 < NULLSMALL) || (o.H2 < NULLSMALL)) return -1;
         H = sqrt(o.H1 * o.H2);
-        if (fabs(1.0 - H / Hold) < (1.0E-8 / H) * tol) {
+        double ratio, lim;
+        S.div2(H, Hold, 1.0E-8, H, ratio, lim);
+        if (fabs(1.0 - ratio) < lim * tol) {
+            Hout = H;
+            CO2out = o.CO2;
+            if (Q == 4 && S.j != 0) return n;
             carb[IC_CONC_CO2 * cs] = o.CO2;
             carb[IC_CONC_CO3 * cs] = o.CO3;
             carb[IC_CONC_HCO3 * cs] = o.HCO3;
@@ -203,23 +281,25 @@ __device__ inline int calc_carb(double DIC, double ALK, double Ca, double PO4, d
     }
 }
 
+template <int Q>
 __device__ inline int calc_carb_RF0(double DIC, double ALK, double PO4, double Bt, double SO4t, double Ft,
-                                    const double* cc, AS_GLOBAL double* carb, size_t cs, double tol, int maxit) {
-    int n = 1;
-    double H = carb[IC_H * cs];
+                                    const double* cc, AS_GLOBAL double* carb, size_t cs, double tol, int maxit,
+                                    double H, double CO2) {
     const double DICr = DIC + 1.0e-6;
+    const CarbSolve<Q> S(DICr, ALK, PO4, Bt, SO4t, Ft, cc);
+    int n = 1;
     Spec o;
     for (;;) {
         const double Hold = H;
-        carb_sweep(H, DICr, ALK, PO4, Bt, SO4t, Ft, cc, o);
+        S.sweep(H, o);
         H = sqrt(o.H1 * o.H2);
         if (fabs(1.0 - H / Hold) < tol) {
-            carb[IC_RF0 * cs] = (o.CO2 / carb[IC_CONC_CO2 * cs] - 1.0) / (DICr / DIC - 1.0);
+            if (Q == 1 || S.j == 0) carb[IC_RF0 * cs] = (o.CO2 / CO2 - 1.0) / (DICr / DIC - 1.0);
             return n;
         }
         n = n + 1;
         if ((o.H1 < NULLSMALL) || (o.H2 < NULLSMALL) || (n > maxit)) {
-            carb[IC_RF0 * cs] = 0.0;
+            if (Q == 1 || S.j == 0) carb[IC_RF0 * cs] = 0.0;
             return -1;
         }
     }

@@ -24,7 +24,7 @@ void launch_flux32(const MemberDev*, const int32_t*, int nlist, const FluxShape&
 void launch_co(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int prec, const FluxSplit&,
                hipStream_t);
 void launch_flip(const MemberDev*, const int32_t*, int nlist, hipStream_t);
-void launch_bio(const MemberDev*, const int32_t*, int nlist, int nwetmax, int W, int prec, hipStream_t);
+void launch_bio(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int W, int prec, hipStream_t);
 void launch_coupling(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int maxL, int prec,
                      int phase, hipStream_t);
 void launch_pack(const PackSrc&, int prec, uint32_t c0, uint32_t nc, double* out, hipStream_t);
@@ -378,7 +378,9 @@ static int rows_out(cgo_engine* e, MemberH* m, const PackSrc& p, int prec, doubl
 }
 
 // L planes of doubles
-static PackSrc planes(const void* p, int L, size_t ncell) { return {{p, nullptr}, {}, nullptr, (uint32_t)L, (uint32_t)ncell}; }
+static PackSrc planes(const void* p, int L, size_t ncell) {
+    return {{p, nullptr}, {}, nullptr, (uint32_t)L, (uint32_t)ncell};
+}
 
 extern "C" {
 
@@ -2193,7 +2195,8 @@ static void enqueue_tstepo(cgo_engine* e, const Lists& ls, const int32_t* d_list
 static void enqueue_bio(cgo_engine* e, const Lists& ls, const int32_t* d_lists, hipStream_t s) {
     for (int p = 0; p < 2; p++)
         if (ls.n[2 + p])
-            launch_bio(e->d_table, d_lists + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.wstream[p], p, s);
+            launch_bio(e->d_table, d_lists + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.maxk_bgc[p], ls.wstream[p],
+                       p, s);
     if (ls.ncol_atm)
         for (int p = 0; p < 2; p++)
             if (ls.n[2 + p]) launch_atchem(e->d_table, d_lists + ls.off[2 + p], ls.n[2 + p], ls.ncol_atm, s);
@@ -2542,9 +2545,11 @@ int cgo_time_kernel(cgo_engine* e, int32_t which, const int32_t* ids, int32_t n,
                 launch_co(e->d_table, l, ls.n[p], ls.maxwet[p], ls.maxk[p], p, ls.sp[p], e->s);
             } else if (which == 4) {
                 if (ls.n[2 + p])
-                    launch_bio(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.wstream[p], p, e->s);
+                    launch_bio(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.maxk_bgc[p],
+                               ls.wstream[p], p, e->s);
             } else if (ls.n[2 + p]) {
-                launch_bio(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.wstream[p], p, e->s);
+                launch_bio(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.maxk_bgc[p],
+                           ls.wstream[p], p, e->s);
                 launch_coupling(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.maxk_bgc[p],
                                 ls.maxL[p], p, 0, e->s);
             }

@@ -4,14 +4,16 @@
 // FP64 results track the CPU restatement to the last bits (only the device
 // exp/log/pow differ from glibc, within 1 ulp).
 //
-// k_bgc_col   one thread per (member, wet column), everything it carries
-//             down the column held in registers: the surface carbonate
-//             chemistry (biogem.f90:1026-1084), then one march from
-//             the surface to k1 that applies, level by level, DOM
-//             remineralisation (biogem_box.f90:2287-2406), particulate
-//             remineralisation (2412-2877), the sediment return of the
-//             previous step's rain (biogem.f90:873-942) and PO4 uptake
-//             (biogem_box.f90:346-1515).  Every cell is read and written once.
+// k_bgc_col   one block per (member, 64 wet columns), a wave for the surface
+//             carbonate chemistry (biogem.f90:1026-1084), the air-sea flux and
+//             the PO4 uptake (biogem_box.f90:346-1515), and a wave for the
+//             march from the surface to k1 that applies, level by level, DOM
+//             remineralisation (2287-2406), particulate remineralisation
+//             (2412-2877) and the sediment return of the previous step's rain
+//             (biogem.f90:873-942), everything it carries down the column held
+//             in registers; the first wave then adds the uptake and the
+//             air-sea flux at the levels they touch (large batches: one wave
+//             for all of it).
 // k_couple_sums    one block per (member, 64 wet columns): the column partial
 //             sums of the state after transport (biogem.f90:1984-1997,
 //             2016-2025).
@@ -175,13 +177,26 @@ struct Streams {
     int mk[W];  // settling level of the stream, -2 for a free slot
 };
 
-template <typename R, int W>
-__global__ __launch_bounds__(64) void k_bgc_col(const MemberDev* __restrict__ mems, const int32_t* __restrict__ list) {
+// What bounds it: two long dependent chains per column, the carbonate solve
+// and the march, and too few columns to hide either.  The march reads nothing
+// of the surface part, whose results come last at the few levels they touch:
+// side by side in two waves, one 36x36x16 FP64 member takes 74 us where one
+// thread did both in 90, eight FP32C members 37 for 54; and neither part
+// carries the other's registers (141 for 161 at W = 5).  Q is the lanes per
+// column of the surface part, 0: both parts in one wave (launch_bio).
+template <typename R, int W, int Q>
+__global__ __launch_bounds__(Q > 0 ? 64 * Q + 64 : 64) void k_bgc_col(const MemberDev* __restrict__ mems,
+                                                         const int32_t* __restrict__ list) {
     const BlockXYZ B = xcd_blk();
     const MemberDev& M = mems[list[B.y]];
     const GridDev& g = M.g;
-    const int w = B.x * 64 + threadIdx.x;
-    if (w >= g.nwet) return;
+    if (B.x * 64 >= g.nwet) return;
+    constexpr int S = Q > 0 ? 64 * Q : 64;  // threads of the surface part
+    const bool marches = Q > 0 && __builtin_amdgcn_readfirstlane((int)threadIdx.x) >= S;  // the wave's part
+    const int w0 = B.x * 64 + (marches ? threadIdx.x - S : threadIdx.x / (S / 64));
+    const bool lead = Q <= 1 || (threadIdx.x & (Q - 1)) == 0;  // the surface part's lane that stores
+    const bool on = w0 < g.nwet;
+    const int w = on ? w0 : g.nwet - 1;
     const BgcParams& p = M.bp;
     const int col = gp(g.wetsorted)[w];
     const int maxi = g.maxi, maxk = g.maxk;
@@ -201,123 +216,128 @@ __global__ __launch_bounds__(64) void k_bgc_col(const MemberDev* __restrict__ me
     make_conv(p, cv);
 
     // (1) surface carbonate chemistry (biogem.f90:1026-1084)
-    double ohm = 0.0;
-    if (p.slot[B_DIC] >= 0 && p.slot[B_ALK] >= 0) {
-        AS_GLOBAL double* carb = gp(M.carb) + col;
-        const size_t cs = cell(maxk);
-        const double Tsur = ocn[cs], Ssur = ocn[ncell + cs];
-        double cc[NCC];
-        calc_carbconst(Dmid[maxk], Tsur, Ssur, cc);
-        const double Ca = salt_Ca(Ssur), B = salt_B(Ssur), SO4 = salt_SO4(Ssur), F = salt_F(Ssur);
-        const double DIC = ocn[(size_t)p.ocn[B_DIC] * ncell + cs], ALK = ocn[(size_t)p.ocn[B_ALK] * ncell + cs];
-        const double PO4 = hasPO4 ? ocn[(size_t)p.ocn[B_PO4] * ncell + cs] : 0.0;
-        // FP64 members: the reference's plain iteration; FP32-form members:
-        // the same fixed point, accelerated
-        constexpr bool fast = sizeof(R) == 4;
-        const int it = fast ? calc_carb_fast(DIC, ALK, Ca, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit)
-                            : calc_carb(DIC, ALK, Ca, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit);
-        if (it < 0)
-            atomicAdd(&M.diag[1], 1);
-        else
-            atomicAdd(&M.diag[2], it);
-        if (fast)
-            calc_carb_RF0_fast(DIC, ALK, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit);
-        else
-            calc_carb_RF0(DIC, ALK, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit);
-        ohm = carb[IC_OHM_CAL * plane];
-    }
-
-    // air-sea exchange (biogem.f90:1044-1046, 1605-1614) with the density of
-    // biogem_climate (fun_calc_rho, gem_util.f90:670-688; biogem.f90:2187)
     double fair[2] = {0.0, 0.0};
-    if (p.airsea) {
-        const size_t cs = cell(maxk);
-        const double T = ocn[cs], S = ocn[ncell + cs];
-        const double TC = T - ZEROC;
-        const double rho = 1000.0 + (0.7968 * S - 0.0559 * TC - 0.0063 * (TC * TC) + 3.7315E-05 * (TC * (TC * TC)));
-        const int J = col / maxi + 1;
-        const double A = cell_area(gp(g.mj) + MJ_SV * (g.maxj + 2), maxi, J);
-        const double dD = gp(g.mk)[MK_DD * KS + maxk];
-        const double u = gp(M.wspeed)[col];
-        const AS_GLOBAL double* atm = gp(M.atm);
-        if (p.slot[B_DIC] >= 0 && p.slot[B_ALK] >= 0) {
-            const AS_GLOBAL double* carb = gp(M.carb) + col;
-            const double sol = solconst(-60.2409, 93.4517, 23.3585, 0.023517, -0.023656, 0.0047036, false, T, S, rho);
-            const double pv = piston(2073.1, 125.62, 3.6276, 0.043219, T, u, p.gas_a);
-            const double CO2 = carb[IC_CONC_CO2 * plane], RF0 = carb[IC_RF0 * plane];
-            double atmv = sol * atm[col], ocnv = CO2, buff;
-            if (RF0 > NULLSMALL) {
-                buff = 1.0 / (RF0 * CO2 / ocn[(size_t)p.ocn[B_DIC] * ncell + cs]);
-            } else {
-                ocnv = 0.0;
-                atmv = 0.0;
-                buff = 1.0;
-            }
-            fair[0] = ocnatm_flux(pv, A, rho, dD, ocnv, atmv, buff, p.dtyr);
-        }
-        if (hasO2) {
-            const double sol = solconst(-58.3877, 85.8079, 23.8439, -0.034892, 0.015568, -0.0019387, true, T, S, rho);
-            const double pv = piston(1953.4, 128.00, 3.9918, 0.050091, T, u, p.gas_a);
-            fair[1] = ocnatm_flux(pv, A, rho, dD, ocn[(size_t)p.ocn[B_O2] * ncell + cs], sol * atm[plane + col], 1.0,
-                                  p.dtyr);
-        }
-        gp(M.fatm)[col] = fair[0];
-        gp(M.fatm)[plane + col] = fair[1];
-    }
-
-    // (2) PO4 uptake of this column (biogem_box.f90:346-1515): the same
-    //     particulate and dissolved change at every level from kstart up
     int kstart = maxk + 1;
     double upart[NSED] = {0.0, 0.0, 0.0, 0.0, 0.0}, upt[4] = {0.0, 0.0, 0.0, 0.0}, domC = 0.0, domP = 0.0;
-    if (hasPO4) {
-        int k_mld = kb;
-        const double mld = gp(M.mld)[col];
-        for (int k = maxk; k >= 1; k--)
-            if (Dbot[k] >= mld) {
-                k_mld = k;
-                break;
+    auto surface = [&]() {
+        double ohm = 0.0;
+        if (p.slot[B_DIC] >= 0 && p.slot[B_ALK] >= 0) {
+            AS_GLOBAL double* carb = gp(M.carb) + col;
+            const size_t cs = cell(maxk);
+            const double Tsur = ocn[cs], Ssur = ocn[ncell + cs];
+            double cc[NCC];
+            calc_carbconst(Dmid[maxk], Tsur, Ssur, cc);
+            const double Ca = salt_Ca(Ssur), B = salt_B(Ssur), SO4 = salt_SO4(Ssur), F = salt_F(Ssur);
+            const double DIC = ocn[(size_t)p.ocn[B_DIC] * ncell + cs], ALK = ocn[(size_t)p.ocn[B_ALK] * ncell + cs];
+            const double PO4 = hasPO4 ? ocn[(size_t)p.ocn[B_PO4] * ncell + cs] : 0.0;
+            // FP64 members: the reference's plain iteration; FP32-form members:
+            // the same fixed point, accelerated
+            constexpr bool fast = sizeof(R) == 4;
+            int it;
+            if constexpr (fast) {
+                it = calc_carb_fast(DIC, ALK, Ca, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit);
+                calc_carb_RF0_fast(DIC, ALK, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit);
+            } else {
+                double H = carb[IC_H * plane], CO2 = carb[IC_CONC_CO2 * plane];
+                it = calc_carb<S / 64>(DIC, ALK, Ca, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit, H, CO2);
+                calc_carb_RF0<S / 64>(DIC, ALK, PO4, B, SO4, F, cc, carb, plane, p.carb_tol, p.carb_maxit, H, CO2);
             }
-        kstart = k_mld < kb ? kb : k_mld;
-        const double lPO4 = ocn[(size_t)p.ocn[B_PO4] * ncell + cell(maxk)];
-        const double kPO4 = lPO4 / (lPO4 + p.c0_PO4);
-        const double ficefree = (1.0 - 0.0);
-        const double kI = gp(M.light)[col];
-        double dPO4 = 0.0;
-        if (lPO4 > NULLSMALL) dPO4 = p.dtyr * ficefree * kI * kPO4 * p.k0_PO4;
-        double DOMfrac = p.DOMfrac;
-        double DOMtotal = DOMfrac + 0.0;
-        if (DOMtotal > 1.0) {
-            DOMfrac = DOMfrac / DOMtotal;
-            DOMtotal = 1.0;
+            if (lead) {
+                atomicAdd(&M.diag[it < 0 ? 1 : 2], it < 0 ? 1 : it);
+                ohm = carb[IC_OHM_CAL * plane];
+            }
         }
-        double rCaCO3 = 0.0;
-        if (p.caco3 && ohm > 1.0) rCaCO3 = (1.0 - DOMtotal) * p.red_POC_CaCO3 * pow(ohm - 1.0, p.red_POC_CaCO3_pP);
-        const double red_POC_POP = 1.0 / p.red_POP_POC;
-        const double kPO4f = lPO4 / (lPO4 + p.POC_c0frac2);
-        const double fr2 = (1.0 - kPO4f) * p.POC_dfrac2 + p.POC_frac2;
-        double bp[NSED];
-        bp[S_POC] = p.red_POP_POC * dPO4;
-        bp[S_CACO3] = p.caco3 ? rCaCO3 * bp[S_POC] : 0.0;
-        bp[S_POP] = red_POC_POP * bp[S_POC];
-        for (int s = 0; s < 3; s++) {
-            if (s == S_CACO3 && !p.caco3) continue;
-            for (int q = 0; q < 4; q++)
-                if (cv.c[s][q] != 0.0) upt[q] = upt[q] + cv.c[s][q] * bp[s];
+        if (!lead) return;
+
+        // air-sea exchange (biogem.f90:1044-1046, 1605-1614) with the density of
+        // biogem_climate (fun_calc_rho, gem_util.f90:670-688; biogem.f90:2187)
+        if (p.airsea) {
+            const size_t cs = cell(maxk);
+            const double T = ocn[cs], S = ocn[ncell + cs];
+            const double TC = T - ZEROC;
+            const double rho = 1000.0 + (0.7968 * S - 0.0559 * TC - 0.0063 * (TC * TC) + 3.7315E-05 * (TC * (TC * TC)));
+            const int J = col / maxi + 1;
+            const double A = cell_area(gp(g.mj) + MJ_SV * (g.maxj + 2), maxi, J);
+            const double dD = gp(g.mk)[MK_DD * KS + maxk];
+            const double u = gp(M.wspeed)[col];
+            const AS_GLOBAL double* atm = gp(M.atm);
+            if (p.slot[B_DIC] >= 0 && p.slot[B_ALK] >= 0) {
+                const AS_GLOBAL double* carb = gp(M.carb) + col;
+                const double sol = solconst(-60.2409, 93.4517, 23.3585, 0.023517, -0.023656, 0.0047036, false, T, S, rho);
+                const double pv = piston(2073.1, 125.62, 3.6276, 0.043219, T, u, p.gas_a);
+                const double CO2 = carb[IC_CONC_CO2 * plane], RF0 = carb[IC_RF0 * plane];
+                double atmv = sol * atm[col], ocnv = CO2, buff;
+                if (RF0 > NULLSMALL) {
+                    buff = 1.0 / (RF0 * CO2 / ocn[(size_t)p.ocn[B_DIC] * ncell + cs]);
+                } else {
+                    ocnv = 0.0;
+                    atmv = 0.0;
+                    buff = 1.0;
+                }
+                fair[0] = ocnatm_flux(pv, A, rho, dD, ocnv, atmv, buff, p.dtyr);
+            }
+            if (hasO2) {
+                const double sol = solconst(-58.3877, 85.8079, 23.8439, -0.034892, 0.015568, -0.0019387, true, T, S, rho);
+                const double pv = piston(1953.4, 128.00, 3.9918, 0.050091, T, u, p.gas_a);
+                fair[1] = ocnatm_flux(pv, A, rho, dD, ocn[(size_t)p.ocn[B_O2] * ncell + cs], sol * atm[plane + col], 1.0,
+                                      p.dtyr);
+            }
+            gp(M.fatm)[col] = fair[0];
+            gp(M.fatm)[plane + col] = fair[1];
         }
-        domC = 1.0 * DOMfrac * bp[S_POC];
-        domP = 1.0 * DOMfrac * bp[S_POP];
-        bp[S_POC] = bp[S_POC] - (domC + 0.0);
-        bp[S_POP] = bp[S_POP] - (domP + 0.0);
-        bp[S_CACO3] = bp[S_CACO3] - (0.0 + 0.0);
-        bp[S_POCFR2] = fr2;
-        bp[S_CACO3FR2] = p.caco3 ? p.CaCO3_frac2 : 0.0;
-        for (int s = 0; s < NSED; s++) upart[s] = bp[s];
-    }
+
+        // (2) PO4 uptake of this column (biogem_box.f90:346-1515): the same
+        //     particulate and dissolved change at every level from kstart up
+        if (hasPO4) {
+            int k_mld = kb;
+            const double mld = gp(M.mld)[col];
+            for (int k = maxk; k >= 1; k--)
+                if (Dbot[k] >= mld) {
+                    k_mld = k;
+                    break;
+                }
+            kstart = k_mld < kb ? kb : k_mld;
+            const double lPO4 = ocn[(size_t)p.ocn[B_PO4] * ncell + cell(maxk)];
+            const double kPO4 = lPO4 / (lPO4 + p.c0_PO4);
+            const double ficefree = (1.0 - 0.0);
+            const double kI = gp(M.light)[col];
+            double dPO4 = 0.0;
+            if (lPO4 > NULLSMALL) dPO4 = p.dtyr * ficefree * kI * kPO4 * p.k0_PO4;
+            double DOMfrac = p.DOMfrac;
+            double DOMtotal = DOMfrac + 0.0;
+            if (DOMtotal > 1.0) {
+                DOMfrac = DOMfrac / DOMtotal;
+                DOMtotal = 1.0;
+            }
+            double rCaCO3 = 0.0;
+            if (p.caco3 && ohm > 1.0) rCaCO3 = (1.0 - DOMtotal) * p.red_POC_CaCO3 * pow(ohm - 1.0, p.red_POC_CaCO3_pP);
+            const double red_POC_POP = 1.0 / p.red_POP_POC;
+            const double kPO4f = lPO4 / (lPO4 + p.POC_c0frac2);
+            const double fr2 = (1.0 - kPO4f) * p.POC_dfrac2 + p.POC_frac2;
+            double bp[NSED];
+            bp[S_POC] = p.red_POP_POC * dPO4;
+            bp[S_CACO3] = p.caco3 ? rCaCO3 * bp[S_POC] : 0.0;
+            bp[S_POP] = red_POC_POP * bp[S_POC];
+            for (int s = 0; s < 3; s++) {
+                if (s == S_CACO3 && !p.caco3) continue;
+                for (int q = 0; q < 4; q++)
+                    if (cv.c[s][q] != 0.0) upt[q] = upt[q] + cv.c[s][q] * bp[s];
+            }
+            domC = 1.0 * DOMfrac * bp[S_POC];
+            domP = 1.0 * DOMfrac * bp[S_POP];
+            bp[S_POC] = bp[S_POC] - (domC + 0.0);
+            bp[S_POP] = bp[S_POP] - (domP + 0.0);
+            bp[S_CACO3] = bp[S_CACO3] - (0.0 + 0.0);
+            bp[S_POCFR2] = fr2;
+            bp[S_CACO3FR2] = p.caco3 ? p.CaCO3_frac2 : 0.0;
+            for (int s = 0; s < NSED; s++) upart[s] = bp[s];
+        }
+    };
 
     // (3) the march, surface to k1
-    AS_GLOBAL double* __restrict__ part = gp(M.part);
+    AS_GLOBAL double* part = gp(M.part);
     const double pscale = gp(M.scal)[SC_PSCALE];  // the last coupling's ratio, pending on part
-    AS_GLOBAL double* __restrict__ vd = gp(M.vd);
+    AS_GLOBAL double* vd = gp(M.vd);  // (both are passed from wave to wave)
     const AS_GLOBAL double* __restrict__ pO2 = hasO2 ? ocn + (size_t)p.ocn[B_O2] * ncell : nullptr;
     const AS_GLOBAL double* __restrict__ pDC = hasDOMC ? ocn + (size_t)p.ocn[B_DOMC] * ncell : nullptr;
     const AS_GLOBAL double* __restrict__ pDP = hasDOMP ? ocn + (size_t)p.ocn[B_DOMP] * ncell : nullptr;
@@ -342,6 +362,30 @@ __global__ __launch_bounds__(64) void k_bgc_col(const MemberDev* __restrict__ me
 #pragma unroll
         for (int s = 0; s < NSED; s++)
             settle[s] = settle[s] + ((s == S_POCFR2 || s == S_CACO3FR2) ? t[s] : Mkb * t[s]);
+    };
+    // the uptake and the air-sea flux of a level, on what the march forms there
+    auto touch = [&](int k, double* v, double& vdc, double& vdp) {
+        if (k >= kstart) {
+            vdc = vdc + domC;
+            vdp = vdp + domP;
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = v[q] - upt[q];
+        }
+        // vdocn = bio_remin + dtyr rM locijk_focn (biogem.f90:1821-1833): the
+        // surface takes minus the ocean -> atmosphere flux
+        if (p.airsea && k == maxk) {
+            const double dtrM = p.dtyr * gp(M.rM)[cell(k)];
+            v[B_DIC] = v[B_DIC] + dtrM * (0.0 - fair[0]);
+            v[B_O2] = v[B_O2] + dtrM * (0.0 - fair[1]);
+        }
+    };
+    auto store = [&](int k, const double* v, double vdc, double vdp) {
+        const size_t c = cell(k);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (p.slot[q] >= 0) vd[(size_t)q * ncell + c] = v[q];
+        if (hasDOMC) vd[(size_t)B_DOMC * ncell + c] = vdc;
+        if (hasDOMP) vd[(size_t)B_DOMP * ncell + c] = vdp;
     };
     // one target level; `streams` steps the live streams in source order
     auto level = [&](int kk, const Lvl& cur, auto&& streams, auto&& push) {
@@ -393,28 +437,11 @@ __global__ __launch_bounds__(64) void k_bgc_col(const MemberDev* __restrict__ me
 #pragma unroll
             for (int q = 0; q < 4; q++) v[q] = rMkb * fsed[q] + v[q];
         }
-        const size_t c = cell(kk);
-        const bool up = hasPO4 && kk >= kstart;
-        if (up) {
-            vdc = vdc + domC;
-            vdp = vdp + domP;
+        const bool up = Q == 0 && kk >= kstart;
+        if constexpr (Q == 0) touch(kk, v, vdc, vdp);
 #pragma unroll
-            for (int q = 0; q < 4; q++) v[q] = v[q] - upt[q];
-        }
-        // vdocn = bio_remin + dtyr rM locijk_focn (biogem.f90:1821-1833): the
-        // surface takes minus the ocean -> atmosphere flux
-        if (p.airsea && kk == maxk) {
-            const double dtrM = p.dtyr * gp(M.rM)[c];
-            v[B_DIC] = v[B_DIC] + dtrM * (0.0 - fair[0]);
-            v[B_O2] = v[B_O2] + dtrM * (0.0 - fair[1]);
-        }
-#pragma unroll
-        for (int s = 0; s < NSED; s++) part[(size_t)s * ncell + c] = up ? upart[s] : np[s];
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (p.slot[q] >= 0) vd[(size_t)q * ncell + c] = v[q];
-        if (hasDOMC) vd[(size_t)B_DOMC * ncell + c] = vdc;
-        if (hasDOMP) vd[(size_t)B_DOMP * ncell + c] = vdp;
+        for (int s = 0; s < NSED; s++) part[(size_t)s * ncell + cell(kk)] = up ? upart[s] : np[s];
+        store(kk, v, vdc, vdp);
     };
     // stepping one live stream through level kk
     auto advance = [&](double* t, int& mk, int kk, double rf, double* v, double* np) {
@@ -431,63 +458,93 @@ __global__ __launch_bounds__(64) void k_bgc_col(const MemberDev* __restrict__ me
         }
     };
 
-    Lvl cur, nxt;
-    load(maxk, cur);
-    if (klim == maxk) {
-        // particles sink out of the column within one step: one source
-        double t1[NSED];
-        int mk1 = -2;
-        for (int kk = maxk; kk >= kb; kk--) {
-            if (kk > kb) load(kk - 1, nxt);
-            level(
-                kk, cur,
-                [&](int k_, double rf, double* v, double* np) {
-                    if (mk1 > -2) advance(t1, mk1, k_, rf, v, np);
-                },
-                [&](const double* t, int mk) {
+    auto march = [&]() {
+        Lvl cur, nxt;
+        load(maxk, cur);
+        if (klim == maxk) {
+            // particles sink out of the column within one step: one source
+            double t1[NSED];
+            int mk1 = -2;
+            for (int kk = maxk; kk >= kb; kk--) {
+                if (kk > kb) load(kk - 1, nxt);
+                level(
+                    kk, cur,
+                    [&](int k_, double rf, double* v, double* np) {
+                        if (mk1 > -2) advance(t1, mk1, k_, rf, v, np);
+                    },
+                    [&](const double* t, int mk) {
 #pragma unroll
-                    for (int s = 0; s < NSED; s++) t1[s] = t[s];
-                    mk1 = mk;
-                });
-            cur = nxt;
-        }
-    } else {
-        // at level kk slot j holds the stream of source kk + 1 + j; after the
-        // level every stream moves down one slot and source kk enters slot 0
-        // (the stream of source kk + W - 1 has settled by then)
-        Streams<W - 1> S;
-#pragma unroll
-        for (int j = 0; j < W - 1; j++) S.mk[j] = -2;
-        for (int kk = maxk; kk >= kb; kk--) {
-            if (kk > kb) load(kk - 1, nxt);
-            double pt[NSED] = {0.0, 0.0, 0.0, 0.0, 0.0};
-            int pmk = -2;
-            level(
-                kk, cur,
-                [&](int k_, double rf, double* v, double* np) {
-#pragma unroll
-                    for (int j = W - 2; j >= 0; j--)  // sources from the top down
-                        if (S.mk[j] > -2) advance(S.t[j], S.mk[j], k_, rf, v, np);
-                },
-                [&](const double* t, int mk) {
-#pragma unroll
-                    for (int s = 0; s < NSED; s++) pt[s] = t[s];
-                    pmk = mk;
-                });
-#pragma unroll
-            for (int j = W - 2; j >= 1; j--) {
-#pragma unroll
-                for (int s = 0; s < NSED; s++) S.t[j][s] = S.t[j - 1][s];
-                S.mk[j] = S.mk[j - 1];
+                        for (int s = 0; s < NSED; s++) t1[s] = t[s];
+                        mk1 = mk;
+                    });
+                cur = nxt;
             }
+        } else {
+            // at level kk slot j holds the stream of source kk + 1 + j; after the
+            // level every stream moves down one slot and source kk enters slot 0
+            // (the stream of source kk + W - 1 has settled by then)
+            Streams<W - 1> S;
 #pragma unroll
-            for (int s = 0; s < NSED; s++) S.t[0][s] = pt[s];
-            S.mk[0] = pmk;
-            cur = nxt;
+            for (int j = 0; j < W - 1; j++) S.mk[j] = -2;
+            for (int kk = maxk; kk >= kb; kk--) {
+                if (kk > kb) load(kk - 1, nxt);
+                double pt[NSED] = {0.0, 0.0, 0.0, 0.0, 0.0};
+                int pmk = -2;
+                level(
+                    kk, cur,
+                    [&](int k_, double rf, double* v, double* np) {
+#pragma unroll
+                        for (int j = W - 2; j >= 0; j--)  // sources from the top down
+                            if (S.mk[j] > -2) advance(S.t[j], S.mk[j], k_, rf, v, np);
+                    },
+                    [&](const double* t, int mk) {
+#pragma unroll
+                        for (int s = 0; s < NSED; s++) pt[s] = t[s];
+                        pmk = mk;
+                    });
+#pragma unroll
+                for (int j = W - 2; j >= 1; j--) {
+#pragma unroll
+                    for (int s = 0; s < NSED; s++) S.t[j][s] = S.t[j - 1][s];
+                    S.mk[j] = S.mk[j - 1];
+                }
+#pragma unroll
+                for (int s = 0; s < NSED; s++) S.t[0][s] = pt[s];
+                S.mk[0] = pmk;
+                cur = nxt;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < NSED; s++) gp(M.settle)[(size_t)s * plane + col] = settle[s];
+    };
+
+    if constexpr (Q == 0) {
+        if (!on) return;
+        surface();
+        march();
+    } else {
+        if (!marches) {
+            if (on) surface();
+        } else {
+            if (on) march();
+        }
+        __syncthreads();
+        if (marches || !on || !lead) return;
+        for (int k = maxk; k >= (p.airsea ? min(kstart, maxk) : kstart); k--) {
+            const size_t c = cell(k);
+            double v[4], vdc = 0.0, vdp = 0.0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = p.slot[q] >= 0 ? vd[(size_t)q * ncell + c] : 0.0;
+            if (hasDOMC) vdc = vd[(size_t)B_DOMC * ncell + c];
+            if (hasDOMP) vdp = vd[(size_t)B_DOMP * ncell + c];
+            touch(k, v, vdc, vdp);
+            if (k >= kstart) {
+#pragma unroll
+                for (int s = 0; s < NSED; s++) part[(size_t)s * ncell + c] = upart[s];
+            }
+            store(k, v, vdc, vdp);
         }
     }
-#pragma unroll
-    for (int s = 0; s < NSED; s++) gp(M.settle)[(size_t)s * plane + col] = settle[s];
 }
 
 // Column kernels of the coupling: one block per (member, 64 wet columns).
@@ -946,26 +1003,42 @@ void launch_atchem(const MemberDev* mems, const int32_t* list, int nlist, int nc
 }
 
 // ------------------------------------------------------------ launchers
-template <typename R>
+template <typename R, int Q>
 static void launch_col(int W, dim3 grid, const MemberDev* mems, const int32_t* list, hipStream_t s) {
     if (W <= 4)
-        hipLaunchKernelGGL((k_bgc_col<R, 4>), grid, dim3(64), 0, s, mems, list);
+        hipLaunchKernelGGL((k_bgc_col<R, 4, Q>), grid, dim3(Q > 0 ? 64 * Q + 64 : 64), 0, s, mems, list);
     else if (W <= 5)
-        hipLaunchKernelGGL((k_bgc_col<R, 5>), grid, dim3(64), 0, s, mems, list);
+        hipLaunchKernelGGL((k_bgc_col<R, 5, Q>), grid, dim3(Q > 0 ? 64 * Q + 64 : 64), 0, s, mems, list);
     else if (W <= 6)
-        hipLaunchKernelGGL((k_bgc_col<R, 6>), grid, dim3(64), 0, s, mems, list);
+        hipLaunchKernelGGL((k_bgc_col<R, 6, Q>), grid, dim3(Q > 0 ? 64 * Q + 64 : 64), 0, s, mems, list);
     else if (W <= 8)
-        hipLaunchKernelGGL((k_bgc_col<R, 8>), grid, dim3(64), 0, s, mems, list);
-    else
-        hipLaunchKernelGGL((k_bgc_col<R, 16>), grid, dim3(64), 0, s, mems, list);
+        hipLaunchKernelGGL((k_bgc_col<R, 8, Q>), grid, dim3(Q > 0 ? 64 * Q + 64 : 64), 0, s, mems, list);
+    else if constexpr (Q <= 1)
+        hipLaunchKernelGGL((k_bgc_col<R, 16, Q>), grid, dim3(Q > 0 ? 64 * Q + 64 : 64), 0, s, mems, list);
 }
 
-void launch_bio(const MemberDev* mems, const int32_t* list, int nlist, int nwetmax, int W, int prec, hipStream_t s) {
-    const dim3 gcol((nwetmax + 63) / 64, nlist);
-    if (prec == 0)
-        launch_col<double>(W, gcol, mems, list, s);
+void launch_bio(const MemberDev* mems, const int32_t* list, int nlist, int nwetmax, int maxkmax, int W, int prec,
+                hipStream_t s) {
+    // A wave for each part while that leaves the flux beside it the CUs (a
+    // second wave's registers keep the flux's blocks off them): up to about 600
+    // blocks for FP64 members, whose surface part is several times as long, and
+    // 1,280 for FP32 ones.  FP64: four lanes a column of the surface part while
+    // every block has a CU of its own (256), on grids so shallow that the march
+    // is not the longer of the two.  us per step, 36x36x16x24, FP64 by four
+    // lanes / one / in one wave: 1 member (15 blocks) 90 / 105 / 126, 16 (240)
+    // 184 / 193, 32 (480) 304 / 269 / 284, 40 (600) 314 / 335 for the last two,
+    // 48 387 / 372, 64 437 / 424, 128 801 / 796; one of 72x72x32x40 299 / 293.
+    // FP32C in two waves / one: 64 members (960) 343 / 352, 128 (1,920) 644 / 631.
+    const dim3 grid((nwetmax + 63) / 64, nlist);
+    const long long blocks = (long long)grid.x * nlist;
+    if (prec != 0)
+        (blocks <= 1280 ? launch_col<float, 1> : launch_col<float, 0>)(W, grid, mems, list, s);
+    else if (maxkmax <= 20 && W <= 8 && blocks <= 256)
+        launch_col<double, 4>(W, grid, mems, list, s);
+    else if (blocks <= 600)
+        launch_col<double, 1>(W, grid, mems, list, s);
     else
-        launch_col<float>(W, gcol, mems, list, s);
+        launch_col<double, 0>(W, grid, mems, list, s);
 }
 
 template <typename R>

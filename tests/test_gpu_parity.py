@@ -596,3 +596,47 @@ def test_download_rows(eng, dims, L, prec, carry):
         want = np.where(np.isinf(x), np.nan, want)
     assert np.array_equal(np.signbit(got) & ~np.isnan(want), np.signbit(want) & ~np.isnan(want))
     assert np.array_equal(got, want, equal_nan=True)
+
+
+@pytest.mark.parametrize("dims,kind,mld,airsea,n", [
+    ((5, 4, 2), "config2", 0.0, 0, 257),        # one ragged block a member
+    ((18, 18, 8), "domc", 400.0, 0, 80),        # uptake at several levels
+    ((13, 11, 20), "config2", 0.0, 1, 140),     # air-sea exchange; the deepest grid of the four-lane solve
+    ((18, 18, 8), "config2", 400.0, 1, 210),    # both parts in one wave
+])
+def test_surface_solve_by_four_lanes(dims, kind, mld, airsea, n):
+    """A lone FP64 member's BIOGEM step solves its carbonate chemistry with
+    four lanes a column, a larger batch's with one, and a large one's in the
+    same wave as the march: the same bits."""
+    say("case", dims, kind, mld, airsea, n)
+    c = make_case(*dims, kind=kind, seed=67, mld_max=mld)
+    eng = E.Engine(0)
+    try:
+        gid = eng.add_grid(c.g, c.k1)
+        extra = dict(airsea=1, atm_pCO2=278e-6) if airsea else {}
+        p = E.default_bgc_params(1.0 / 96, c.tset, carb_tol=1e-12, carb_maxit=1000, **extra)
+        ids = []
+        for _ in range(n + 1):
+            m = eng.add_member(gid, c.tset.L, E.FP64, c.diff)
+            eng.set_velocity(m, c.u)
+            eng.upload(m, c.ts)
+            eng.bgc_init(m, p, c.light, c.mld)
+            if airsea:
+                eng.set_windspeed(m, np.full((c.g.maxj, c.g.maxi), 8.0))
+            ids.append(m)
+        eng.step(ids[:1], 3)
+        eng.step(ids[1:], 3)
+        shp = (c.g.maxk, c.g.maxj, c.g.maxi)
+
+        def whole(m):
+            out = [eng.download(m, c.ts.shape), eng.bgc_download(m, 0, c.ts.shape), eng.bgc_download(m, 3, c.ts.shape),
+                   eng.bgc_download(m, 1, shp + (5,)), eng.bgc_download(m, 2, shp[1:] + (10,))]
+            return out + ([eng.atmosphere(m, c.g.maxi, c.g.maxj)] if airsea else [])
+
+        alone = whole(ids[0])
+        for m in (ids[1], ids[-1]):
+            for q, (a, b) in enumerate(zip(alone, whole(m))):
+                assert np.array_equal(a, b), q
+            assert eng.diag(m).carb_iters == eng.diag(ids[0]).carb_iters
+    finally:
+        eng.close()
