@@ -769,13 +769,13 @@ __global__ __launch_bounds__(RED_THREADS) void k_couple_reduce(const MemberDev* 
 // (2001-2013), the new cell masses (2049-2052) and the particulates
 // (2042-2043).  The block owns its cells, so the old salinity and masses the
 // tracers need are read before the same threads rewrite them.
-// A block holds TL groups of CPL_THREADS threads, each with its own tracers
+// A block holds TL groups of threads, each with its own tracers
 // (every TL-th): small batches take several, so that a block's chain of
 // rounds, two barriers and a column sum each, is TL times shorter.
-template <typename R, int NJ, int TG, int TL>  // NJ cells per thread (NJ * CPL_LG >= maxk), TG >= tg
-__global__ __launch_bounds__(CPL_THREADS * TL) void k_couple_apply(const MemberDev* __restrict__ mems,
-                                                                   const int32_t* __restrict__ list, int lds_stride) {
-    extern __shared__ double prod_all[];  // [TL][tg][maxk][CPL_COLS]
+template <typename R, int LG, int NJ, int TL>  // LG level groups of NJ cells a thread (NJ * LG >= maxk)
+__global__ __launch_bounds__(CPL_COLS * LG * TL) void k_couple_apply(const MemberDev* __restrict__ mems,
+                                                                     const int32_t* __restrict__ list, int lds_stride) {
+    extern __shared__ double prod_all[];  // [TL][maxk][CPL_COLS]
     __shared__ CplTile T;
     const BlockXYZ B = xcd_blk();
     const MemberDev& M = mems[list[B.y]];
@@ -784,10 +784,10 @@ __global__ __launch_bounds__(CPL_THREADS * TL) void k_couple_apply(const MemberD
     if (w0 >= g.nwet) return;  // uniform over the block
     cpl_tile(g, w0, T);
     const BgcParams& p = M.bp;
-    const int tl = (int)threadIdx.x / CPL_THREADS, tx = (int)threadIdx.x % CPL_THREADS;
+    const int tl = (int)threadIdx.x / (CPL_COLS * LG), tx = (int)threadIdx.x % (CPL_COLS * LG);
     const int c = tx % CPL_COLS, lg = tx / CPL_COLS;
     double* const prod = prod_all + (size_t)tl * lds_stride;
-    const int maxk = g.maxk, L = M.L, tg = cpl_tg(maxk) < TG ? cpl_tg(maxk) : TG;
+    const int maxk = g.maxk, L = M.L;
     const int col = T.col[c], kb = T.kb[c];
     const size_t plane = (size_t)g.ncol, ncell = (size_t)g.ncell, tstride = (size_t)maxk * plane;
     const int par = *gp(M.parity);
@@ -802,7 +802,7 @@ __global__ __launch_bounds__(CPL_THREADS * TL) void k_couple_apply(const MemberD
         typename StateIO<R>::Raw sr[NJ];
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            const int k = 1 + lg + CPL_LG * j;
+            const int k = 1 + lg + LG * j;
             if (k <= maxk && k >= kb) {
                 const size_t cc = (size_t)(k - 1) * plane + col;
                 so[j] = ocn[ncell + cc];
@@ -812,7 +812,7 @@ __global__ __launch_bounds__(CPL_THREADS * TL) void k_couple_apply(const MemberD
         }
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
-            const int k = 1 + lg + CPL_LG * j;
+            const int k = 1 + lg + LG * j;
             if (k <= maxk && k >= kb) {
                 const double snew = StateIO<R>::val(sr[j], lo != nullptr) + SALN0 + 0.0;
                 rs[j] = Snew / snew;
@@ -820,62 +820,44 @@ __global__ __launch_bounds__(CPL_THREADS * TL) void k_couple_apply(const MemberD
             }
         }
     }
-    for (int lb = 2; lb < L; lb += tg * TL) {
-        const int l0 = lb + tl * tg;  // past L for the last round's idle groups
-        // all loads of the group first, then the rescale
-        typename StateIO<R>::Raw lv[TG][NJ];
-        double vv[TG][NJ];
-        int bs[TG];
-#pragma unroll
-        for (int lt = 0; lt < TG; lt++) {
-            const int l = l0 + lt;
+    for (int lb = 2; lb < L; lb += TL) {
+        const int l = lb + tl;  // past L for the last round's idle groups
+        if (l < L) {
+            // all loads first, then the rescale
+            typename StateIO<R>::Raw lv[NJ];
+            double vv[NJ];
             int b = -1;
             for (int q = 0; q < NBGC; q++)
                 if (p.slot[q] == l) b = q;
-            bs[lt] = b;
-            const bool hasv = M.bgc && b >= 0;
-            if (lt < tg && l < L) {
 #pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    const int k = 1 + lg + CPL_LG * j;
-                    if (k <= maxk && k >= kb) {
-                        const size_t cc = (size_t)(k - 1) * plane + col;
-                        lv[lt][j] = StateIO<R>::ldr(st, lo, (size_t)l * tstride + cc);
-                        vv[lt][j] = hasv ? gp(M.vd)[(size_t)b * ncell + cc] : 0.0;
-                    }
+            for (int j = 0; j < NJ; j++) {
+                const int k = 1 + lg + LG * j;
+                if (k <= maxk && k >= kb) {
+                    const size_t cc = (size_t)(k - 1) * plane + col;
+                    lv[j] = StateIO<R>::ldr(st, lo, (size_t)l * tstride + cc);
+                    vv[j] = b >= 0 ? gp(M.vd)[(size_t)b * ncell + cc] : 0.0;
                 }
             }
-        }
+            const double fact = gp(M.scal)[SC_FACT0 + l];
 #pragma unroll
-        for (int lt = 0; lt < TG; lt++) {
-            const int l = l0 + lt;
-            if (lt < tg && l < L) {
-                const int b = bs[lt];
-                const double fact = gp(M.scal)[SC_FACT0 + l];
-#pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    const int k = 1 + lg + CPL_LG * j;
-                    if (k <= maxk && k >= kb) {
-                        const size_t cc = (size_t)(k - 1) * plane + col;
-                        const double x = StateIO<R>::val(lv[lt][j], lo != nullptr) * so[j] * rSold;
-                        double v = fact * x + vv[lt][j];
-                        v = Sratio * v;
-                        if (b >= 0) ocn[(size_t)p.ocn[b] * ncell + cc] = v;
-                        StateIO<R>::st(st, lo, (size_t)l * tstride + cc, rs[j] * v);
-                        prod[((size_t)lt * maxk + (k - 1)) * CPL_COLS + c] = v * mn[j];
-                    }
+            for (int j = 0; j < NJ; j++) {
+                const int k = 1 + lg + LG * j;
+                if (k <= maxk && k >= kb) {
+                    const size_t cc = (size_t)(k - 1) * plane + col;
+                    const double x = StateIO<R>::val(lv[j], lo != nullptr) * so[j] * rSold;
+                    double v = fact * x + vv[j];
+                    v = Sratio * v;
+                    if (b >= 0) ocn[(size_t)p.ocn[b] * ncell + cc] = v;
+                    StateIO<R>::st(st, lo, (size_t)l * tstride + cc, rs[j] * v);
+                    prod[(k - 1) * CPL_COLS + c] = v * mn[j];
                 }
             }
         }
         __syncthreads();
-        {
-            const int lt = lg;
-            const int l = l0 + lt;
-            if (lt < tg && l < L && w0 + c < g.nwet) {
-                double acc = 0.0;
-                for (int k = kb; k <= maxk; k++) acc += prod[((size_t)lt * maxk + (k - 1)) * CPL_COLS + c];
-                gp(M.colold)[(size_t)l * g.nwet + T.slot[c]] = acc;
-            }
+        if (lg == 0 && l < L && w0 + c < g.nwet) {
+            double acc = 0.0;
+            for (int k = kb; k <= maxk; k++) acc += prod[(k - 1) * CPL_COLS + c];
+            gp(M.colold)[(size_t)l * g.nwet + T.slot[c]] = acc;
         }
         __syncthreads();
     }
@@ -892,7 +874,7 @@ __global__ __launch_bounds__(CPL_THREADS * TL) void k_couple_apply(const MemberD
     // T, S, masses and particulates of the thread's cells
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
-        const int k = 1 + lg + CPL_LG * j;
+        const int k = 1 + lg + LG * j;
         if (k <= maxk && k >= kb) {
             const size_t cc = (size_t)(k - 1) * plane + col;
             const auto rT = StateIO<R>::ldr(st, lo, cc);
@@ -1067,20 +1049,26 @@ static void launch_coupling_t(const MemberDev* mems, const int32_t* list, int nl
     }
     if (phase == 1 || phase == 3) return;
     const int st = (int)(b / 8);
-    // a batch of fewer than 512 blocks (two per CU) takes blocks of up to four
-    // groups, as many as the kernel's registers and LDS allow: one FP64 member of
-    // 36x36x16x24 33 -> 17 us, eight FP32C members 45 -> 24, six of 72x72x32x40
-    // (two groups) 157 -> 147.  Larger ones fill the chip either way, and their
-    // small blocks come and go without waiting for 16 waves' room.
-    const bool small = (long long)grid.x * nlist < 512;
-#define CGO_APPLY(NJ_, TL_)                                                                                         \
-    hipLaunchKernelGGL((k_couple_apply<R, NJ_, 1, TL_>), grid, dim3(CPL_THREADS * TL_), b * TL_, s, mems, list, st)
-    if (maxkmax <= 4 * CPL_LG) {
-        if (small) CGO_APPLY(4, 4); else CGO_APPLY(4, 1);
-    } else if (maxkmax <= 8 * CPL_LG) {
-        if (small) CGO_APPLY(8, 2); else CGO_APPLY(8, 1);
+    // A batch of fewer than 512 blocks (two per CU) takes larger ones: four
+    // groups of tracers (one FP64 member of 36x36x16x24 33 -> 17 us, eight FP32C
+    // members 45 -> 24), or on grids of 17 to 32 levels twice the level groups
+    // and half the cells a thread (six FP32C members of 72x72x32x40 149 -> 129
+    // us; one FP64 member, with two tracer groups as well, 297 -> 286 us per
+    // step), on deeper ones two tracer groups (six FP64 members of 48x40x40x30
+    // 318 us per step, 324 with twelve level groups).  Larger batches fill the
+    // chip either way, and their small blocks come and go without waiting for
+    // 16 waves' room (twelve members of 72x72x32x40 965 us per step against
+    // 1,031 with twice the level groups).
+    const long long blocks = (long long)grid.x * nlist;
+    const bool small = blocks < 512;
+#define CGO_APPLY(LG_, NJ_, TL_)                                                                                    \
+    hipLaunchKernelGGL((k_couple_apply<R, LG_, NJ_, TL_>), grid, dim3(CPL_COLS * LG_ * TL_), b * TL_, s, mems, list, st)
+    if (maxkmax <= 16) {
+        if (small) CGO_APPLY(4, 4, 4); else CGO_APPLY(4, 4, 1);
+    } else if (maxkmax <= 32) {
+        if (blocks < 256) CGO_APPLY(8, 4, 2); else if (small) CGO_APPLY(8, 4, 1); else CGO_APPLY(4, 8, 1);
     } else {
-        if (small) CGO_APPLY(12, 2); else CGO_APPLY(12, 1);
+        if (small) CGO_APPLY(4, 12, 2); else CGO_APPLY(4, 12, 1);
     }
 #undef CGO_APPLY
 }
