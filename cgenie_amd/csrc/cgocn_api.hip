@@ -22,8 +22,7 @@ void launch_flux64(const MemberDev*, const int32_t*, int nlist, const FluxShape&
 void launch_flux32(const MemberDev*, const int32_t*, int nlist, const FluxShape&, int maxL, int lb, int nt, int nbuf,
                    int iso_split, const FluxSplit&, int part, size_t lds_cap, hipStream_t);
 void launch_co(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int prec, const FluxSplit&,
-               hipStream_t);
-void launch_flip(const MemberDev*, const int32_t*, int nlist, hipStream_t);
+               bool flip, hipStream_t);
 void launch_bio(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int W, int prec, hipStream_t);
 void launch_coupling(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int maxL, int prec,
                      int phase, hipStream_t);
@@ -604,7 +603,7 @@ static MemLayout layout(const GridH* g, int L, int prec, int carry, int bgc) {
     m.sflux = take(L * ncol * 8);
     m.rho = take(ncell * 8);
     m.cost = take(ncol * 8);
-    m.ctrl = take(256);  // parity, steps, diag[4], dmax, sfresh
+    m.ctrl = take(256);  // parity, steps, diag[4], dmax, sfresh, cofin
     m.isoc = take((size_t)10 * ncell * 8);
     if (bgc) {
         m.ocn = take((2 + NBGC) * ncell * 8);
@@ -685,6 +684,7 @@ static int alloc_member(cgo_engine* e, MemberH* m) {
     d.diag = reinterpret_cast<int32_t*>(b + ly.ctrl + 16);
     d.dmax = reinterpret_cast<double*>(b + ly.ctrl + 32);
     d.sfresh = reinterpret_cast<int32_t*>(b + ly.ctrl + 40);
+    d.cofin = reinterpret_cast<int32_t*>(b + ly.ctrl + 48);
     d.ulist = reinterpret_cast<int32_t*>(b + ly.total);
     d.useg = d.ulist + nwet;
     if (m->bgc) {
@@ -2160,11 +2160,10 @@ static void enqueue_flux(cgo_engine* e, const Lists& ls, const int32_t* d_lists,
     }
 }
 
-// co and the parity flip that end tstepo
-static void enqueue_co_flip(cgo_engine* e, const Lists& ls, const int32_t* d_lists) {
+// co, with the parity flip that ends tstepo
+static void enqueue_co(cgo_engine* e, const Lists& ls, const int32_t* d_lists) {
     for (int p = 0; p < 2; p++)
-        if (ls.n[p]) launch_co(e->d_table, d_lists + ls.off[p], ls.n[p], ls.maxwet[p], ls.maxk[p], p, ls.sp[p], e->s);
-    launch_flip(e->d_table, d_lists + ls.off[4], ls.n[4], e->s);
+        if (ls.n[p]) launch_co(e->d_table, d_lists + ls.off[p], ls.n[p], ls.maxwet[p], ls.maxk[p], p, ls.sp[p], true, e->s);
 }
 
 // the velocity solve of the members that have one (step_goldstein 198-233),
@@ -2185,7 +2184,7 @@ static void enqueue_sfx(cgo_engine* e, const Lists& ls, const int32_t* d_lists) 
 static void enqueue_tstepo(cgo_engine* e, const Lists& ls, const int32_t* d_lists) {
     enqueue_mom(e, ls, d_lists, e->s);
     enqueue_flux(e, ls, d_lists, 3);
-    enqueue_co_flip(e, ls, d_lists);
+    enqueue_co(e, ls, d_lists);
 }
 
 // step_biogem for the members with BIOGEM state (biogem.f90:528-1877), then
@@ -2240,7 +2239,7 @@ static void enqueue_steps(cgo_engine* e, const Lists& ls, const int32_t* d_lists
             hipEventRecord(e->ev_join, e->s2);
         }
         enqueue_flux(e, ls, d_lists, 2);
-        enqueue_co_flip(e, ls, d_lists);
+        enqueue_co(e, ls, d_lists);
         if (bgc) {
             enqueue_coupling(e, ls, d_lists, 3);  // the sums are fresh: tstepo formed them
             hipStreamWaitEvent(e->s, e->ev_join, 0);
@@ -2542,7 +2541,7 @@ int cgo_time_kernel(cgo_engine* e, int32_t which, const int32_t* ids, int32_t n,
             if (which == 0) {
                 if (p == 0 || !ls.n[0]) enqueue_flux(e, ls, e->d_list, 3);  // both precisions
             } else if (which == 1) {
-                launch_co(e->d_table, l, ls.n[p], ls.maxwet[p], ls.maxk[p], p, ls.sp[p], e->s);
+                launch_co(e->d_table, l, ls.n[p], ls.maxwet[p], ls.maxk[p], p, ls.sp[p], false, e->s);
             } else if (which == 4) {
                 if (ls.n[2 + p])
                     launch_bio(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], ls.maxwet_bgc[p], ls.maxk_bgc[p],

@@ -250,6 +250,7 @@ struct MemberDev {
     int32_t* diag;          // [4] limps, carb_fail, carb_iters, co guard hits
     int32_t* ulist;         // [nwet] the wet columns in the flux's segments, each's unstable columns first
     int32_t* useg;          // segments of ulist, then per segment its start and its count of unstable columns
+    int32_t* cofin;         // device scalar: blocks of a convection launch that have finished, 0 between launches
     int32_t* sfresh;        // device flag: colsum holds the sums of the current state
     double* dmax;           // device scalar
     // velocity solve: null when the velocities are prescribed

@@ -1,7 +1,6 @@
 // k_tstep_f64.hip -- FP64 instantiations of the GOLDSTEIN tracer-step
-// kernels, the end-of-step flip and the inventory reduction.  Built with
+// kernels, the inventory reduction and the downloads' packing.  Built with
 // -ffp-contract=off (see tstep_impl.h).
-#define CGO_DEFINE_FLIP
 #include "tstep_impl.h"
 
 namespace cgo {
@@ -12,7 +11,7 @@ void launch_flux64(const MemberDev* t, const int32_t* l, int n, const FluxShape&
 }
 
 void launch_co(const MemberDev* t, const int32_t* l, int n, int nwetmax, int maxkmax, int prec, const FluxSplit& sp,
-               hipStream_t s) {
+               bool flip, hipStream_t s) {
     // A large batch (more chunks of CO_CB columns than the chip holds blocks:
     // 4,096) runs one wave per block and up to four chunks per block, so that
     // blocks that find no unstable column are few; a small one runs every
@@ -28,13 +27,9 @@ void launch_co(const MemberDev* t, const int32_t* l, int n, int nwetmax, int max
     const dim3 grid(large ? (chunks + 3) / 4 : chunks, n);
     const size_t lds = co_lds_bytes(nt, KM);
     if (prec == 0)
-        hipLaunchKernelGGL(k_co<double>, grid, dim3(nt), lds, s, t, l, KM, sp);
+        hipLaunchKernelGGL(k_co<double>, grid, dim3(nt), lds, s, t, l, KM, sp, (int)flip);
     else
-        hipLaunchKernelGGL(k_co<float>, grid, dim3(nt), lds, s, t, l, KM, sp);
-}
-
-void launch_flip(const MemberDev* t, const int32_t* l, int n, hipStream_t s) {
-    hipLaunchKernelGGL(k_flip, dim3((n + 63) / 64), dim3(64), 0, s, t, l, n);
+        hipLaunchKernelGGL(k_co<float>, grid, dim3(nt), lds, s, t, l, KM, sp, (int)flip);
 }
 
 // Per-tracer volume-weighted sum over the member's current state, one block
