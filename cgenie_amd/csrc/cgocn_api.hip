@@ -2080,9 +2080,12 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
     size_t cells = 0;  // most tracer cells of an FP32 member with BIOGEM
     std::vector<int> dgrid;                 // grids of the dense solve, in order of first appearance
     std::vector<std::vector<int32_t>> dmem;
+    std::vector<bool> seen(e->members.size());  // a member listed twice steps once
     for (int i = 0; i < n; i++) {
         MemberH* m = member(e, ids[i]);
         if (!m) return fail(e, CGO_E_ARG, "step: bad member %d", ids[i]);
+        if (seen[ids[i]]) continue;
+        seen[ids[i]] = true;
         const int p = m->prec == CGO_FP64 ? 0 : 1;
         g[p].push_back(ids[i]);
         if (m->bgc) g[2 + p].push_back(ids[i]);

@@ -640,3 +640,26 @@ def test_surface_solve_by_four_lanes(dims, kind, mld, airsea, n):
             assert eng.diag(m).carb_iters == eng.diag(ids[0]).carb_iters
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("prec", [E.FP64, E.FP32C])
+def test_member_listed_twice_steps_once(eng, prec):
+    """Every member's blocks count themselves off at the end of a step: a list
+    that names a member twice gives the bits of one that names it once."""
+    c = make_case(18, 18, 8, kind="config2", L=9, seed=79)
+    out = []
+    for twice in (False, True):
+        ids = []
+        for _ in range(2):
+            m = eng.add_member(eng.add_grid(c.g, c.k1), c.tset.L, prec, c.diff)
+            eng.set_velocity(m, c.u)
+            eng.upload(m, c.ts)
+            eng.bgc_init(m, E.default_bgc_params(1.0 / 96, c.tset), c.light, c.mld)
+            ids.append(m)
+        eng.step([ids[0], ids[1], ids[0]] if twice else ids, 3)
+        eng.tstepo([ids[0], ids[0]] if twice else ids[:1], 2)
+        out.append([eng.download(m, c.ts.shape) for m in ids] + [eng.diag(m).steps for m in ids])
+        for m in ids:
+            eng.remove_member(m)
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    assert out[0][2:] == [5, 3]
