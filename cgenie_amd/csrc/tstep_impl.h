@@ -14,6 +14,7 @@
 // down to level k of the next iteration.
 #pragma once
 #include "cgocn_dev.h"
+#include "flux_rules.h"
 
 #include <type_traits>
 
@@ -185,7 +186,8 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
     // slot q < LB: tracer l0+q; T and S sit in slots 0/1 when l0 == 0, else
     // (coefficients computed here) LB/LB+1
     const int qT = (l0 == 0 || IM != 0) ? 0 : LB, qS = (l0 == 0 || IM != 0) ? 1 : LB + 1;
-    const int nslot = (l0 == 0 || IM != 0) ? nl : LB + 2;  // slots staged per level
+    // (a slot past the block's last tracer is not loaded: the member's state ends there)
+    auto staged = [&](int q) { return flux_staged(q, l0, nl, LB, IM); };
     __shared__ int s_kmin;
     const int tid = threadIdx.x;
     if (tid == 0) s_kmin = maxk + 1;
@@ -256,7 +258,6 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
         return SP(bu, q, pp) - SP(bc, q, pp);
     };
     auto FB = [&](int q) -> R& { return sfb[q * FLUX_THREADS + tid]; };
-    auto slot_tracer = [&](int q) { return q < LB ? l0 + q : q - LB; };
     // prefetch of one plane into registers, then into the LDS ring
     constexpr int FLUX_PF = flux_pf(FLUX_THREADS);
     R pf[NS][FLUX_PF];
@@ -269,11 +270,10 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
             const bool ok = pp < TW && kz + 1 >= sk1[pp < TW ? pp : 0];
 #pragma unroll
             for (int q = 0; q < NS; q++)
-                if (q < nslot || (IM == 0 && q >= LB)) {
-                    const bool ld = ok && (q < nslot);
-                    const uint32_t i = (uint32_t)(slot_tracer(q) * tstride + o + pp);
-                    pf[q][r] = ld ? at(src, i) : (R)0;
-                    if (ANOM) pc[ANOM ? q : 0][r] = (ld && lo_src) ? at(lo_src, i) : (int16_t)0;
+                if (staged(q)) {
+                    const uint32_t i = (uint32_t)(flux_slot_tracer(q, l0, LB) * tstride + o + pp);
+                    pf[q][r] = ok ? at(src, i) : (R)0;
+                    if (ANOM) pc[ANOM ? q : 0][r] = (ok && lo_src) ? at(lo_src, i) : (int16_t)0;
                 }
         }
     };
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
             if (pp < TW) {
 #pragma unroll
                 for (int q = 0; q < NS; q++)
-                    if (q < nslot) {
+                    if (staged(q)) {
                         SP(buf, q, pp) = pf[q][r];
                         if (ANOM) SR(buf, q, pp) = carry_residual((float)pf[q][r], pc[ANOM ? q : 0][r]);
                     }
@@ -293,6 +293,14 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
     };
 
     for (int q = 0; q < LB; q++) FB(q) = (R)0;
+    // the idle slots of the last block hold zeros
+    for (int q = nl; q < LB; q++)
+        for (int pp = tid; pp < TW; pp += FLUX_THREADS)
+#pragma unroll
+            for (int b = 0; b < FLUX_NBUF; b++) {
+                SP(b, q, pp) = (R)0;
+                if (ANOM) SR(b, q, pp) = 0.0f;
+            }
     double rlow = 0.0;     // the new density of the level below, and whether
     bool falls = true;     // it falls strictly from k1 up (co leaves such a column as it is)
     int32_t limps = 0;
