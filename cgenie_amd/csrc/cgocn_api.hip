@@ -336,7 +336,12 @@ static int settle(cgo_engine* e, MemberH* m) { return m->queued ? drain(e) : CGO
 template <typename F>
 static int rows_to_host(cgo_engine* e, MemberH* m, const PackSrc& p, int prec, F&& take) {
     HIPCHK(e, hipSetDevice(e->device));
-    if (!m->queued && !e->sx) HIPCHK(e, hipStreamCreateWithFlags(&e->sx, hipStreamNonBlocking));
+    if (!m->queued) {
+        if (!e->sx) HIPCHK(e, hipStreamCreateWithFlags(&e->sx, hipStreamNonBlocking));
+        // a member that is being set up: its fills are on the null stream,
+        // and the host has not waited for them
+        HIPCHK(e, hipStreamSynchronize(nullptr));
+    }
     const hipStream_t s = m->queued ? e->s : e->sx;
     const size_t ncell = p.ncell, want = std::min(STAGE_D, ncell * p.L);
     if (want > e->stage_d) {

@@ -1,0 +1,84 @@
+"""The engine's host side on the CPU: what it allocates, waits for and
+launches, over a HIP runtime that runs nothing (tests/hip_stub.cpp).  Every
+test runs its program in a process of its own, where the stand-in's entry
+points come before the runtime's."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+
+PRELUDE = """
+import ctypes, sys
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+stub.stub_log.restype = ctypes.c_char_p
+stub.stub_live.restype = ctypes.c_long
+sys.path[:0] = [sys.argv[2], sys.argv[2] + "/tests"]
+import numpy as np
+from cgenie_amd import engine as E
+from cgenie_amd import grid as G
+from cases import make_case
+
+def log():
+    t = stub.stub_log().decode().splitlines()
+    stub.stub_clear()
+    return t
+
+def fail(what, n):
+    stub.stub_fail(what.encode(), ctypes.c_long(n))
+
+def member(eng, c, prec=E.FP64, bgc=False, diso=True):
+    m = eng.add_member(eng.add_grid(c.g, c.k1), c.tset.L, prec, c.diff, diso=diso)
+    eng.set_velocity(m, c.u)
+    eng.upload(m, c.ts)
+    if bgc:
+        eng.bgc_init(m, E.default_bgc_params(1.0 / 96, c.tset), c.light, c.mld)
+    return m
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = tmp_path_factory.mktemp("stub") / "hip_stub.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", os.path.join(ROOT, "tests", "hip_stub.cpp"), "-o", str(so)],
+                   check=True)
+    return str(so)
+
+
+def run(stub, body):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body, stub, ROOT], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.stdout + r.stderr)[-4000:]
+    return r.stdout
+
+
+def test_downloads_follow_the_fills_of_a_new_member(stub):
+    """A member's arrays are cleared by fills that the host does not wait for.
+    A download packs on a stream of its own and comes after them: until then
+    the state's buffer index holds anything."""
+    run(stub, """
+c = make_case(8, 6, 4, kind="config2", seed=3)
+eng = E.Engine(0)
+
+def ordered(t):
+    packs = [i for i, s in enumerate(t) if s.startswith("launch k_pack")]
+    fills = [i for i, s in enumerate(t) if s == "memset null"]
+    assert packs and fills, t
+    waits = [i for i, s in enumerate(t) if s == "sync null" and fills[-1] < i < packs[0]]
+    assert waits or t[packs[0]].endswith("null"), t
+
+gid = eng.add_grid(c.g, c.k1)
+for prec in (E.FP64, E.FP32C):
+    log()
+    m = eng.add_member(gid, c.tset.L, prec, c.diff)
+    eng.download(m, c.ts.shape)
+    ordered(log())
+eng.upload(m, c.ts)
+eng.bgc_init(m, E.default_bgc_params(1.0 / 96, c.tset), c.light, c.mld)
+eng.bgc_download(m, 3, c.ts.shape)
+ordered(log())
+eng.close()
+""")
