@@ -663,3 +663,33 @@ def test_member_listed_twice_steps_once(eng, prec):
             eng.remove_member(m)
     assert all(np.array_equal(a, b) for a, b in zip(*out))
     assert out[0][2:] == [5, 3]
+
+
+@pytest.mark.parametrize("prec", [E.FP64, E.FP32C])
+@pytest.mark.parametrize("which,tile", [(0, None), (1, None), (0, (4, 256, 2, 1)), (1, (4, 256, 2, 1))])
+def test_timing_a_kernel_leaves_the_coupling_its_state(prec, which, tile):
+    """Timing the flux or the convection alone forms the next state's column
+    sums and does not step.  A bio_step and tracercoupling behind it take the
+    sums of the state there is: the bits of a member that was not timed."""
+    say("kernel", which, "tile", tile, "precision", prec)
+    c = make_case(18, 18, 8, kind="config2", L=8, seed=83)
+    eng = E.Engine(0)
+    try:
+        if tile:
+            eng.set_tile(prec, *tile)
+        gid = eng.add_grid(c.g, c.k1)
+        out = []
+        for timed in (False, True):
+            m = eng.add_member(gid, c.tset.L, prec, c.diff)
+            eng.set_velocity(m, c.u)
+            eng.upload(m, c.ts)
+            eng.bgc_init(m, E.default_bgc_params(1.0 / 96, c.tset), c.light, c.mld)
+            eng.step([m], 2)
+            if timed:
+                eng.time_kernel(which, [m], 3)
+            eng.bio_step([m])
+            eng.tracercoupling([m])
+            out.append((eng.download(m, c.ts.shape), eng.bgc_download(m, 0, c.ts.shape)))
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    finally:
+        eng.close()
