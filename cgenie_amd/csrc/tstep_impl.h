@@ -243,7 +243,9 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
     const R diff1 = sizeof(R) == 8 ? (R)M.diff1 : (R)M.diff1f;
     const R diffv = sizeof(R) == 8 ? (R)M.diff2 : (R)M.diff2f;
     const R e0 = (R)g.ec[0], e1 = (R)g.ec[1], e2 = (R)g.ec[2], e3 = (R)g.ec[3];
-    const R scc = M.diso ? e1 : (R)0;
+    const bool mixes = __builtin_amdgcn_readfirstlane(M.diso) != 0;
+    const uint32_t has_mix = (uint32_t)__builtin_amdgcn_readfirstlane(M.diso ? ~0 : 0);
+    const R scc = mixes ? e1 : (R)0;
 
     auto SP = [&](int buf, int q, int pp) -> R& { return sp[(buf * NS + q) * TWS + pp]; };
     auto SR = [&](int buf, int q, int pp) -> float& { return sr[(buf * NS + q) * TWS + pp]; };
@@ -317,7 +319,7 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
     const double rdsvnD = wallN ? 0.0 : gp(g.mj)[MJ_RDSV * JS + J], rdsvsD = wallS ? 0.0 : gp(g.mj)[MJ_RDSV * JS + J - 1];
     const double rdphiD = g.rdphi, diff1D = M.diff1;
     const double e0D = g.ec[0], e1D = g.ec[1], e2D = g.ec[2], e3D = g.ec[3];
-    const double sccD = M.diso ? e1D : 0.0;
+    const double sccD = mixes ? e1D : 0.0;
     auto SPD = [&](int buf, int q, int pp) -> double {
         if (ANOM) return (double)SP(buf, q, pp) + (double)SR(buf, q, pp);
         return (double)SP(buf, q, pp);
@@ -358,7 +360,7 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
         const double tatw = 0.5 * (Tc + Tu);
         const double tec = -e0D - e2D * tatw * 2 - e3D * tatw * tatw * 3;
         dzrho = (e1D * DKD(ub, cb, qS, p) - tec * DKD(ub, cb, qT, p)) * rdza;
-        if (M.diso && dzrho < -1.0E-12) {
+        if (mixes && dzrho < -1.0E-12) {
             const Nbr nc = nbrs(k), nu = nbrs(k + 1);
             iso = true;
             rdzrho = fdiv(1.0, dzrho);
@@ -437,7 +439,7 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
         const bool more = k + 2 <= (SPLIT ? min(khi + 1, maxk) : maxk);
         const bool own = !SPLIT || k >= klo;
         if (more) fetch(kz + 2);
-        if (IM == 1 && active && k >= k1c && !top && M.diso) {
+        if (IM == 1 && active && k >= k1c && !top && mixes) {
             // the pre-pass: the cell's isoneutral coefficients, once
             const uint32_t oc = (uint32_t)(kz * plane + col);
             bool iso = false;
@@ -494,7 +496,7 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
             R ax[4] = {0, 0, 0, 0}, ay[4] = {0, 0, 0, 0}, qq = 0;  // the FP32 form's coefficients
             if (!top) {
                 if constexpr (IM == 2) {
-                    if (M.diso) {
+                    if (ANOM ? M.diso != 0 : mixes) {
                         if constexpr (ANOM) {
                             // zero coefficients give the flux without the isoneutral term exactly
                             const AS_GLOBAL float* ic = reinterpret_cast<const AS_GLOBAL float*>(gp(M.isoc));
@@ -527,6 +529,13 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
             // (evaluated in FP64 from the FP64 velocities when they are set)
             const R divu = ANOM ? at(u, 6 * ncell + oc) : (R)0;
             const R isoc = (R)0.25 * slim * diff1;
+            // A cell without the isoneutral flux has zero gradients (the FP32
+            // form: coefficients), and its flux is masked as well: an infinity at
+            // a corner stays out of it.  (Hidden from the compiler, which makes a
+            // branch per tracer of a select: 256 FP64 members of 36x36x16x24 729
+            // us a launch, 612 so.)
+            uint32_t has_iso = iso ? ~0u : 0u;
+            if (!ANOM) asm("" : "+v"(has_iso));
             double newT = 0, newS = 0;
             double s_os = 0.0, s_mm = 0.0, s_vv = 0.0;
             if (sums) {
@@ -588,7 +597,7 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
                             tv = fma_(ax[3], D(ub, q, pe, p), tv);
                             tv = fma_(ay[2], D(ub, q, ps, p), tv);
                             tv = fma_(ay[3], D(ub, q, pn, p), tv);
-                            tv = fma_(-qq, dU, tv);
+                            tv = __uint_as_float(__float_as_uint(fma_(-qq, dU, tv)) & has_mix);
                             fa = fma_(dU, ca, tv);
                             fbn = fma_(dU, cbn, tv);
                         }
@@ -646,7 +655,8 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
                             const R a = isoc * tv;
                             const R q0 = a * rdz2;
                             const R q1 = __builtin_fma(__builtin_fma(-dz2, q0, a), rdz2, q0);
-                            fa = fa + __builtin_fma(__builtin_fma(-dz2, q1, a), rdz2, q1);
+                            const R fi = __builtin_fma(__builtin_fma(-dz2, q1, a), rdz2, q1);
+                            fa = fa + __hiloint2double(__double2hiint(fi) & has_iso, __double2loint(fi) & has_iso);
                         }
                         const R div = ((fe - fw) * rdphi + (fn - fs) * rds) + (fa - FB(q)) * rdz;
                         const int idx = (l0 + q) * tstride + o + col;

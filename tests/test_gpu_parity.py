@@ -693,3 +693,33 @@ def test_timing_a_kernel_leaves_the_coupling_its_state(prec, which, tile):
         assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("prec,diso,tile", [
+    (E.FP64, True, None), (E.FP64, True, (8, 256, 2, 1)), (E.FP64, True, (4, 128, 3, 0)),
+    (E.FP64, False, None), (E.FP64, False, (8, 256, 2, 1)), (E.FP64, False, (4, 128, 3, 0)),
+    (E.FP32C, False, None), (E.FP32C, False, (6, 256, 2, 1)), (E.FP32C, False, (4, 128, 3, 0))])
+def test_infinities_stay_where_they_are_read(prec, diso, tile):
+    """An infinity reaches the cells whose fluxes read it and no others: those
+    of the FP64 oracle.  A cell without the isoneutral flux does not read its
+    corners, be the water unstable there or the mixing off."""
+    c = make_case(36, 36, 16, kind="ts", L=4, seed=97, random_u=True)
+    rng = np.random.default_rng(98)
+    w = wet(c)
+    c.ts[..., 0] = np.where(w, rng.uniform(0.0, 25.0, w.shape), 0.0)   # unstable in places
+    cells = np.argwhere(w)
+    for q, (k, j, i) in enumerate(cells[rng.choice(len(cells), 24, replace=False)]):
+        c.ts[k, j, i, 2 + q % 2] = np.inf if q % 3 else -np.inf
+    eng = E.Engine(0)
+    try:
+        if tile:
+            eng.set_tile(prec, *tile)
+        m = new_member(eng, c, prec=prec, diso=diso)
+        gold = O.GoldsteinOracle(c.og, c.k1, c.ts, c.u, diso=diso)
+        eng.tstepo([m], 1)
+        gold.step(1)
+        a, b = np.isfinite(eng.download(m, c.ts.shape)[w]), np.isfinite(gold.ts[w])
+        say("case", prec, diso, tile, "not finite", np.count_nonzero(~a), "oracle", np.count_nonzero(~b))
+        assert np.array_equal(a, b)
+    finally:
+        eng.close()
