@@ -2042,6 +2042,7 @@ struct Lists {
     int maxcol[2] = {0, 0}, maxL[2] = {0, 0}, maxwet[2] = {0, 0}, maxwet_bgc[2] = {0, 0}, maxi[2] = {0, 0};
     int maxk_bgc[2] = {0, 0}, wstream[2] = {0, 0}, maxk[2] = {0, 0};
     int ncol_atm = 0;  // widest grid of the members with air-sea exchange, 0 if none
+    bool mix[2] = {};  // some member mixes along isoneutrals
     FluxShape fs[2] = {};
     FluxSplit sp[2] = {};
     size_t nv = 0;  // doubles of workspace the FP32 list's split flux needs
@@ -2057,13 +2058,21 @@ struct Lists {
 // 265, 24 members 299 / 247, 32 members (1536) 363 / 360; FP32C 16 members
 // 204 / 193, 24 members 261 / 291; transport of 5 members of 25x21x11x7 78 /
 // 33, one of 72x72x32x40 255 / 133.
+// Without isoneutral mixing whole columns need no pre-pass and read no
+// corners, so that they take over earlier: on shallow grids, where there is
+// little to split, and on deep ones, where the convection that then walks
+// every column costs the most.  us per step of transport, whole columns /
+// split: FP64 36x36x16x24 8 members (nb 384) 58 / 54, 10 (480) 59 / 53, 12
+// (576) 59 / 75; 36x36x8x24 4 (192) 33 / 30, 8 (384) 32 / 36; 72x72x32x8 4
+// (256) 102 / 88, 6 (384) 103 / 100, 8 (512) 103 / 148; FP32C 36x36x16x24 8 42
+// / 39, 10 45 / 46; 72x72x32x8 4 76 / 73, 6 78 / 86.
 static void flux_split(const cgo_engine* e, Lists& ls, size_t cells) {
     constexpr int FULL = 768;
     for (int p = 0; p < 2; p++) {
         if (!e->auto_tile[p] || !ls.n[p] || ls.fs[p].nblk[1] == 0) continue;
         const long long nb = (long long)ls.fs[p].nblk[1] * ((ls.maxL[p] + 1) / 2) * ls.n[p];
-        if (nb > (p == 0 ? FULL * 3 / 2 : FULL)) continue;
-        const int maxk = ls.fs[p].maxk;
+        const int maxk = ls.fs[p].maxk, plain = std::min(30 * maxk, 12288 / maxk);
+        if (nb > (ls.mix[p] ? (p == 0 ? FULL * 3 / 2 : FULL) : (p == 0 ? plain : plain * 17 / 20))) continue;
         const int chunks = (int)std::min<long long>(std::max<long long>(FULL / nb, 1), (maxk + 1) / 2);
         ls.sp[p].kc = (maxk + chunks - 1) / chunks;
         ls.sp[p].nbx = ls.fs[p].nblk[1];
@@ -2130,6 +2139,7 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
             ls.fs[p].tw[v] = std::max(ls.fs[p].tw[v], e->grids[m->grid]->ftw[v]);
         }
         ls.fs[p].maxk = std::max(ls.fs[p].maxk, m->dev.g.maxk);
+        ls.mix[p] = ls.mix[p] || m->dev.diso;
         if (m->bgc && p) cells = std::max(cells, (size_t)m->L * m->dev.g.ncell);
         if (m->bgc) {
             ls.maxwet_bgc[p] = std::max(ls.maxwet_bgc[p], m->dev.g.nwet);
@@ -2157,14 +2167,16 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
 // the flux launches of both precisions; part as launch_flux_t
 static void enqueue_flux(cgo_engine* e, const Lists& ls, const int32_t* d_lists, int part) {
     for (int p = 0; p < 2; p++) {
-        if (!ls.n[p]) continue;
+        // a batch in which nobody mixes along isoneutrals has no coefficients to form beforehand
+        const int pt = ls.mix[p] ? part : part & 2;
+        if (!ls.n[p] || !pt) continue;
         const int32_t* l = d_lists + ls.off[p];
         if (p == 0)
             launch_flux64(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[0], e->nt[0], e->nbuf[0], e->isosplit[0],
-                          ls.sp[0], part, e->lds_cap, e->s);
+                          ls.sp[0], pt, e->lds_cap, e->s);
         else
             launch_flux32(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[1], e->nt[1], e->nbuf[1], e->isosplit[1],
-                          ls.sp[1], part, e->lds_cap, e->s);
+                          ls.sp[1], pt, e->lds_cap, e->s);
     }
 }
 

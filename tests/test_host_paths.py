@@ -82,3 +82,29 @@ eng.bgc_download(m, 3, c.ts.shape)
 ordered(log())
 eng.close()
 """)
+
+
+def test_batches_without_isoneutral_mixing(stub):
+    """Where no member mixes along isoneutrals the flux has no pre-pass, and
+    whole columns take over from the split by levels at smaller batches; one
+    member that mixes brings both back."""
+    run(stub, """
+c = make_case(36, 36, 16, kind="ts", L=24, seed=5)
+
+def flux(n, mixing, prec=E.FP64):
+    eng = E.Engine(0)
+    ids = [member(eng, c, prec, diso=q < mixing) for q in range(n)]
+    log()
+    eng.tstepo(ids, 1)
+    names = [s.split()[1] for s in log() if s.startswith("launch k_flux")]
+    eng.close()
+    return names
+
+split, whole, pre = "k_flux<double,2,256,2,3>", "k_flux<double,8,256,2,2>", "k_flux<double,2,256,2,1>"
+assert flux(12, 12) == [split] and flux(32, 32) == [pre, whole]
+assert flux(10, 0) == [split] and flux(12, 0) == [whole] and flux(32, 0) == [whole]
+assert flux(12, 1) == [split] and flux(32, 1) == [pre, whole]
+split, whole, pre = "k_flux<float,2,256,2,3>", "k_flux<float,6,256,2,2>", "k_flux<float,2,256,2,1>"
+assert flux(16, 16, E.FP32C) == [split] and flux(20, 20, E.FP32C) == [pre, whole]
+assert flux(8, 0, E.FP32C) == [split] and flux(10, 0, E.FP32C) == [whole]
+""")
