@@ -622,7 +622,7 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
                     }
                 } else {
                     // a cell without the isoneutral flux has zero gradients here
-                    const R dzr = iso ? (R)dzrho : (R)1, dz2 = dzr * dzr, rdz2 = (R)1 / dz2;
+                    const R dzr = iso ? (R)dzrho : (R)1, dz2 = dzr * dzr;
 #pragma unroll
                     for (int q = 0; q < LB; q++) {
                         const R Tc = SP(cb, q, p), Te = SP(cb, q, nc.e), Tw = SP(cb, q, nc.w);
@@ -649,13 +649,10 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
                                 const R dy = east ? D(b, q, m.n, p) * cvn * rdsvn : D(b, q, p, m.s) * cvs * rdsvs;
                                 tv = tv + ((R)2 * dzr * dx - dxr[n] * dzts) * dxr[n] + ((R)2 * dzr * dy - dyr[n] * dzts) * dyr[n];
                             }
-                            // (isoc tv) / dz2, rounded as the division rounds
-                            // (Markstein 1990): with y = RN(1 / dz2) and q1 within an
-                            // ulp of the quotient, q1 + (a - dz2 q1) y rounds to it
-                            const R a = isoc * tv;
-                            const R q0 = a * rdz2;
-                            const R q1 = __builtin_fma(__builtin_fma(-dz2, q0, a), rdz2, q0);
-                            const R fi = __builtin_fma(__builtin_fma(-dz2, q1, a), rdz2, q1);
+                            // divided, not multiplied by a corrected reciprocal: that
+                            // rounds alike only while its remainders are normal
+                            // numbers (256 FP64 members 610 us a launch, 616 so)
+                            const R fi = isoc * tv / dz2;
                             fa = fa + __hiloint2double(__double2hiint(fi) & has_iso, __double2loint(fi) & has_iso);
                         }
                         const R div = ((fe - fw) * rdphi + (fn - fs) * rds) + (fa - FB(q)) * rdz;

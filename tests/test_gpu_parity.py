@@ -723,3 +723,39 @@ def test_infinities_stay_where_they_are_read(prec, diso, tile):
         assert np.array_equal(a, b)
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("tile", [None, (8, 256, 2, 1), (4, 128, 3, 0)])
+@pytest.mark.parametrize("diso", [True, False])
+def test_flux_of_extreme_values_matches_oracle(tile, diso):
+    """Tracers over the whole range of a double, where the isoneutral flux's
+    quotient or its remainders leave the normal numbers (most cells empty, so
+    that a cell's new value is one such flux alone), and infinities, which reach
+    the cells whose fluxes read them and no others: the oracle's bits."""
+    say("tile", tile, "diso", diso)
+    c = make_case(36, 36, 16, kind="ts", L=8, seed=89, random_u=True)
+    rng = np.random.default_rng(90)
+    w = wet(c)
+    tiny, wide, huge = (-308.0, -304.0, 0.2), (-307.0, 285.0, 1.0), (270.0, 285.0, 0.1)
+    for q, (lo, hi, share) in enumerate((tiny, tiny, tiny, wide, huge)):
+        c.ts[..., 2 + q] = np.where(rng.random(w.shape) < share, 10.0 ** rng.uniform(lo, hi, w.shape), 0.0)
+    cells = np.argwhere(w)
+    for q, (k, j, i) in enumerate(cells[rng.choice(len(cells), 12, replace=False)]):
+        c.ts[k, j, i, 7] = np.inf if q % 2 else -np.inf
+    c.ts[~w] = 0.0
+    eng = E.Engine(0)
+    try:
+        if tile:
+            eng.set_tile(E.FP64, *tile)
+        m = new_member(eng, c, diso=diso)
+        gold = O.GoldsteinOracle(c.og, c.k1, c.ts, c.u, diso=diso)
+        for _ in range(2):
+            eng.tstepo([m], 1)
+            gold.step(1)
+            got = eng.download(m, c.ts.shape)
+            bad = [np.count_nonzero((got[w][:, q] != gold.ts[w][:, q]) & ~(np.isnan(got[w][:, q]) & np.isnan(gold.ts[w][:, q])))
+                   for q in range(8)]
+            say("  cells differing per tracer", bad, "not finite", np.count_nonzero(~np.isfinite(gold.ts[w][:, 7])))
+            assert not any(bad)
+    finally:
+        eng.close()
