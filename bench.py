@@ -205,8 +205,8 @@ def run_gpu(args):
             eng.remove_member(m)
     # plain FP64 single member, eager launches (the reference-shaped path:
     # a host calling the step once per ocean step)
-    eng.set_tile(E.FP64, tuned["fp64"]["tracer_block"], tuned["fp64"]["cols"], tuned["fp64"]["ring"],
-                 tuned["fp64"]["iso_prepass"])
+    # with the shape an engine starts with, not the ensemble's
+    eng.set_tile(E.FP64, *autotune.AUTOMATIC[E.FP64])
     ids, tset, n_wet, n_col, g = build_ensemble(eng, E, 1, E.FP64)
     eng.step(ids, STEPS_PER_YEAR)
     eng.sync()

@@ -4,7 +4,9 @@ For a batch of members (grid, tracer count, precision, member count) the
 autotuner times every compiled tile shape of the flux kernel -- tracers per
 block, wet columns per block, level planes resident in LDS, isoneutral
 coefficients computed in every tracer block or once by a pre-pass -- with HIP
-events on the engine's stream (cgo_time_kernel) and keeps the fastest.  The
+events on the engine's stream (cgo_time_kernel) and keeps the fastest.  Among
+them is the shape an engine starts with (AUTOMATIC), by which a batch too small
+to fill the chip takes the flux split by levels.  The
 flux kernel only reads the current state and writes the other ping-pong
 buffer, so timing it repeatedly leaves the model state unchanged.
 
@@ -24,6 +26,7 @@ TRACER_BLOCKS = (2, 4, 6, 8)
 FLUX_COLS = (128, 256)
 FLUX_RINGS = (2, 3)
 ISO_PREPASS = (0, 1)
+AUTOMATIC = {E.FP64: (8, 256, 2, 1), E.FP32C: (6, 256, 2, 1)}   # leaves the form to each batch's size
 
 
 def _key(grid_dims, L, precision, n_members) -> str:
@@ -53,7 +56,9 @@ def tune(eng: E.Engine, members, grid_dims, L: int, precision: int, reps: int = 
     """Pick the flux kernel's tile shape for this batch.
 
     Returns {"tracer_block": tb, "cols": cols, "ring": planes, "iso_prepass": 0|1,
-    "times_ms": {"tbxcolsxplanesxprepass": ms}} and applies the choice to the engine."""
+    "times_ms": {"tbxcolsxplanesxprepass": ms}} and applies the choice to the engine.
+    It holds for every later batch of the precision: set AUTOMATIC[precision]
+    again (Engine.set_tile) before batches of other sizes."""
     key = _key(grid_dims, L, precision, len(members))
     cache = load_cache() if use_cache else {}
     if key in cache:

@@ -14,13 +14,14 @@
 
 #include "../../include/cgocn.h"
 #include "cgocn_dev.h"
+#include "flux_rules.h"
 #include "mom_host.h"
 
 namespace cgo {
-void launch_flux64(const MemberDev*, const int32_t*, int nlist, const FluxShape&, int maxL, int lb, int nt, int nbuf,
-                   int iso_split, const FluxSplit&, int part, size_t lds_cap, hipStream_t);
-void launch_flux32(const MemberDev*, const int32_t*, int nlist, const FluxShape&, int maxL, int lb, int nt, int nbuf,
-                   int iso_split, const FluxSplit&, int part, size_t lds_cap, hipStream_t);
+void launch_flux64(const MemberDev*, const int32_t*, int nlist, const FluxShape&, int maxL, const FluxTile&,
+                   const FluxSplit&, int part, size_t lds_cap, hipStream_t);
+void launch_flux32(const MemberDev*, const int32_t*, int nlist, const FluxShape&, int maxL, const FluxTile&,
+                   const FluxSplit&, int part, size_t lds_cap, hipStream_t);
 void launch_co(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int prec, const FluxSplit&,
                bool flip, hipStream_t);
 void launch_bio(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int W, int prec, hipStream_t);
@@ -151,15 +152,8 @@ struct cgo_engine {
     // destroyed or re-laid-out (BIOGEM state added), so captured graphs can
     // tell that a slot no longer holds what they captured
     std::vector<uint64_t> gen;
-    // flux tile per precision (FP64, FP32C): the shapes the autotuner picks
-    // for a large ensemble on MI355X; cgo_set_tile and its companions change them
-    int lb[2] = {8, 6};       // tracers per block
-    int nt[2] = {256, 256};   // wet columns per block
-    int nbuf[2] = {2, 2};     // level planes resident in LDS
-    int isosplit[2] = {1, 1}; // isoneutral coefficients from a pre-pass
-    // no tile was set for the precision: a batch too small to fill the chip
-    // may take the flux split by levels (flux_split)
-    bool auto_tile[2] = {true, true};
+    // flux shape per precision (FP64, FP32C); cgo_set_tile and its companions change it
+    FluxTile tile[2] = {FLUX_TILE[0], FLUX_TILE[1]};
     size_t lds_cap = 65536;   // LDS one workgroup may take
     std::vector<Graph> graphs;
     int32_t* d_list = nullptr;  // scratch lists for eager steps
@@ -2069,7 +2063,7 @@ struct Lists {
 static void flux_split(const cgo_engine* e, Lists& ls, size_t cells) {
     constexpr int FULL = 768;
     for (int p = 0; p < 2; p++) {
-        if (!e->auto_tile[p] || !ls.n[p] || ls.fs[p].nblk[1] == 0) continue;
+        if (!flux_auto(e->tile[p], p) || !ls.n[p] || ls.fs[p].nblk[1] == 0) continue;
         const long long nb = (long long)ls.fs[p].nblk[1] * ((ls.maxL[p] + 1) / 2) * ls.n[p];
         const int maxk = ls.fs[p].maxk, plain = std::min(30 * maxk, 12288 / maxk);
         if (nb > (ls.mix[p] ? (p == 0 ? FULL * 3 / 2 : FULL) : (p == 0 ? plain : plain * 17 / 20))) continue;
@@ -2172,11 +2166,9 @@ static void enqueue_flux(cgo_engine* e, const Lists& ls, const int32_t* d_lists,
         if (!ls.n[p] || !pt) continue;
         const int32_t* l = d_lists + ls.off[p];
         if (p == 0)
-            launch_flux64(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[0], e->nt[0], e->nbuf[0], e->isosplit[0],
-                          ls.sp[0], pt, e->lds_cap, e->s);
+            launch_flux64(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->tile[0], ls.sp[0], pt, e->lds_cap, e->s);
         else
-            launch_flux32(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->lb[1], e->nt[1], e->nbuf[1], e->isosplit[1],
-                          ls.sp[1], pt, e->lds_cap, e->s);
+            launch_flux32(e->d_table, l, ls.n[p], ls.fs[p], ls.maxL[p], e->tile[1], ls.sp[1], pt, e->lds_cap, e->s);
     }
 }
 
@@ -2494,32 +2486,28 @@ int cgo_graph_destroy(cgo_engine* e, int32_t gid) {
 int cgo_set_tile(cgo_engine* e, int32_t precision, int32_t tb) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (tb != 2 && tb != 4 && tb != 6 && tb != 8))
         return fail(e, CGO_E_ARG, "set_tile: precision %d tracer block %d", precision, tb);
-    e->lb[precision == CGO_FP64 ? 0 : 1] = tb;
-    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
+    e->tile[precision == CGO_FP64 ? 0 : 1].lb = tb;
     return CGO_OK;
 }
 
 int cgo_set_flux_cols(cgo_engine* e, int32_t precision, int32_t cols) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (cols != 128 && cols != 256))
         return fail(e, CGO_E_ARG, "set_flux_cols: precision %d columns %d", precision, cols);
-    e->nt[precision == CGO_FP64 ? 0 : 1] = cols;
-    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
+    e->tile[precision == CGO_FP64 ? 0 : 1].nt = cols;
     return CGO_OK;
 }
 
 int cgo_set_flux_ring(cgo_engine* e, int32_t precision, int32_t planes) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (planes != 2 && planes != 3))
         return fail(e, CGO_E_ARG, "set_flux_ring: precision %d planes %d", precision, planes);
-    e->nbuf[precision == CGO_FP64 ? 0 : 1] = planes;
-    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
+    e->tile[precision == CGO_FP64 ? 0 : 1].nbuf = planes;
     return CGO_OK;
 }
 
 int cgo_set_flux_iso(cgo_engine* e, int32_t precision, int32_t prepass) {
     if (!e || (precision != CGO_FP64 && precision != CGO_FP32C) || (prepass != 0 && prepass != 1))
         return fail(e, CGO_E_ARG, "set_flux_iso: precision %d prepass %d", precision, prepass);
-    e->isosplit[precision == CGO_FP64 ? 0 : 1] = prepass;
-    e->auto_tile[precision == CGO_FP64 ? 0 : 1] = false;
+    e->tile[precision == CGO_FP64 ? 0 : 1].iso = prepass;
     return CGO_OK;
 }
 

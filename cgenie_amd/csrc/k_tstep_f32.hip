@@ -4,9 +4,9 @@
 
 namespace cgo {
 
-void launch_flux32(const MemberDev* t, const int32_t* l, int n, const FluxShape& fs, int maxL, int lb, int nt,
-                   int nbuf, int iso_split, const FluxSplit& sp, int part, size_t lds_cap, hipStream_t s) {
-    launch_flux_t<float>(t, l, n, fs, maxL, lb, nt, nbuf, iso_split, sp, part, lds_cap, s);
+void launch_flux32(const MemberDev* t, const int32_t* l, int n, const FluxShape& fs, int maxL,
+                   const FluxTile& tile, const FluxSplit& sp, int part, size_t lds_cap, hipStream_t s) {
+    launch_flux_t<float>(t, l, n, fs, maxL, tile, sp, part, lds_cap, s);
 }
 
 }  // namespace cgo

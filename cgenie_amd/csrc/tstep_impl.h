@@ -728,9 +728,11 @@ __global__ __launch_bounds__(FLUX_THREADS, 2) void k_flux(const MemberDev* __res
 // stage only their tracers.  part: 1 the pre-pass, 2 the tracer blocks, 3 both.  The tracer block, then the block width, then the
 // ring shrink until the workgroup fits the LDS the device grants one block.
 template <typename R>
-void launch_flux_t(const MemberDev* t, const int32_t* l, int n, const FluxShape& fs, int maxL, int lb, int nt,
-                   int nbuf, int iso_split, const FluxSplit& sp, int part, size_t lds_cap, hipStream_t s) {
+void launch_flux_t(const MemberDev* t, const int32_t* l, int n, const FluxShape& fs, int maxL,
+                   const FluxTile& tile, const FluxSplit& sp, int part, size_t lds_cap, hipStream_t s) {
     constexpr int es = sizeof(R);
+    int lb = tile.lb, nt = tile.nt, nbuf = tile.nbuf;
+    const int iso_split = tile.iso;
     if (sp.kc > 0) {
         if (!(part & 2) || fs.nblk[1] == 0) return;
         const dim3 grid(sp.nbx * ((fs.maxk + sp.kc - 1) / sp.kc), (maxL + 1) / 2, n);

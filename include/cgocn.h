@@ -304,7 +304,11 @@ int cgo_graph_capture(cgo_engine *e, const int32_t *members, int32_t n, int32_t 
 int cgo_graph_launch(cgo_engine *e, int32_t graph_id, int32_t nreps);
 int cgo_graph_destroy(cgo_engine *e, int32_t graph_id);
 
-/* tuning and measurement */
+/* tuning and measurement.  The four flux shape settings of a precision start
+ * as 8, 256, 2, 1 (FP64) and 6, 256, 2, 1 (FP32C).  While they stand so,
+ * untouched or set again, a batch too small to fill the chip takes a form of
+ * the flux made for it; any other shape holds for batches of every size.  The
+ * results do not depend on it. */
 int cgo_set_tile(cgo_engine *e, int32_t precision, int32_t tracer_block);   /* 2, 4, 6 or 8 */
 int cgo_set_flux_cols(cgo_engine *e, int32_t precision, int32_t cols);      /* 128 or 256 wet columns per block */
 int cgo_set_flux_ring(cgo_engine *e, int32_t precision, int32_t planes);    /* 2 or 3 level planes in LDS */

@@ -83,6 +83,44 @@ ordered(log())
 eng.close()
 """)
 
+FLUX = """
+def flux(eng, ids):
+    log()
+    eng.tstepo(ids, 1)
+    return [s.split()[1] for s in log() if s.startswith("launch k_flux")]
+"""
+
+
+@pytest.mark.parametrize("prec,shape", [("FP64", "(8, 256, 2, 1)"), ("FP32C", "(6, 256, 2, 1)")])
+def test_the_starting_shape_set_again_is_the_automatic_one(stub, prec, shape):
+    """A small batch takes the split by levels with the shape an engine starts
+    with, also when that was changed and set again, and whole columns with any
+    other; the tuner times the split among its shapes and leaves it on where it
+    is the fastest."""
+    run(stub, FLUX + f"""
+from cgenie_amd import autotune
+prec, shape = E.{prec}, {shape}
+c = make_case(36, 36, 16, kind="ts", L=24, seed=5)
+eng = E.Engine(0)
+ids = [member(eng, c, prec)]
+split = ["k_flux<%s,2,256,2,3>" % ("double" if prec == E.FP64 else "float")]
+assert autotune.AUTOMATIC[prec] == shape
+assert flux(eng, ids) == split
+for other in ((2,) + shape[1:], shape[:1] + (128,) + shape[2:], shape[:2] + (3, 1), shape[:3] + (0,)):
+    eng.set_tile(prec, *other)
+    got = flux(eng, ids)
+    assert split[0] not in got and len(got) == 1 + other[3], (other, got)
+    eng.set_tile(prec, *shape)
+    assert flux(eng, ids) == split, other
+eng.set_tile(prec, 4, 128, 3, 0)
+best = autotune.tune(eng, ids, (36, 36, 16), 24, prec, reps=2, use_cache=False, write_cache=False)
+assert (best["tracer_block"], best["cols"], best["ring"], best["iso_prepass"]) == shape
+assert flux(eng, ids) == split
+many = [member(eng, c, prec) for _ in range(40)]
+assert split[0] not in flux(eng, many)
+eng.close()
+""")
+
 
 def test_batches_without_isoneutral_mixing(stub):
     """Where no member mixes along isoneutrals the flux has no pre-pass, and
