@@ -2409,29 +2409,29 @@ int cgo_graph_capture(cgo_engine* e, const int32_t* ids, int32_t n, int32_t nste
     Graph gr;
     gr.ids.assign(ids, ids + n);
     for (int i = 0; i < n; i++) gr.gens.push_back(ids[i] < (int32_t)e->gen.size() ? e->gen[ids[i]] : 0);
+    struct Undo {  // whatever step fails, nothing of the graph is left behind
+        Graph& g;
+        bool on = true;
+        ~Undo() {
+            if (!on) return;
+            if (g.graph) hipGraphDestroy(g.graph);
+            hipFree(g.d_lists);
+            hipFree(g.d_nv);
+        }
+    } undo{gr};
+    HIPCHK(e, hipMalloc(&gr.d_lists, ls.v.size() * 4));
     if (ls.nv && hipMalloc(&gr.d_nv, ls.nv * 8) != hipSuccess) {
         gr.d_nv = nullptr;
         no_flux_split(ls);
     }
     ls.sp[1].nv = gr.d_nv;
-    HIPCHK(e, hipMalloc(&gr.d_lists, ls.v.size() * 4));
     HIPCHK(e, hipMemcpy(gr.d_lists, ls.v.data(), ls.v.size() * 4, hipMemcpyHostToDevice));
     HIPCHK(e, hipStreamSynchronize(e->s));
     HIPCHK(e, hipStreamBeginCapture(e->s, hipStreamCaptureModeThreadLocal));
     enqueue_steps(e, ls, gr.d_lists, nsteps);
-    hipError_t r = hipStreamEndCapture(e->s, &gr.graph);
-    if (r != hipSuccess) {
-        hipFree(gr.d_lists);
-        hipFree(gr.d_nv);
-        return fail(e, CGO_E_HIP, "hipStreamEndCapture: %s", hipGetErrorString(r));
-    }
-    r = hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0);
-    if (r != hipSuccess) {
-        hipGraphDestroy(gr.graph);
-        hipFree(gr.d_lists);
-        hipFree(gr.d_nv);
-        return fail(e, CGO_E_HIP, "hipGraphInstantiate: %s", hipGetErrorString(r));
-    }
+    HIPCHK(e, hipStreamEndCapture(e->s, &gr.graph));
+    HIPCHK(e, hipGraphInstantiate(&gr.exec, gr.graph, nullptr, nullptr, 0));
+    undo.on = false;
     int slot = -1;
     for (size_t i = 0; i < e->graphs.size(); i++)
         if (!e->graphs[i].exec) slot = (int)i;

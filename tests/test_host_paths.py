@@ -146,3 +146,31 @@ split, whole, pre = "k_flux<float,2,256,2,3>", "k_flux<float,6,256,2,2>", "k_flu
 assert flux(16, 16, E.FP32C) == [split] and flux(20, 20, E.FP32C) == [pre, whole]
 assert flux(8, 0, E.FP32C) == [split] and flux(10, 0, E.FP32C) == [whole]
 """)
+
+
+def test_a_capture_that_fails_leaves_nothing(stub):
+    """Each allocation and each step of a capture fails once: what it had
+    allocated is given back, and the workspace of the flux split by levels,
+    where it is what cannot be had, is done without."""
+    run(stub, """
+c = make_case(18, 18, 8, kind="config2", L=8, seed=5)
+eng = E.Engine(0)
+m = member(eng, c, E.FP32C, bgc=True)
+eng.step([m], 1)
+before = stub.stub_live()
+refused = 0
+for what in ("malloc", "capture"):
+    for n in range(3):
+        fail(what, n)
+        try:
+            g = eng.capture([m], 2)
+        except E.CgoError:
+            refused += 1
+        else:
+            eng.drop_graph(g)
+        fail(what, -1)
+        assert stub.stub_live() == before, (what, n, log())
+assert refused == 4, refused        # the lists, and the capture's three steps; not the workspace
+assert "bad" not in " ".join(log())
+eng.close()
+""")
