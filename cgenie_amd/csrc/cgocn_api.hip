@@ -239,12 +239,12 @@ int cgo_create(int32_t device, cgo_engine** out) {
         hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming) != hipSuccess ||
         hipHostMalloc((void**)&e->stage, STAGE_N * STAGE_D0 * 8, hipHostMallocDefault) != hipSuccess) {
-        delete e;
+        cgo_destroy(e);
         return CGO_E_HIP;
     }
     for (hipEvent_t& ev : e->ev_stage)
         if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
-            delete e;
+            cgo_destroy(e);
             return CGO_E_HIP;
         }
     int lds = 0;
@@ -269,12 +269,14 @@ int cgo_destroy(cgo_engine* e) {
         if (m) {
             if (m->dbuf) hipFree(m->dbuf);
             if (m->mbuf) hipFree(m->mbuf);
+            if (m->sbuf) hipFree(m->sbuf);
             delete m;
         }
     for (auto* g : e->grids)
         if (g) {
             if (g->dbuf) hipFree(g->dbuf);
             if (g->mbuf) hipFree(g->mbuf);
+            if (g->sbuf) hipFree(g->sbuf);
             delete g->mom;
             delete g;
         }

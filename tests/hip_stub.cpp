@@ -126,10 +126,11 @@ int hipMemcpy(void* d, const void* s, size_t n, int) {
 }
 int hipStreamCreateWithFlags(void** s, unsigned) {
     *s = malloc(1);
+    g_live[*s] = 1;
     g_stream[*s] = "s" + std::to_string(g_stream.size() + 1);
     return 0;
 }
-int hipStreamDestroy(void*) { return 0; }
+int hipStreamDestroy(void* s) { return release(s, "streamdestroy"); }
 int hipStreamSynchronize(void* s) {
     line("sync " + stream(s));
     return 0;

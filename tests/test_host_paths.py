@@ -174,3 +174,36 @@ assert refused == 4, refused        # the lists, and the capture's three steps; 
 assert "bad" not in " ".join(log())
 eng.close()
 """)
+
+
+def test_engines_leave_nothing(stub):
+    """An engine that cannot be created, and one that is closed with members,
+    a graph, surface fluxes and downloads behind it, gives everything back."""
+    run(stub, """
+import ctypes as C
+from cgenie_amd import surface as SF
+L = E.load()
+for what, k in (("malloc", 2), ("event", 8)):
+    for n in range(k):
+        fail(what, n)
+        h = C.c_void_p()
+        assert L.cgo_create(0, C.byref(h)) == -2 and not h.value
+        fail(what, -1)
+        assert stub.stub_live() == 0, (what, n, log())
+g = G.make_grid(36, 36, 8, nyear=96)
+w = G.read_world(sys.argv[2] + "/tests/golden/worbe2", 36, 36)
+su = SF.surflux_setup(g, w.k1)
+eng = E.Engine(0)
+gid = eng.add_grid(g, w.k1)
+eng.set_momentum(gid, g, w)
+eng.set_surflux(gid, su)
+m = eng.add_member(gid, 2, E.FP64, G.diffusivities(2000.0, 1e-5))
+eng.set_wind(m, np.load(sys.argv[2] + "/tests/golden/worbe2_wind.npz")["stress"])
+eng.set_surface(m, *SF.atmosphere(g, w.k1, 64, ice=True))
+gr = eng.capture([m], 2)
+eng.sync()
+eng.download(m, (8, 36, 36, 2))
+eng.close()
+assert stub.stub_live() == 0, log()
+assert "bad" not in " ".join(log())
+""")
