@@ -322,6 +322,17 @@ static int drain(cgo_engine* e) {
 // other members step.
 static int settle(cgo_engine* e, MemberH* m) { return m->queued ? drain(e) : CGO_OK; }
 
+// device memory; where none is left, the eager steps' workspace is given up for it
+static bool dev_alloc(cgo_engine* e, void** p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    hipGetLastError();
+    if (!e->d_nv || hipStreamSynchronize(e->s) != hipSuccess) return false;
+    hipFree(e->d_nv);
+    e->d_nv = nullptr;
+    e->d_nv_cap = 0;
+    return hipMalloc(p, bytes) == hipSuccess;
+}
+
 // Planes of member m as rows [ncell][L] to the host: take(c, n, rows) gets the
 // rows of cells [c, c + n) from pinned memory, in order.  The member's work in
 // flight precedes the packing on its stream, so nothing waits for it
@@ -508,7 +519,7 @@ int cgo_grid_create(cgo_engine* e, const cgo_grid_desc* d, int32_t* grid_id) {
     }
     const size_t o_fb0 = take(fb[0].size() * sizeof(FluxBlk) + 16), o_fb1 = take(fb[1].size() * sizeof(FluxBlk) + 16);
     hipSetDevice(e->device);
-    if (hipMalloc(&g->dbuf, off) != hipSuccess) {
+    if (!dev_alloc(e, &g->dbuf, off)) {
         delete g;
         return fail(e, CGO_E_NOMEM, "grid_create: hipMalloc(%zu)", off);
     }
@@ -629,9 +640,18 @@ static MemLayout layout(const GridH* g, int L, int prec, int carry, int bgc) {
     return m;
 }
 
+// behind a member's state, what a step's flux hands its convection: the
+// columns it sorted (nwet) and their segments.  Formed anew in every step, so
+// it is no part of the layout that checkpoints hold.
+static size_t flux_lists_bytes(const GridH* g) {
+    const size_t nseg = (size_t)std::max(g->dev.nfblk[0], g->dev.nfblk[1]);
+    return ((size_t)g->dev.nwet + 1 + 2 * nseg) * 4;
+}
+
 int64_t cgo_member_bytes(cgo_engine* e, int32_t grid_id, int32_t maxl, int32_t precision, int32_t bgc) {
     if (!e || grid_id < 0 || grid_id >= (int)e->grids.size()) return CGO_E_ARG;
-    return (int64_t)layout(e->grids[grid_id], maxl, precision, 1, bgc).total;
+    const GridH* g = e->grids[grid_id];
+    return (int64_t)(layout(g, maxl, precision, 1, bgc).total + flux_lists_bytes(g));
 }
 
 static int alloc_member(cgo_engine* e, MemberH* m) {
@@ -646,12 +666,8 @@ static int alloc_member(cgo_engine* e, MemberH* m) {
         HIPCHK(e, hipMemcpy(keep.data(), old, oldly.total, hipMemcpyDeviceToHost));
     }
     void* buf = nullptr;
-    // behind the member's state, what a step's flux hands its convection: the
-    // columns it sorted and their segments.  Formed anew in every step, so it
-    // is no part of the layout that checkpoints hold.
-    const size_t nwet = (size_t)g->dev.nwet, nseg = (size_t)std::max(g->dev.nfblk[0], g->dev.nfblk[1]);
-    const size_t scratch = (nwet + 1 + 2 * nseg) * 4;
-    if (hipMalloc(&buf, ly.total + scratch) != hipSuccess)
+    const size_t scratch = flux_lists_bytes(g);
+    if (!dev_alloc(e, &buf, ly.total + scratch))
         return fail(e, CGO_E_NOMEM, "member: hipMalloc(%zu) failed", ly.total + scratch);
     HIPCHK(e, hipMemset(buf, 0, ly.total + scratch));
     if (old) {
@@ -687,7 +703,7 @@ static int alloc_member(cgo_engine* e, MemberH* m) {
     d.sfresh = reinterpret_cast<int32_t*>(b + ly.ctrl + 40);
     d.cofin = reinterpret_cast<int32_t*>(b + ly.ctrl + 48);
     d.ulist = reinterpret_cast<int32_t*>(b + ly.total);
-    d.useg = d.ulist + nwet;
+    d.useg = d.ulist + g->dev.nwet;
     if (m->bgc) {
         d.ocn = reinterpret_cast<double*>(b + ly.ocn);
         d.part = reinterpret_cast<double*>(b + ly.part);
@@ -944,7 +960,7 @@ int cgo_grid_set_momentum(cgo_engine* e, int32_t grid_id, const cgo_momentum_des
     }
     hipSetDevice(e->device);
     void* buf = nullptr;
-    if (hipMalloc(&buf, off) != hipSuccess) {
+    if (!dev_alloc(e, &buf, off)) {
         delete M;
         return fail(e, CGO_E_NOMEM, "grid_set_momentum: hipMalloc(%zu)", off);
     }
@@ -1023,7 +1039,7 @@ static int mom_attach(cgo_engine* e, MemberH* m, int32_t id) {
     const MomSetup& S = *g->mom;
     const MomMemberLayout L = mom_member_layout(S.mi, S.mj, S.mk, m->prec != CGO_FP64);
     void* buf = nullptr;
-    if (hipMalloc(&buf, L.total * 8) != hipSuccess) return fail(e, CGO_E_NOMEM, "set_wind: hipMalloc(%zu)", L.total * 8);
+    if (!dev_alloc(e, &buf, L.total * 8)) return fail(e, CGO_E_NOMEM, "set_wind: hipMalloc(%zu)", L.total * 8);
     if (hipMemset(buf, 0, L.total * 8) != hipSuccess ||
         hipMemset(const_cast<void*>(m->dev.u), 0, (size_t)m->dev.g.ncell * (m->prec == CGO_FP64 ? 3 * 8 : 7 * 4)) != hipSuccess) {
         hipFree(buf);
@@ -1119,7 +1135,7 @@ int cgo_grid_set_surflux(cgo_engine* e, int32_t grid_id, const cgo_surflux_desc*
                  o_src = take(std::max<size_t>(rsrc.size(), 1) * 4);
     void* buf = nullptr;
     hipSetDevice(e->device);
-    if (hipMalloc(&buf, off) != hipSuccess) return fail(e, CGO_E_NOMEM, "grid_set_surflux: hipMalloc(%zu)", off);
+    if (!dev_alloc(e, &buf, off)) return fail(e, CGO_E_NOMEM, "grid_set_surflux: hipMalloc(%zu)", off);
     char* b = static_cast<char*>(buf);
     SfxGridDev h{};
     h.nyear = d->nyear;
@@ -1241,7 +1257,7 @@ int cgo_set_surface(cgo_engine* e, int32_t id, const double* atemp, const double
     sc[SS_N2O] = g->sfx_gas[2];
     sc[SS_ISTEP] = 0.0;
     void* buf = nullptr;
-    if (hipMalloc(&buf, nd * 8) != hipSuccess) return fail(e, CGO_E_NOMEM, "set_surface: hipMalloc(%zu)", nd * 8);
+    if (!dev_alloc(e, &buf, nd * 8)) return fail(e, CGO_E_NOMEM, "set_surface: hipMalloc(%zu)", nd * 8);
     const MemLayout ly = layout(g, m->L, m->prec, m->p.carry, m->bgc);
     double* slot = reinterpret_cast<double*>(static_cast<char*>(m->dbuf) + ly.sflux);
     if (hipMemcpy(buf, h.data(), h.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1678,7 +1694,7 @@ int cgo_restore(cgo_engine* e, int32_t id, const void* buf, size_t n) {
         HIPCHK(e, hipMemcpy(m->mbuf, static_cast<const char*>(buf) + sizeof h + h.payload, h.mom_bytes, hipMemcpyHostToDevice));
     if (h.sfx && !m->sbuf) {
         void* sb = nullptr;
-        if (hipMalloc(&sb, h.sfx_bytes) != hipSuccess) return fail(e, CGO_E_NOMEM, "restore: hipMalloc(%zu)", (size_t)h.sfx_bytes);
+        if (!dev_alloc(e, &sb, h.sfx_bytes)) return fail(e, CGO_E_NOMEM, "restore: hipMalloc(%zu)", (size_t)h.sfx_bytes);
         m->sbuf = sb;
         m->sbytes = h.sfx_bytes;
     } else if (!h.sfx && m->sbuf) {
@@ -2044,38 +2060,17 @@ struct Lists {
     size_t nv = 0;  // doubles of workspace the FP32 list's split flux needs
 };
 
-// The flux split by levels, for batches whose blocks of two tracers and whole
-// columns (nb) leave the chip short of work.  768 such blocks are resident at
-// once: up to there the levels are cut into as many chunks (of two levels at
-// least) as fill it.  Past it the two-tracer blocks still beat the wide
-// tracer blocks with their pre-pass for a while, for FP64 members up to half
-// as many again.  us per step, wide blocks against this: one FP64 member of
-// 36x36x16x24 206 / 141 (nb 48), 4 members 231 / 150, 16 members (768) 308 /
-// 265, 24 members 299 / 247, 32 members (1536) 363 / 360; FP32C 16 members
-// 204 / 193, 24 members 261 / 291; transport of 5 members of 25x21x11x7 78 /
-// 33, one of 72x72x32x40 255 / 133.
-// Without isoneutral mixing whole columns need no pre-pass and read no
-// corners, so that they take over earlier: on shallow grids, where there is
-// little to split, and on deep ones, where the convection that then walks
-// every column costs the most.  us per step of transport, whole columns /
-// split: FP64 36x36x16x24 8 members (nb 384) 58 / 54, 10 (480) 59 / 53, 12
-// (576) 59 / 75; 36x36x8x24 4 (192) 33 / 30, 8 (384) 32 / 36; 72x72x32x8 4
-// (256) 102 / 88, 6 (384) 103 / 100, 8 (512) 103 / 148; FP32C 36x36x16x24 8 42
-// / 39, 10 45 / 46; 72x72x32x8 4 76 / 73, 6 78 / 86.
 static void flux_split(const cgo_engine* e, Lists& ls, size_t cells) {
-    constexpr int FULL = 768;
     for (int p = 0; p < 2; p++) {
         if (!flux_auto(e->tile[p], p) || !ls.n[p] || ls.fs[p].nblk[1] == 0) continue;
-        const long long nb = (long long)ls.fs[p].nblk[1] * ((ls.maxL[p] + 1) / 2) * ls.n[p];
-        const int maxk = ls.fs[p].maxk, plain = std::min(30 * maxk, 12288 / maxk);
-        if (nb > (ls.mix[p] ? (p == 0 ? FULL * 3 / 2 : FULL) : (p == 0 ? plain : plain * 17 / 20))) continue;
-        const int chunks = (int)std::min<long long>(std::max<long long>(FULL / nb, 1), (maxk + 1) / 2);
-        ls.sp[p].kc = (maxk + chunks - 1) / chunks;
+        const size_t nv = p == 1 && ls.n[3] ? cells * ls.n[1] : 0;
+        const int kc = flux_split_levels((long long)ls.fs[p].nblk[1] * ((ls.maxL[p] + 1) / 2) * ls.n[p], ls.fs[p].maxk, p,
+                                         ls.mix[p], nv);
+        if (!kc) continue;
+        ls.sp[p].kc = kc;
         ls.sp[p].nbx = ls.fs[p].nblk[1];
-        if (p == 1 && ls.n[3]) {
-            ls.sp[p].stride = cells;
-            ls.nv = cells * ls.n[1];
-        }
+        ls.sp[p].stride = nv ? cells : 0;
+        ls.nv += nv;
     }
 }
 // where its workspace cannot be had the flux marches whole columns

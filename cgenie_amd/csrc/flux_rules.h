@@ -2,6 +2,7 @@
 // engine's launches take, as plain constexpr functions: the engine takes them
 // as they are, and a CPU program can go through them over their whole range.
 #pragma once
+#include <cstddef>
 
 namespace cgo {
 
@@ -29,6 +30,38 @@ constexpr FluxTile FLUX_TILE[2] = {{8, 256, 2, 1}, {6, 256, 2, 1}};
 // for every batch.
 constexpr bool flux_auto(const FluxTile& t, int p) {
     return t.lb == FLUX_TILE[p].lb && t.nt == FLUX_TILE[p].nt && t.nbuf == FLUX_TILE[p].nbuf && t.iso == FLUX_TILE[p].iso;
+}
+
+// Levels per block of the flux split by levels, 0: whole columns.  nb: a
+// batch's blocks of two tracers and whole columns, maxk its deepest grid's
+// levels, p its precision (0 FP64, 1 FP32C), mix: some member mixes along
+// isoneutrals, nv: doubles of workspace the split needs (FP32C members with
+// BIOGEM: their new values).
+// 768 such blocks are resident at once: up to there the levels are cut into as
+// many chunks (of two levels at least) as fill the chip.  Past it the
+// two-tracer blocks still beat the wide tracer blocks with their pre-pass for
+// a while, for FP64 members up to half as many again.  us per step, wide
+// blocks against this: one FP64 member of 36x36x16x24 206 / 141 (nb 48), 4
+// members 231 / 150, 16 members (768) 308 / 265, 24 members 299 / 247, 32
+// members (1536) 363 / 360; FP32C 16 members 204 / 193, 24 members 261 / 291;
+// transport of 5 members of 25x21x11x7 78 / 33, one of 72x72x32x40 255 / 133.
+// Without isoneutral mixing whole columns need no pre-pass and read no
+// corners, so that they take over earlier: on shallow grids, where there is
+// little to split, and on deep ones, where the convection that then walks
+// every column costs the most.  us per step of transport, whole columns /
+// split: FP64 36x36x16x24 8 members (nb 384) 58 / 54, 10 (480) 59 / 53, 12
+// (576) 59 / 75; 36x36x8x24 4 (192) 33 / 30, 8 (384) 32 / 36; 72x72x32x8 4
+// (256) 102 / 88, 6 (384) 103 / 100, 8 (512) 103 / 148; FP32C 36x36x16x24 8 42
+// / 39, 10 45 / 46; 72x72x32x8 4 76 / 73, 6 78 / 86.
+constexpr size_t FLUX_NV_MAX = (size_t)64 << 20;  // 512 MiB; a third of it is a full chip on 48 levels
+constexpr int flux_split_levels(long long nb, int maxk, int p, bool mix, size_t nv) {
+    constexpr int FULL = 768;
+    const int plain = 30 * maxk < 12288 / maxk ? 30 * maxk : 12288 / maxk;
+    const int most = mix ? (p == 0 ? FULL * 3 / 2 : FULL) : (p == 0 ? plain : plain * 17 / 20);
+    if (nb > most || nv > FLUX_NV_MAX) return 0;
+    const long long fill = FULL / nb > 1 ? FULL / nb : 1, deep = (maxk + 1) / 2;
+    const int chunks = (int)(fill < deep ? fill : deep);
+    return (maxk + chunks - 1) / chunks;
 }
 
 }  // namespace cgo

@@ -18,6 +18,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libcgocn.so")
 
 FP64, FP32C = 0, 1
+WORKSPACE_MAX = 512 << 20   # most an engine holds beside its members for its eager steps, and for each graph
 
 _d, _i32, _i64 = C.c_double, C.c_int32, C.c_int64
 _dp = C.POINTER(C.c_double)

@@ -143,6 +143,13 @@ class Server:
         gid = self.grids.get(req.dims)[0]
         return self.eng.member_bytes(gid, req.L, req.precision, req.L >= 7)
 
+    def _workspace(self, reqs) -> int:
+        """Most that a round graph of these runs holds beside them: its FP32C
+        runs' new values, sized for the largest run with BIOGEM (cgocn.h)."""
+        cells = [r.dims[0] * r.dims[1] * r.dims[2] * r.L for r in reqs if r.precision == E.FP32C and r.L >= 7]
+        n = sum(r.precision == E.FP32C for r in reqs)
+        return min(8 * n * max(cells), E.WORKSPACE_MAX) if cells else 0
+
     def _prepare(self, req: Request):
         if req.rid not in self.prep:
             gid, g, k1, base_u = self.grids.get(req.dims)
@@ -167,7 +174,8 @@ class Server:
             if not fut.done():
                 break                    # inputs still being prepared
             nb = self._bytes(req)
-            if self.used + nb > self.budget:
+            ws = self._workspace([*self.active.values(), req])
+            if self.used + nb + (ws if self.active else 0) > self.budget:
                 break                    # first come, first served: wait for memory
             if self.max_active is not None and len(self.active) >= self.max_active:
                 break                    # the batch is full: wait for a run to finish

@@ -115,6 +115,11 @@ int cgo_grid_create(cgo_engine *e, const cgo_grid_desc *g, int32_t *grid_id);   
 int cgo_member_create(cgo_engine *e, int32_t grid_id, int32_t maxl, int32_t precision,
                       const cgo_member_params *p, int32_t *member_id);
 int cgo_member_destroy(cgo_engine *e, int32_t member_id);
+/* device memory of one member.  Beside its members an engine holds, where small
+ * batches of CGO_FP32C members with BIOGEM are stepped, a workspace of maxl
+ * doubles per cell and member of the batch, at most 512 MiB: one for the eager
+ * steps, given up when a member cannot be allocated otherwise, and one per
+ * captured graph */
 int64_t cgo_member_bytes(cgo_engine *e, int32_t grid_id, int32_t maxl, int32_t precision, int32_t bgc);
 
 /* uploads / downloads in reference layouts */

@@ -207,3 +207,53 @@ eng.close()
 assert stub.stub_live() == 0, log()
 assert "bad" not in " ".join(log())
 """)
+
+
+def test_member_bytes_cover_the_allocation(stub):
+    """cgo_member_bytes, by which runs are admitted, is what a member takes."""
+    run(stub, """
+for dims, L in (((8, 6, 4), 2), ((18, 18, 8), 9), ((36, 36, 16), 24)):
+    for prec in (E.FP64, E.FP32C):
+        c = make_case(*dims, kind="config2" if L > 7 else "ts", L=L, seed=5)
+        eng = E.Engine(0)
+        gid = eng.add_grid(c.g, c.k1)
+        for bgc in (False, True)[:1 + (L > 7)]:
+            log()
+            m = eng.add_member(gid, L, prec, c.diff)
+            if bgc:
+                log()
+                eng.bgc_init(m, E.default_bgc_params(1.0 / 96, c.tset), c.light, c.mld)
+            got = [int(s.split()[1]) for s in log() if s.startswith("malloc")]
+            assert got == [eng.member_bytes(gid, L, prec, bgc)], (dims, L, prec, bgc, got)
+        eng.close()
+""")
+
+
+def test_the_eager_workspace_gives_way_to_a_member(stub):
+    """Where no memory is left for a member, the eager steps' workspace is
+    freed for it; the next small step takes one again, or whole columns."""
+    run(stub, FLUX + """
+c = make_case(18, 18, 8, kind="config2", L=8, seed=5)
+eng = E.Engine(0)
+m = member(eng, c, E.FP32C, bgc=True)
+eng.step([m], 1)
+gid = eng.add_grid(c.g, c.k1)
+log()
+fail("malloc", 0)
+q = eng.add_member(gid, 8, E.FP32C, c.diff)
+t = log()
+assert t.index("free") < [i for i, s in enumerate(t) if s.startswith("malloc")][0] and "sync s1" in t[:t.index("free")], t
+eng.remove_member(q)
+fail("malloc", 0)
+assert flux(eng, [m]) == ["k_flux<float,2,256,2,1>", "k_flux<float,6,256,2,2>"]
+assert flux(eng, [m]) == ["k_flux<float,2,256,2,3>"]
+for given_up in (True, False):
+    fail("malloc", 0)
+    try:
+        eng.add_member(gid, 8, E.FP32C, c.diff)
+        assert given_up
+    except E.CgoError:
+        assert not given_up
+eng.close()
+assert stub.stub_live() == 0
+""")

@@ -120,6 +120,25 @@ def test_batch_cap_limits_active_runs(monkeypatch):
     assert [r.rid for r in sorted(reqs, key=lambda r: r.admitted)] == [0, 1, 2, 3, 4]
 
 
+@pytest.mark.parametrize("precision,together", [(E.FP64, 2), (E.FP32C, 1)])
+def test_admission_counts_the_round_graphs_workspace(monkeypatch, precision, together):
+    """Two runs whose members fill the budget share a round only if what a
+    graph of small FP32C batches holds beside them fits too; a run alone is
+    admitted by its member's memory, and every run is served."""
+    monkeypatch.setattr(S, "request_inputs", lambda req, g, k1, u: (None, np.zeros(1), None, (0, 0), None, None))
+    monkeypatch.setattr(S.GridCache, "get", lambda self, dims: (0, None, None, None))
+    eng = CountingEngine(bytes_per_member=1_000_000)
+    srv = S.Server(eng, hbm_budget=16.5e6, round_steps=48)
+    srv.pool = SyncPool()
+    for q in range(3):
+        srv.submit(S.Request(q, (36, 36, 16), 8, years=1, precision=precision, seed=q))
+    big = S.Request(3, (36, 36, 16), 16, years=1, precision=precision, seed=3)   # 16 MB of the 16.5, and 2.7 of workspace
+    srv.submit(big)
+    st = srv.run()
+    assert st["requests_done"] == 4 and max(len(ids) for ids, _ in eng.calls) == together
+    assert srv._workspace([S.Request(q, (72, 72, 32), 40, 1, E.FP32C, q) for q in range(64)]) == E.WORKSPACE_MAX
+
+
 def test_suspended_run_resumes_where_it_stopped(monkeypatch):
     """A run suspended between rounds leaves the GPU (its memory is
     returned to the budget), waits like a new request and, restored from its
