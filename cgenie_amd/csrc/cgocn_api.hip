@@ -2044,11 +2044,11 @@ int cgo_set_windspeed(cgo_engine* e, int32_t id, const double* wspeed) {
 
 // ---------------------------------------------------------------- stepping
 struct Lists {
-    // [p64 list][p32 list][bgc p64][bgc p32][all][velocity solve][surface fluxes]
+    // [p64 list][p32 list][bgc p64][bgc p32][velocity solve][surface fluxes]
     // [velocity solve through the band][velocity solve by the dense inverse, grouped by grid]
     std::vector<int32_t> v;
-    int n[9] = {}, off[9] = {};
-    std::vector<int> momGroups;             // per grid of the dense solve: offset in list 8, count, N
+    int n[8] = {}, off[8] = {};
+    std::vector<int> momGroups;             // per grid of the dense solve: offset in list 7, count, N
     int momN = 0, momCol = 0, momBand = 0;  // most psi points, columns and maxi of a member with a velocity solve
     int sfxCol = 0;                         // most columns of a member with surface fluxes
     int maxcol[2] = {0, 0}, maxL[2] = {0, 0}, maxwet[2] = {0, 0}, maxwet_bgc[2] = {0, 0}, maxi[2] = {0, 0};
@@ -2081,7 +2081,7 @@ static void no_flux_split(Lists& ls) {
 }
 
 static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
-    std::vector<int32_t> g[9];
+    std::vector<int32_t> g[8];
     size_t cells = 0;  // most tracer cells of an FP32 member with BIOGEM
     std::vector<int> dgrid;                 // grids of the dense solve, in order of first appearance
     std::vector<std::vector<int32_t>> dmem;
@@ -2094,9 +2094,8 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
         const int p = m->prec == CGO_FP64 ? 0 : 1;
         g[p].push_back(ids[i]);
         if (m->bgc) g[2 + p].push_back(ids[i]);
-        g[4].push_back(ids[i]);
         if (m->mbuf) {
-            g[5].push_back(ids[i]);
+            g[4].push_back(ids[i]);
             ls.momN = std::max(ls.momN, e->grids[m->grid]->mom->N);
             ls.momCol = std::max(ls.momCol, m->dev.g.ncol);
             ls.momBand = std::max(ls.momBand, m->dev.g.maxi);
@@ -2110,14 +2109,14 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
                 }
                 dmem[q].push_back(ids[i]);
             } else {
-                g[7].push_back(ids[i]);
+                g[6].push_back(ids[i]);
             }
         }
         if (m->sbuf) {
             if (e->grids[m->grid]->sfx_atchem && !(m->bgc && m->dev.bp.airsea))
                 return fail(e, CGO_E_STATE, "step: member %d's surface fluxes read CO2 from an atmosphere it does not have "
                                             "(cgo_bgc_init with air-sea exchange)", ids[i]);
-            g[6].push_back(ids[i]);
+            g[5].push_back(ids[i]);
             ls.sfxCol = std::max(ls.sfxCol, m->dev.g.ncol);
         }
         ls.maxcol[p] = std::max(ls.maxcol[p], m->dev.g.ncol);
@@ -2140,12 +2139,12 @@ static int make_lists(cgo_engine* e, const int32_t* ids, int32_t n, Lists& ls) {
         }
     }
     for (size_t q = 0; q < dgrid.size(); q++) {
-        ls.momGroups.push_back((int)g[8].size());
+        ls.momGroups.push_back((int)g[7].size());
         ls.momGroups.push_back((int)dmem[q].size());
         ls.momGroups.push_back(e->grids[dgrid[q]]->mom->N);
-        g[8].insert(g[8].end(), dmem[q].begin(), dmem[q].end());
+        g[7].insert(g[7].end(), dmem[q].begin(), dmem[q].end());
     }
-    for (int q = 0; q < 9; q++) {
+    for (int q = 0; q < 8; q++) {
         ls.off[q] = (int)ls.v.size();
         ls.n[q] = (int)g[q].size();
         ls.v.insert(ls.v.end(), g[q].begin(), g[q].end());
@@ -2179,15 +2178,15 @@ static void enqueue_co(cgo_engine* e, const Lists& ls, const int32_t* d_lists) {
 // which precedes their tstepo
 // part 1: the column kernel before the solve; 2: the rest; 3: both
 static void enqueue_mom(cgo_engine* e, const Lists& ls, const int32_t* d_lists, hipStream_t s, int part = 3) {
-    if (ls.n[5])
-        launch_mom(e->d_table, d_lists + ls.off[5], ls.n[5], d_lists + ls.off[7], ls.n[7], d_lists + ls.off[8],
+    if (ls.n[4])
+        launch_mom(e->d_table, d_lists + ls.off[4], ls.n[4], d_lists + ls.off[6], ls.n[6], d_lists + ls.off[7],
                    ls.momGroups.data(), (int)ls.momGroups.size() / 3, ls.momN, ls.momCol, ls.momBand, part, s);
 }
 
 // the surface fluxes of the members that have them (surflux, called by
 // genie before the ocean step, genie.f90:271-282)
 static void enqueue_sfx(cgo_engine* e, const Lists& ls, const int32_t* d_lists) {
-    if (ls.n[6]) launch_sfx(e->d_table, d_lists + ls.off[6], ls.n[6], ls.sfxCol, 0, e->s);
+    if (ls.n[5]) launch_sfx(e->d_table, d_lists + ls.off[5], ls.n[5], ls.sfxCol, 0, e->s);
 }
 
 static void enqueue_tstepo(cgo_engine* e, const Lists& ls, const int32_t* d_lists) {
@@ -2346,7 +2345,7 @@ int cgo_surface_slot(cgo_engine* e, int32_t id, const double* fx0sic, const doub
     HIPCHK(e, hipMemcpy(static_cast<double*>(m->sbuf) + SW_FX0SIC * ncol, h.data(), h.size() * 8, hipMemcpyHostToDevice));
     Lists ls;
     if (int rc = prepare(e, &id, 1, ls, false)) return rc;
-    launch_sfx(e->d_table, e->d_list + ls.off[6], ls.n[6], ls.sfxCol, 1, e->s);
+    launch_sfx(e->d_table, e->d_list + ls.off[5], ls.n[5], ls.sfxCol, 1, e->s);
     HIPCHK(e, hipGetLastError());
     return CGO_OK;
 }

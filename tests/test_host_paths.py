@@ -257,3 +257,18 @@ for given_up in (True, False):
 eng.close()
 assert stub.stub_live() == 0
 """)
+
+
+def test_captured_lists_hold_what_the_kernels_read(stub):
+    """A captured step's lists name a member once per kernel family that it
+    takes part in: transport, and BIOGEM."""
+    run(stub, """
+eng = E.Engine(0)
+for kind, L, n in (("ts", 3, 1), ("config2", 8, 2)):
+    m = member(eng, make_case(18, 18, 8, kind=kind, L=L, seed=5), bgc=kind != "ts")
+    eng.step([m], 1)
+    log()
+    eng.capture([m], 1)
+    assert "malloc %d" % (4 * n) in log()
+eng.close()
+""")
