@@ -759,3 +759,47 @@ def test_flux_of_extreme_values_matches_oracle(tile, diso):
             assert not any(bad)
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("dims,kind,L,mld,airsea,n", [
+    ((18, 18, 8), "domc", 9, 400.0, 1, 321),      # 4 blocks a member: 1,284 in one wave each
+    ((36, 36, 16), "config2", 8, 400.0, 1, 86),   # 15 blocks, 1,290
+    ((36, 36, 16), "domc", 8, 0.0, 0, 86),
+])
+def test_fp32_column_step_in_one_wave_and_two(dims, kind, L, mld, airsea, n):
+    """An FP32C member's BIOGEM step in a large batch, both parts of a column
+    in one wave, and alone, a wave for each: the same bits, also where the
+    uptake spans levels and where air-sea exchange adds to the surface."""
+    say("case", dims, kind, L, mld, airsea, n)
+    c = make_case(*dims, kind=kind, L=L, seed=101, mld_max=mld)
+    eng = E.Engine(0)
+    try:
+        gid = eng.add_grid(c.g, c.k1)
+        extra = dict(airsea=1, atm_pCO2=278e-6) if airsea else {}
+        p = E.default_bgc_params(1.0 / 96, c.tset, carb_tol=1e-12, carb_maxit=1000, **extra)
+        ids = []
+        for _ in range(n + 1):
+            m = eng.add_member(gid, L, E.FP32C, c.diff)
+            eng.set_velocity(m, c.u)
+            eng.upload(m, c.ts)
+            eng.bgc_init(m, p, c.light, c.mld)
+            if airsea:
+                eng.set_windspeed(m, np.full((c.g.maxj, c.g.maxi), 8.0))
+            ids.append(m)
+        assert n * -(-int((c.k1[1:-1, 1:-1] <= c.g.maxk).sum()) // 64) > 1280
+        eng.step(ids[:1], 3)
+        eng.step(ids[1:], 3)
+        shp = (c.g.maxk, c.g.maxj, c.g.maxi)
+
+        def whole(m):
+            out = [eng.download(m, c.ts.shape), eng.bgc_download(m, 0, c.ts.shape), eng.bgc_download(m, 3, c.ts.shape),
+                   eng.bgc_download(m, 1, shp + (5,)), eng.bgc_download(m, 2, shp[1:] + (10,))]
+            return out + ([eng.atmosphere(m, c.g.maxi, c.g.maxj)] if airsea else [])
+
+        alone = whole(ids[0])
+        for m in (ids[1], ids[-1]):
+            for q, (a, b) in enumerate(zip(alone, whole(m))):
+                assert np.array_equal(a, b), q
+            assert eng.diag(m).carb_iters == eng.diag(ids[0]).carb_iters
+    finally:
+        eng.close()
