@@ -2064,8 +2064,8 @@ static void flux_split(const cgo_engine* e, Lists& ls, size_t cells) {
     for (int p = 0; p < 2; p++) {
         if (!flux_auto(e->tile[p], p) || !ls.n[p] || ls.fs[p].nblk[1] == 0) continue;
         const size_t nv = p == 1 && ls.n[3] ? cells * ls.n[1] : 0;
-        const int kc = flux_split_levels((long long)ls.fs[p].nblk[1] * ((ls.maxL[p] + 1) / 2) * ls.n[p], ls.fs[p].maxk, p,
-                                         ls.mix[p], nv);
+        const int kc = flux_split_levels((long long)ls.fs[p].nblk[1] * ((ls.maxL[p] + 1) / 2) * ls.n[p],
+                                         (long long)ls.maxwet[p] * ls.n[p], ls.fs[p].maxk, p, ls.mix[p], ls.n[2 + p] > 0, nv);
         if (!kc) continue;
         ls.sp[p].kc = kc;
         ls.sp[p].nbx = ls.fs[p].nblk[1];

@@ -49,21 +49,24 @@ def test_split_by_levels_over_its_range(tmp_path):
     out = run(tmp_path, """
     for (int p = 0; p < 2; p++)
         for (int mix = 0; mix < 2; mix++)
-            for (int maxk = 2; maxk <= 48; maxk++)
-                for (int nb = 1; nb <= 2000; nb++) {
-                    const int kc = flux_split_levels(nb, maxk, p, mix, FLUX_NV_MAX);
-                    bool ok = kc == 0 || (kc >= 2 && kc <= maxk);
-                    if (kc) ok = ok && (kc == maxk || (long long)nb * ((maxk + kc - 1) / kc) <= 768);
-                    ok = ok && (kc != 0) <= (flux_split_levels(1, maxk, p, mix, 0) != 0) && !(nb > 1152 && kc);
-                    ok = ok && flux_split_levels(nb, maxk, p, mix, FLUX_NV_MAX + 1) == 0;
-                    ok = ok && !(kc && !flux_split_levels(nb, maxk, p, true, 0));
-                    if (!ok) std::printf("p %d mix %d maxk %d nb %d: %d\\n", p, mix, maxk, nb, kc);
-                }
-    // where it was measured
-    const int at[][4] = {{0, 1, 16, 48}, {0, 1, 16, 1152}, {1, 1, 16, 768}, {0, 0, 16, 480}, {0, 0, 8, 192}, {0, 0, 32, 384},
-                         {1, 0, 16, 384}, {1, 0, 32, 256}};
-    const int no[][4] = {{0, 1, 16, 1153}, {1, 1, 16, 769}, {0, 0, 16, 576}, {0, 0, 8, 384}, {0, 0, 32, 512}, {1, 0, 16, 480},
-                         {1, 0, 32, 384}};
-    for (auto& a : at) if (!flux_split_levels(a[3], a[2], a[0], a[1], 0)) std::printf("no split %d %d\\n", a[2], a[3]);
-    for (auto& a : no) if (flux_split_levels(a[3], a[2], a[0], a[1], 0)) std::printf("split %d %d\\n", a[2], a[3]);""")
+            for (int bgc = 0; bgc < 2; bgc++)
+                for (int maxk = 2; maxk <= 48; maxk++)
+                    for (int nb = 1; nb <= 1000; nb++)
+                        for (int cols = 16; cols <= 200000; cols *= 5) {
+                            const int kc = flux_split_levels(nb, cols, maxk, p, mix, bgc, FLUX_NV_MAX);
+                            bool ok = kc == 0 || (kc >= 2 && kc <= maxk);
+                            if (kc) ok = ok && ((maxk + kc - 1) / kc == 1 || (long long)nb * ((maxk + kc - 1) / kc) <= 768);
+                            ok = ok && !(nb > 832 && kc) && !(nb <= 192 && maxk >= 8 && mix && cols <= 1000 && !kc);
+                            ok = ok && flux_split_levels(nb, cols, maxk, p, mix, bgc, FLUX_NV_MAX + 1) == 0;
+                            if (!ok) std::printf("p %d mix %d bgc %d maxk %d nb %d cols %d: %d\\n", p, mix, bgc, maxk, nb, cols, kc);
+                        }
+    // nb, columns, levels, precision, mixing, BIOGEM: on either side of the line, where both were measured
+    const int at[][6] = {{48, 907, 16, 0, 1, 1}, {480, 27210, 16, 0, 1, 1}, {768, 14512, 16, 0, 1, 1}, {816, 43548, 32, 0, 1, 1},
+                         {224, 12698, 16, 1, 1, 1}, {384, 7256, 16, 1, 1, 1}, {768, 43536, 16, 1, 1, 0}, {480, 9070, 16, 0, 0, 0},
+                         {192, 3628, 8, 0, 0, 0}, {408, 21774, 32, 0, 0, 0}, {384, 7256, 16, 1, 0, 0}, {272, 14516, 32, 1, 0, 0}};
+    const int no[][6] = {{576, 32652, 16, 0, 1, 1}, {576, 32688, 8, 0, 1, 1}, {864, 16326, 16, 0, 1, 1}, {1152, 21768, 16, 0, 1, 1},
+                         {320, 18140, 16, 1, 1, 1}, {480, 9070, 16, 1, 1, 1}, {769, 9000, 16, 1, 1, 0}, {576, 10884, 16, 0, 0, 0},
+                         {384, 7256, 8, 0, 0, 0}, {544, 29032, 32, 0, 0, 0}, {480, 9070, 16, 1, 0, 0}, {408, 21774, 32, 1, 0, 0}};
+    for (auto& a : at) if (!flux_split_levels(a[0], a[1], a[2], a[3], a[4], a[5], 0)) std::printf("no split %d %d\\n", a[0], a[1]);
+    for (auto& a : no) if (flux_split_levels(a[0], a[1], a[2], a[3], a[4], a[5], 0)) std::printf("split %d %d\\n", a[0], a[1]);""")
     assert out == "", out[:2000]

@@ -272,3 +272,21 @@ for kind, L, n in (("ts", 3, 1), ("config2", 8, 2)):
     assert "malloc %d" % (4 * n) in log()
 eng.close()
 """)
+
+
+def test_many_columns_take_whole_columns(stub):
+    """Batches of many wet columns take whole columns, FP32C ones where they
+    have BIOGEM; fewer, or transport alone, the split by levels."""
+    run(stub, FLUX + """
+c, t = (make_case(18, 18, 8, kind=k, L=8, seed=5) for k in ("config2", "ts"))
+
+def form(n, prec, case):
+    eng = E.Engine(0)
+    got = flux(eng, [member(eng, case, prec, bgc=case is c) for _ in range(n)])
+    eng.close()
+    return "split" if got[-1].endswith(",3>") else "whole"
+
+assert [form(n, E.FP32C, c) for n in (32, 80, 120)] == ["split", "whole", "whole"]
+assert [form(n, E.FP32C, t) for n in (80, 120)] == ["split", "split"]
+assert [form(n, E.FP64, c) for n in (120, 144)] == ["split", "whole"]
+""")
