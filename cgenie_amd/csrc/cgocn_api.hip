@@ -27,6 +27,7 @@ void launch_co(const MemberDev*, const int32_t*, int nlist, int nwetmax, int max
 void launch_bio(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int W, int prec, hipStream_t);
 void launch_coupling(const MemberDev*, const int32_t*, int nlist, int nwetmax, int maxkmax, int maxL, int prec,
                      int phase, hipStream_t);
+void launch_sums_stale(const MemberDev*, const int32_t*, int nlist, hipStream_t);
 void launch_pack(const PackSrc&, int prec, uint32_t c0, uint32_t nc, double* out, hipStream_t);
 void launch_inventory(const MemberDev*, int32_t member, int L, double* out, const double* w, int prec, hipStream_t);
 void launch_carbconst_surface(const MemberDev*, int32_t member, int nwet, double* out, hipStream_t);
@@ -2564,10 +2565,11 @@ int cgo_time_kernel(cgo_engine* e, int32_t which, const int32_t* ids, int32_t n,
     *avg_ms = (double)ms / reps;
     // the flux and the convection formed the sums of a state that no step
     // hands over: a coupling that follows forms those of the state there is
-    const int32_t stale = 0;
-    for (int i = 0; i < n && (which == 0 || which == 1 || which == 3); i++) {
-        const MemberH* m = member(e, ids[i]);
-        if (m->bgc) HIPCHK(e, hipMemcpy(m->dev.sfresh, &stale, 4, hipMemcpyHostToDevice));
+    if (which == 0 || which == 1 || which == 3) {
+        for (int p = 0; p < 2; p++)
+            if (ls.n[2 + p]) launch_sums_stale(e->d_table, e->d_list + ls.off[2 + p], ls.n[2 + p], e->s);
+        HIPCHK(e, hipGetLastError());
+        HIPCHK(e, hipStreamSynchronize(e->s));
     }
     return CGO_OK;
 }

@@ -984,7 +984,18 @@ void launch_atchem(const MemberDev* mems, const int32_t* list, int nlist, int nc
                        lds_cols);
 }
 
+// marks the members' column sums stale: the next coupling forms them itself
+__global__ __launch_bounds__(64) void k_sums_stale(const MemberDev* __restrict__ mems, const int32_t* __restrict__ list,
+                                                   int n) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i < n) *gp(mems[list[i]].sfresh) = 0;
+}
+
 // ------------------------------------------------------------ launchers
+void launch_sums_stale(const MemberDev* mems, const int32_t* list, int nlist, hipStream_t s) {
+    hipLaunchKernelGGL(k_sums_stale, dim3((nlist + 63) / 64), dim3(64), 0, s, mems, list, nlist);
+}
+
 template <typename R, int Q>
 static void launch_col(int W, dim3 grid, const MemberDev* mems, const int32_t* list, hipStream_t s) {
     if (W <= 4)
