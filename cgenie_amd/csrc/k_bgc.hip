@@ -1022,6 +1022,8 @@ void launch_bio(const MemberDev* mems, const int32_t* list, int nlist, int nwetm
     // 184 / 193, 32 (480) 304 / 269 / 284, 40 (600) 314 / 335 for the last two,
     // 48 387 / 372, 64 437 / 424, 128 801 / 796; one of 72x72x32x40 299 / 293.
     // FP32C in two waves / one: 64 members (960) 343 / 352, 128 (1,920) 644 / 631.
+    // (Measured at 16 and 32 levels, between which the line at 20 lies, and for
+    // the numbers of blocks on 36x36x16 alone.)
     const dim3 grid((nwetmax + 63) / 64, nlist);
     const long long blocks = (long long)grid.x * nlist;
     if (prec != 0)

@@ -94,9 +94,11 @@ void launch_inventory(const MemberDev* t, int32_t m, int L, double* out, const d
 // host takes them in (go_ts(maxl, ...)), into pinned host memory: a block
 // turns CT cells around in LDS (an odd stride, so that neither side
 // meets a bank twice), reads whole lines of every plane and writes one
-// contiguous range.  Bound by PCIe (~56 GB/s).  FP32 states are decoded as the
-// host did it: float plus carry times 2^-16 ulp, the ulp of an infinity
-// infinite (an infinite value comes out NaN where its carry is zero).
+// contiguous range.  A piece of 1 MiB takes 28 us (37 GB/s into host memory);
+// the host's copy of it out of the staging, ~35 us, bounds a download.  FP32
+// states are decoded as the host did it: float plus carry times 2^-16 ulp, the
+// ulp of an infinity infinite (an infinite value comes out NaN where its carry
+// is zero).
 template <typename R, uint32_t CT>
 __global__ __launch_bounds__(256) void k_pack(PackSrc p, uint32_t c0, uint32_t nc, double* __restrict__ out) {
     extern __shared__ __align__(16) double tile[];  // [L][CT + 1]
